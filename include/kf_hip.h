@@ -108,7 +108,8 @@ int kf_hip_gated_act_q8(const float* gate, const float* up, int rows, int n, int
  * row_bytes must equal the type's row size for n (rows are packed). */
 
 /* Decode and small-batch product of `rows` activation rows: one row is the streaming GEMV, several rows the
- * multi-row product that reads each weight row once per eight activation rows. Replaces matvec_i8_launch
+ * multi-row product that reads each weight row once per eight activation rows (q8_0) or sixteen (the K types, which take
+ * the tile GEMM of kf_hip_gemm_i8 instead where a cost model fitted on MI355X favours it). Replaces matvec_i8_launch
  * (exec.rs:1996-2039) with the kernels matvec_i8 / matvec_i8_1 / matvec_i8_1s / mm_i8_{8,16,32} /
  * mm_frag_{8,16,24,32} (crates/kf-backend-cuda/src/kernels/quant.cuh:604-627, mm_frag.cuh:294-300).
  * q5_K and q6_K weights (Q8K-kind activations, any row count: one launch per eight activation rows) run their own
@@ -119,13 +120,11 @@ int kf_hip_gemv(uint32_t ty, const void* w, int64_t row_bytes, const void* act, 
 
 /* Batched / prefill int8 GEMM on native rows: y [rows][n_out] from `rows` activation rows of the weight type's kind.
  * q8_0 (Q8_0-kind activations, n a multiple of 128): one int8 MFMA per 32-column group gives the exact int32 block
- * dots, rescaled by the group's activation and weight scales. q4_K (Q8K-kind activations, n a multiple of 256): the
- * 6-bit scales split into two 3-bit halves folded into two int8 operand planes, so two int8 MFMA chains form the
- * exact super-block integer; the mins term by an exact f16 MFMA per super-block, and the float rescale once per 256
- * columns. q5_K and q6_K (Q8K-kind activations, n a multiple of 256; q6_K: a multiple of 2048, so that its 210-byte
- * super-block rows start 16-byte aligned): one int8 MFMA per 32-column group (q6_K: per 16-column scale) gives the
- * exact int32 sub-block dots, the integer sub-scales are applied by multiply-adds into the exact super-block integer,
- * q5_K's mins by an exact f16 MFMA; other shapes return KF_E_UNSUPPORTED (kf_hip_gemv takes them).
+ * dots, rescaled by the group's activation and weight scales. q4_K, q5_K
+ * and q6_K (Q8K-kind activations, n a multiple of 256; q6_K here only a multiple of 2048, kf_hip_matmul and kf_hip_gemv
+ * take any): the products scale x value as two int8 operand planes, so two int8 MFMA chains form the exact super-block
+ * integer; the mins term by an exact f16 MFMA per super-block, and the float rescale once per 256 columns; other shapes
+ * return KF_E_UNSUPPORTED.
  * Replaces kf8_gemm_dense / Store::gemm (crates/kf-backend-cuda/src/kernels/kf8.cu:375-395, HAS_M for q4_K / q5_K;
  * crates/kf-backend-cuda/src/kf8.rs:310-323) without the KF8 unpack pass (kf_unpack_i8, quant.cuh:585-601, instantiated
  * for q5_K / q6_K at quant_q5_K.cu:114 / quant_q6_K.cu:131): the native bytes are read directly. */
@@ -224,9 +223,9 @@ int kf_hip_moe_gemv(uint32_t ty, const void* w, const void* w_up, int64_t expert
  * from w + s * expert_bytes and columns n_split.. from w2 + s * expert_bytes (gate and up as one product). Output row p
  * of the group order is written to y row out_rows[p] (device, nullable: row p); y is [*][n_out]. Rows of act past
  * offsets[n_slots] are not read. Replaces kf8_gemm_moe (crates/kf-backend-cuda/src/kernels/kf8.cu:400-416) without the
- * KF8 unpack; kf_hip_moe_ffn takes it past 64 routed pairs, as expert_gemm_chunks (exec.rs:2196-2237). A grid of at
- * most two rounds of the CUs runs each tile as two K halves through the split scratch (the stream's slot); the first
- * half's partial passes through the tile's rows of y before the sum lands there. */
+ * KF8 unpack; kf_hip_moe_ffn takes it past 64 routed pairs, as expert_gemm_chunks (exec.rs:2196-2237). The tiles of all
+ * slots are cut into equal ranges, one a CU; a cut tile's parts meet in the split scratch (the stream's slot) and a second
+ * launch adds them. */
 int kf_hip_moe_gemm(uint32_t ty, const void* w, const void* w2, int64_t expert_bytes, int64_t row_bytes, int n_split, const void* act,
                     int pairs, int n, int n_out, const int32_t* offsets, int n_slots, const int32_t* out_rows, float* y, void* stream);
 

@@ -46,15 +46,12 @@ hipError_t kf_launch_gemm_q8_0(const void* w, int64_t row_bytes, const void* act
 int kf_gemm_k_multiple();
 
 bool kf_gemm_kq_ok(uint32_t ty, const void* w, int64_t row_bytes, int K, int N);
-double kf_gemm_kq_sb_rounds(int M, int N, int K);
-double kf_gemm_q4k_sb_rounds(int M, int N, int K);
+double kf_gemm_kq_us(uint32_t ty, int M, int N, int K);
 hipError_t kf_launch_gemm_kq_moe(const void* w, const void* w2, int64_t expert_bytes, int64_t row_bytes, int n_split, const void* act, int pairs,
                                  int n_slots, const int32_t* offsets, const int32_t* out_rows, float* y, int N, int K, hipStream_t s);
-static bool q4k_gemm_kq_pays(int rows, int n_in, int n_out);
+static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes);
 hipError_t kf_launch_gemm_kq(uint32_t ty, const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y,
                              int M, int N, int K, hipStream_t s);
-hipError_t kf_launch_gemm_q4k(const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y, int M,
-                              int N, int K, hipStream_t s);
 int kf_rows_max_n(uint32_t ty);
 hipError_t kf_launch_rows(uint32_t ty, const void* w, const void* w2, int64_t expert_bytes, int64_t row_bytes, const void* act, int act_rows,
                           int n, int n_out, const int32_t* order, const int32_t* offsets, int n_slots, int pairs, int n_used, int per_slot,
@@ -62,9 +59,6 @@ hipError_t kf_launch_rows(uint32_t ty, const void* w, const void* w2, int64_t ex
 hipError_t kf_launch_moe_group(const int32_t* slots, int total, int n_slots, int32_t* order, int32_t* offsets, hipStream_t s);
 hipError_t kf_launch_moe_gather_act(const void* src, int src_rows, void* dst, int pairs, const int32_t* order, const int32_t* offsets,
                                     int n_slots, int n_used, int n, hipStream_t s);
-hipError_t kf_launch_gemm_q4k_moe(const void* w, const void* w2, int64_t expert_bytes, int64_t row_bytes, int n_split, const void* act,
-                                  int pairs, int n_slots, const int32_t* offsets, const int32_t* out_rows, float* y, int N, int K,
-                                  hipStream_t s);
 hipError_t kf_launch_moe_combine(const float* part, const float* wts, const int32_t* slots, const float* host, float* out, int rows, int n_used,
                                  int n_embd, float scale, int n_slots, hipStream_t s);
 
@@ -217,6 +211,11 @@ int kf_hip_gemv(uint32_t ty, const void* w, int64_t row_bytes, const void* act, 
     const int rc = check_product(ty, w, row_bytes, act, y, rows, n, n_out);
     if (rc != KF_OK) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // the K types: the tile GEMM where its cost is below the few-row product's
+    if (ty != KF_TYPE_Q8_0 && n_out > 0 && kq_gemm_pays(ty, w, rows, n, n_out, row_bytes)) {
+        const hipError_t e = kf_launch_gemm_kq(ty, w, row_bytes, act, bias, res, y, rows, n_out, n, s);
+        return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
+    }
     // q5_K / q6_K: several rows on the matrix cores (16 activation rows a weight pass), one row (or a layout the
     // matrix-core form does not take: q6_K rows with an odd number of super-blocks) on their own per-lane product
     if ((ty == KF_TYPE_Q5_K || ty == KF_TYPE_Q6_K) && rows > 1 && !kf_knob_on(KF_KNOB_ROWS_VALU) && kf_rows_mma_1_ok(ty, w, row_bytes, n, n_out, rows)) {
@@ -253,16 +252,8 @@ int kf_hip_gemm_i8(uint32_t ty, const void* w, int64_t row_bytes, const void* ac
                    int rows, int n, int n_out, void* stream) {
     const int rc = check_product(ty, w, row_bytes, act, y, rows, n, n_out);
     if (rc != KF_OK) return rc;
-    if (ty == KF_TYPE_Q4_K) {
-        if (q4k_gemm_kq_pays(rows, n, n_out) && kf_gemm_kq_ok(ty, w, row_bytes, n, n_out)) {
-            const hipError_t e = kf_launch_gemm_kq(ty, w, row_bytes, act, bias, res, y, rows, n_out, n, static_cast<hipStream_t>(stream));
-            return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
-        }
-        const hipError_t e = kf_launch_gemm_q4k(w, row_bytes, act, bias, res, y, rows, n_out, n, static_cast<hipStream_t>(stream));
-        return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
-    }
-    if (ty == KF_TYPE_Q5_K || ty == KF_TYPE_Q6_K) {
-        if (!kf_gemm_kq_ok(ty, w, row_bytes, n, n_out))
+    if (ty == KF_TYPE_Q4_K || ty == KF_TYPE_Q5_K || ty == KF_TYPE_Q6_K) {
+        if (ty != KF_TYPE_Q4_K && (row_bytes % 16 != 0 || (int64_t)n_out * row_bytes >= (1ll << 31)))
             return fail(KF_E_UNSUPPORTED, "the q5_K/q6_K GEMM needs 16-byte aligned weights and rows (q6_K: %d columns, a multiple of 2048) and a matrix below 2 GB; kf_hip_gemv takes any", n);
         const hipError_t e = kf_launch_gemm_kq(ty, w, row_bytes, act, bias, res, y, rows, n_out, n, static_cast<hipStream_t>(stream));
         return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
@@ -317,48 +308,22 @@ int kf_hip_rms_norm_matmul(uint32_t ty, const void* w, int n_in, int n_out, cons
 
 }  // extern "C"
 
-// q4_K GEMM costs (MI355X, Llama-3-8B QKV / O / gate / down shapes at 32-2048 rows, least squares over the rounds each
-// launcher plans): the split-scale kernel (gemm_q4k.hip, 128 x 256 tiles, two K halves for a half-full last round)
-// about 7.4 us plus 4.84 us per super-block of its rounds; the one-MFMA-per-group kernel (gemm_kq.hip, 64 x 256
-// tiles, 2-4 K ranges for a half-full last round) 13.2 us plus 2.95 us. The first wins where its rounds are full
-// (gate from about 384 rows, down from 768), the second on smaller grids.
-static double q4k_gemm_us(int rows, int n_in, int n_out, bool kq) {
-    return kq ? 13.2 + 2.95 * kf_gemm_kq_sb_rounds(rows, n_out, n_in) : 7.4 + 4.84 * kf_gemm_q4k_sb_rounds(rows, n_out, n_in);
-}
-
-// Which q4_K GEMM kf_hip_gemm_i8 runs: the one-MFMA-per-group kernel where it costs less (KF_Q4K_KQ=0 / 1 forces the
-// choice, a comparison knob)
-static bool q4k_gemm_kq_pays(int rows, int n_in, int n_out) {
-    if (kf_knob_on(KF_KNOB_Q4K_KQ)) return kf_knob(KF_KNOB_Q4K_KQ) != 0;
-    return q4k_gemm_us(rows, n_in, n_out, true) < q4k_gemm_us(rows, n_in, n_out, false);
-}
-
-// q4_K: whether the tile GEMM beats the few-row product. The few-row product streams the weights once per 16
-// activation rows: about 0.28 us per MB and pass plus 1 us (fitted at the Llama shapes, 8-256 rows); the GEMM costs
-// the cheaper of the two kernels above. Rows wider than the few-row product stages go one GEMV launch per row, so the
-// GEMM takes them from 96 rows.
-static bool q4k_gemm_pays(int rows, int n_in, int n_out, int64_t row_bytes) {
-    if (rows < 2) return false;
-    if (n_in > kf_rows_max_n(KF_TYPE_Q4_K)) return rows >= 96;
+// The few-row products' cost on the K types (MI355X, us; fitted over 4-128 rows at 4096 -> 4096, 4096 -> 14336 and
+// 14336 -> 4096): about 5.5 plus, per 16 activation rows and MB of weights, 0.22 (q4_K), 0.20 (q5_K) or 0.32 (q6_K). q6_K
+// rows that start off a dword (an odd number of super-blocks) run the per-lane product, 1.35 us per MB and eight rows;
+// q4_K rows wider than the few-row product stages run as one GEMV launch per row.
+static double kq_few_rows_us(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes) {
     const double mb = (double)n_out * row_bytes / 1e6;
-    const double t_rows = ((rows + 15) / 16) * (0.28 * mb + 1.0);
-    const double t_gemm = std::min(q4k_gemm_us(rows, n_in, n_out, true), q4k_gemm_us(rows, n_in, n_out, false));
-    return t_gemm < t_rows;
+    if (ty == KF_TYPE_Q4_K && n_in > kf_rows_max_n(ty)) return rows * (2.5 + 0.22 * mb);
+    if (!kf_rows_mma_1_ok(ty, w, row_bytes, n_in, n_out, rows)) return 5.5 + (rows + 7) / 8 * (1.35 * mb + 2.0);
+    return 5.5 + (rows + 15) / 16 * mb * (ty == KF_TYPE_Q4_K ? 0.22 : ty == KF_TYPE_Q5_K ? 0.20 : 0.32);
 }
 
-// q5_K / q6_K: whether the tile GEMM beats the few-row product. The few-row product streams the weights once per 64
-// activation rows, about 1.05 (q5_K) / 1.55 (q6_K) us per MB and pass; the GEMM costs about 14.5 us plus 3.23 / 5.72
-// us per super-block of its rounds (kf_gemm_kq_sb_rounds: one 64 x 256 tile a CU a round, a last round at most half
-// full split over 2 or 4 K ranges). Fitted on MI355X at the Llama-3-8B gate and down shapes, 32-512 rows: the model
-// picks the faster product at every measured point. KF_KQ_GEMM=0 / 1 forces the choice (a comparison knob).
-static bool kq_gemm_pays(uint32_t ty, int rows, int n_in, int n_out, int64_t row_bytes) {
+// Whether the tile GEMM beats the few-row product (KF_KQ_GEMM=0 / 1 forces the choice, a comparison knob)
+static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes) {
+    if (rows < 2 || !kf_gemm_kq_ok(ty, w, row_bytes, n_in, n_out)) return false;
     if (kf_knob_on(KF_KNOB_KQ_GEMM)) return kf_knob(KF_KNOB_KQ_GEMM) != 0;
-    if (rows < 2) return false;
-    const bool q6 = ty == KF_TYPE_Q6_K;
-    const double mb = (double)n_out * row_bytes / 1e6;
-    const double t_rows = rows / 64.0 * mb * (q6 ? 1.55 : 1.05);
-    const double t_gemm = 14.5 + kf_gemm_kq_sb_rounds(rows, n_out, n_in) * (q6 ? 5.72 : 3.23);
-    return t_gemm < t_rows;
+    return kf_gemm_kq_us(ty, rows, n_out, n_in) < kq_few_rows_us(ty, w, rows, n_in, n_out, row_bytes);
 }
 
 namespace {
@@ -370,10 +335,7 @@ int product(uint32_t ty, const void* w, int64_t rb, const void* act, const float
     // several q8_0 rows are the int8 GEMM, which reads each weight byte once per 128 rows
     if (rows > 1 && ty == KF_TYPE_Q8_0 && n_in % kf_gemm_k_multiple() == 0 && n_out > 0)
         return kf_hip_gemm_i8(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream);
-    if (ty == KF_TYPE_Q4_K && n_out > 0 && q4k_gemm_pays(rows, n_in, n_out, rb))
-        return kf_hip_gemm_i8(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream);
-    if ((ty == KF_TYPE_Q5_K || ty == KF_TYPE_Q6_K) && n_out > 0 && kq_gemm_pays(ty, rows, n_in, n_out, rb) && kf_gemm_kq_ok(ty, w, rb, n_in, n_out))
-        return kf_hip_gemm_i8(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream);
+    // the K types: kf_hip_gemv picks the tile GEMM or the few-row product
     return kf_hip_gemv(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream);
 }
 
@@ -524,13 +486,8 @@ int kf_hip_moe_gemm(uint32_t ty, const void* w, const void* w2, int64_t expert_b
         return fail(KF_E_INVALID, "split at column %d of %d (a multiple of 256 inside the output) or unaligned second matrix", n_split, n_out);
     if (expert_bytes < (int64_t)mat_rows * row_bytes || expert_bytes % 16 != 0)
         return fail(KF_E_INVALID, "expert stride %lld for %d rows of %lld bytes (16-byte multiple)", (long long)expert_bytes, mat_rows, (long long)row_bytes);
-    // the one-MFMA-per-group kernel (64-row tiles: less of each slot's partial tile idle; 839 against 894 us for the
-    // split-scale kernel at 512 tokens top-2 over 8 experts) unless KF_MOE_KQ=0 (a comparison knob)
-    const bool kq = kf_knob(KF_KNOB_MOE_KQ) != 0 && row_bytes % 16 == 0 && aligned(w, 16);
-    const hipError_t e = kq ? kf_launch_gemm_kq_moe(w, w2, expert_bytes, row_bytes, w2 ? n_split : 0, act, pairs, n_slots, offsets, out_rows, y,
-                                                    n_out, n, static_cast<hipStream_t>(stream))
-                            : kf_launch_gemm_q4k_moe(w, w2, expert_bytes, row_bytes, w2 ? n_split : 0, act, pairs, n_slots, offsets, out_rows, y,
-                                                     n_out, n, static_cast<hipStream_t>(stream));
+    const hipError_t e = kf_launch_gemm_kq_moe(w, w2, expert_bytes, row_bytes, w2 ? n_split : 0, act, pairs, n_slots, offsets, out_rows, y, n_out, n,
+                                               static_cast<hipStream_t>(stream));
     return e == hipSuccess ? KF_OK : hip_fail(e, "grouped GEMM launch");
 }
 

@@ -1,25 +1,37 @@
-// Prefill GEMM on native q5_K and q6_K bytes: y[m][n] = sum over super-blocks b of dx[m][b] * (d[n][b] * S_b[m][n]
-// - dmin[n][b] * mins_b[m][n]) (+ bias[n] + res[m][n]), with S_b the reference's exact super-block integer:
-//   * q5_K (crates/kf-quant/src/types/q5_k.rs): S_b = sum_g sc_g I_g over the eight 32-column groups, I_g the int32
-//     dot of the group's 5-bit values (the fifth bit from qh) with the int8 activations; mins_b = sum_g m_g bsum_g;
+// Tile GEMM on native q4_K, q5_K and q6_K bytes, from a few rows to prefill, one matrix or the grouped experts:
+// y[m][n] = sum over super-blocks b of dx[m][b] * (d[n][b] * S_b[m][n] - dmin[n][b] * mins_b[m][n]) (+ bias[n] + res[m][n]),
+// with S_b the reference's exact super-block integer:
+//   * q4_K, q5_K (crates/kf-quant/src/types/q4_k.rs:10-58, q5_k.rs): S_b = sum_g sc_g I_g over the eight 32-column groups,
+//     I_g the int32 dot of the group's values with the int8 activations; mins_b = sum_g m_g bsum_g;
 //   * q6_K (crates/kf-quant/src/types/q6_k.rs): S_b = sum_s sc_s (dot_s - 32 bsum_s) over the sixteen 16-column
-//     sub-blocks with int8 scales, formed as sum_s sc_s dot'_s with the operand q - 32 (an int8); no mins term.
+//     sub-blocks with int8 scales, formed as sum_s sc_s dot'_s with the operand q - 32; no mins term.
 // It replaces the reference's unpack + KF8 GEMM for these types (crates/kf-backend-cuda/src/kernels/quant.cuh:585-601,
-// KF_QUANT_KERNELS_I8 in quant_q5_K.cu:114 / quant_q6_K.cu:131, kf8.cu:116-369), reading the native bytes directly.
+// kf8.cu:116-369, 400-416), reading the native bytes directly.
 //
-// Arithmetic: per group and 32 x 32 tile one v_mfma_i32_32x32x32_i8 gives I_g exactly (q6_K: two, each with the
-// other 16 columns' operand bytes zeroed, for the two scales of the group); S_b accumulates by 24-bit multiply-adds
-// with the integer sub-scales (every product below 2^23), mins_b by one exact v_mfma_f32_32x32x16_f16 against
-// quant_act's split sums (as the q4_K GEMM), and the float rescale runs once per super-block and output.
+// Arithmetic: the product scale x value of every weight, v, is exact in two int8 planes, v = lo + (hi << SHIFT): q4_K's
+// nibble times the 6-bit scale's two 3-bit halves, q5_K's and q6_K's 16-bit product split into its signed low byte and
+// the rest. Two v_mfma_i32_32x32x32_i8 chains a 32 x 32 tile run through the super-block, so S_b needs no work per group;
+// mins_b is one exact v_mfma_f32_32x32x16_f16 against quant_act's split sums, and the float rescale runs once per
+// super-block and output (five VALU instructions). A form with one MFMA a group and the scales applied to its results by
+// multiply-adds spent 2-3 times the vector work of this one on q5_K and q6_K.
 //
-// Schedule: eight waves (two a SIMD), one block a CU, block tile 64 x 256: each wave a 64 x 32 tile (two 32 x 32
-// MFMA tiles down M, one weight column tile), so a wave's weight operands serve two MFMAs. One super-block (K = 256)
-// per stage, two stage buffers: activations [row 64][256] with the 16-byte chunk swizzle c ^ (row % 16), weights
-// [row 256][WROW] (q5_K: the 176-byte super-block; q6_K: the 224-byte 16-byte aligned window around the 210-byte
-// block, which needs rows that start 16-byte aligned: K a multiple of 2048), the stage's activation scales and (q5_K)
-// mins operands. Every DMA instruction reads whole 16-byte pieces of consecutive rows, issued through inline assembly
-// with explicit waits; rows past M or N read as zeros through the hardware range check. Blocks run in XCD order (each
-// XCD a contiguous range of tiles, M fastest), so the blocks in flight on an XCD share their weight tiles in its L2.
+// Schedule: eight waves (two a SIMD), one block a CU, block tile 32 TM x 256, each wave a column of TM 32 x 32 tiles, so a
+// weight operand is expanded once for TM tiles. The operands of a whole super-block stay in registers (64) and the tiles
+// run one after another, eight group steps each: a step's two MFMAs go with an eighth of the previous tile's rescale
+// and, in the last tile, with the expansion of the next super-block's operands, so no phase of a wave is without MFMAs
+// and the two waves of a SIMD need no offset. What bounds it at TM = 4: MFMA busy 47% and VALU issue 51% of the cycles,
+// which overlap only in part, and LDS and DMA waits. Choices that measured (2048 rows, us): reloads of spilled registers
+// in the K loop wait for every load in flight (446 -> 295, 4096 -> 14336 q4_K); the loads of a super-block spread over
+// the steps instead of all at its start, where eight waves queue them behind each other, and each step's LDS
+// reads one step ahead (267 -> 241, 14336 -> 4096 q4_K).
+// Weights land by DMA in each wave's own LDS buffers ([row 32][WROW]; q6_K: the 16-byte aligned window around the 210-byte
+// block, whose rows may start at any even byte, so every width of whole super-blocks is taken), activations in buffers all
+// waves share ([tile][row 32][256] with the 16-byte chunk swizzle c ^ (row % 16)); every wait is explicit. Blocks run in
+// XCD order, so the blocks in flight on an XCD share their weight tiles in its L2.
+// Measured, us, before (the one-MFMA form on q5_K / q6_K, a 128 x 256 tile kernel without the interleaved rescale on q4_K, the
+// per-lane product on q6_K rows off 16 bytes) and now, 4096 -> 14336 / 14336 -> 4096: 2048 rows q4_K 281 / 260 -> 270 / 239, q5_K
+// 370 / 345 -> 304 / 272, q6_K 620 / 597 -> 325 / 287; 128 rows q4_K 46 / 62 -> 34 / 32, q5_K 74 / 78 -> 36 / 37, q6_K
+// 138 / 125 -> 39 / 40; 63 rows of q6_K 2816 -> 7052 305 -> 25.
 #include "kf_knobs.h"
 #include "kf_blocks.h"
 #include "kf_device.h"
@@ -27,10 +39,9 @@
 
 #include <type_traits>
 
-// The split-K fixups rely on gfx9 cache behaviour (system-scope relaxed atomics write through to memory, stores are
-// counted in vmcnt), not on a release/acquire pair: build for gfx950 only.
+// The K loop relies on gfx950's LDS DMA and vmcnt order: build for gfx950 only.
 #if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
-#error "the split-K fixups assume gfx950's cache and counter behaviour"
+#error "the DMA waits assume gfx950"
 #endif
 
 namespace {
@@ -43,50 +54,78 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 
 constexpr int KQ_WAVES = 8, KQ_THREADS = 64 * KQ_WAVES;
-constexpr int KQ_TM = 2;                       // 32-row tiles per wave (all of the block's rows)
-constexpr int KQ_BM = 32 * KQ_TM;              // 64
-constexpr int KQ_BN = 32 * KQ_WAVES;           // 256: one 32-column tile per wave
+constexpr int KQ_BN = 32 * KQ_WAVES;  // 256: one 32-column tile per wave
+constexpr int KQ_LDS = 160 * 1024;
+constexpr int KQ_EPI = 256;  // LDS for the parked state
+// Cost model of a launch (MI355X, us; least squares over 4-2048 rows at 2048 -> 6144, 4096 -> 4096, 4096 -> 14336 and
+// 14336 -> 4096, rms 3-8%): 1.8 for the launch, KQ_ROUND_US a round of the CUs (a block's first loads and its stores), the
+// super-blocks of the rounds, and the partial tiles' way through memory where the tail is split (per CU's worth of them).
+// The tile height is the cheapest by it: few rows take short tiles (32 rows of 14336 -> 4096 q4_K: 19 / 22 / 29 us with 1 / 2 / 4
+// tiles), 2048 tall ones (373 / 292 / 239).
+constexpr double KQ_ROUND_US[3] = {4.2, 4.8, 5.6};                                               // [1, 2, 4 tiles]
+constexpr double KQ_SB_US[3][3] = {{1.60, 2.44, 4.01}, {2.46, 3.23, 4.66}, {3.03, 3.83, 5.03}};  // [q4_K, q5_K, q6_K][1, 2, 4 tiles]
+constexpr double KQ_PART_US[3] = {6.2, 4.5, 2.4};                                                // per tile row, [1, 2, 4 tiles]
 
-template <uint32_t TY>
+// LDS of a block of TM 32-row tiles: NA buffers of a super-block's activations ([tile][row 32][256]), NW buffers a wave of
+// its 32 weight rows' super-block ([row 32][WROW]), NS records of a super-block's activation scales and mins operands.
+template <uint32_t TY, int TM>
 struct KqGeo {
-    static constexpr bool Q6 = TY == KF_TYPE_Q6_K, Q4 = TY == KF_TYPE_Q4_K;
+    static constexpr bool Q6 = TY == KF_TYPE_Q6_K, Q4 = TY == KF_TYPE_Q4_K, Q5 = TY == KF_TYPE_Q5_K;
+    static constexpr int BM = 32 * TM;
     static constexpr int SBB = Q6 ? KF_Q6_K_BYTES : Q4 ? KF_Q4_K_BYTES : KF_Q5_K_BYTES;  // bytes of a super-block
-    static constexpr int WROW = Q6 ? 224 : SBB;                      // LDS bytes of a weight row's super-block
-    static constexpr int QS = Q4 ? 16 : 48;                          // q4_K / q5_K: the nibbles' offset
-    static constexpr int PR = WROW / 16;                             // its 16-byte pieces
-    static constexpr int A = 0;                                      // activations [row 64][256]
-    static constexpr int W = A + KQ_BM * 256;                        // weights [row 256][WROW]
-    static constexpr int DX = W + KQ_BN * WROW;                      // activation scales [row 64] f32
-    static constexpr int XS = DX + KQ_BM * 4;                        // q5_K: mins operands [row 64][16] f16
-    static constexpr int STAGE = XS + (Q6 ? 0 : KQ_BM * 32);
-    static constexpr int NA = KQ_BM * 256 / 1024;                    // activation DMA instructions (4 rows each)
-    static constexpr int NW = (KQ_BN * PR + 63) / 64;                // weight DMA instructions (64 pieces each)
-    static_assert(NA % KQ_WAVES == 0, "whole activation instructions a wave");
-    static_assert(2 * STAGE <= 160 * 1024, "two stages fit the LDS");
+    static constexpr int WROW = Q6 ? 224 : SBB;   // LDS bytes of a weight row's super-block (q6_K: its 16-byte aligned window)
+    static constexpr int QS = Q4 ? 16 : 48;       // q4_K / q5_K: the nibbles' offset
+    static constexpr int PR = WROW / 16;          // 16-byte pieces of a row's super-block
+    static constexpr int PW = 32 * PR;            // pieces of a wave's rows
+    static constexpr int NWI = (PW + 63) / 64;    // weight DMA instructions a wave and super-block
+    static constexpr int NSI = Q6 ? 1 : 2;        // record DMA instructions a wave and super-block
+    static constexpr int SHIFT = Q4 ? 3 : 8;      // S = S_lo + (S_hi << SHIFT)
+    static constexpr int ABUF = BM * 256;
+    static constexpr int WBUF = 32 * WROW;        // one wave's
+    static constexpr int REC = BM * (Q6 ? 4 : 36);  // dx f32 [BM], then the mins operands f16 [BM][16]
+    static constexpr int NA = TM == 1 ? 3 : 2;
+    static constexpr int NS = NA + 1;             // one more than ahead: a tile is rescaled one super-block late
+    static constexpr int ROOM = KQ_LDS - KQ_EPI - NA * ABUF - NS * REC;
+    static constexpr int NW = ROOM >= 3 * KQ_WAVES * WBUF ? 3 : ROOM >= 2 * KQ_WAVES * WBUF ? 2 : 1;
+    static constexpr int A = 0, W = A + NA * ABUF, R = W + NW * KQ_WAVES * WBUF, LDS = R + NS * REC;
+    static_assert(LDS + KQ_EPI <= KQ_LDS, "the buffers fit the LDS");
+    // vector memory operations issued after the loads that the next super-block needs, where they are waited for
+    static constexpr int wait(int TL) {
+        const int batch = NSI + TL + NWI;
+        const int w = (NW - 1) * batch, a = NWI + (NA - 2) * batch;
+        return w < a ? w : a;
+    }
 };
 
-// XCD-aware tile order over the first T tiles: block b < T runs tile (b % 8) (T / 8) + b / 8 (tiles numbered
-// M-fastest), so XCD x (blocks go to the eight XCDs round-robin) works through a contiguous range of weight tiles
-// against every activation panel. Identity when T is not a multiple of eight.
-__device__ __forceinline__ void kq_tile(int T, int mt, int b, int& tm, int& tn) {
-    const int t = (T & 7) ? b : (b & 7) * (T >> 3) + (b >> 3);
-    tn = t / mt;
-    tm = t - tn * mt;
-}
+// XCD-aware order over T work items: block b < T runs item (b % 8) (T / 8) + b / 8, so XCD x (blocks go to the eight
+// XCDs round-robin) works through a contiguous range of weight tiles against every activation panel. Identity when T is
+// not a multiple of eight.
+__device__ __forceinline__ int kq_order(int T, int b) { return (T & 7) ? b : (b & 7) * (T >> 3) + (b >> 3); }
 
-// The grid's tail: the tiles from `full` on (a last round of blocks at most half full, or a whole grid below half
-// the CUs) run as S blocks each over S consecutive ranges of K; each writes its 64 x 256 partial tile to `part`
-// ([tail tile][split][register][thread]), and the last of them to arrive (a ticket per tail tile) adds all S in split
-// order and stores the tile. part == nullptr: no split.
-struct KqTail {
+// A tile whose super-blocks several range blocks shared: its rows and columns and how many partial tiles make it (0: none)
+struct KqDesc {
+    int m0, m_end, n0, count;
+};
+
+// The launch's work besides whole tiles. Partial tiles go to `part` ([slot][register][thread]) and kq_reduce_kernel adds
+// them.
+//  * One matrix: tiles below `full` (whole rounds of the CUs) are a block each; the others run as S blocks each, over S
+//    consecutive ranges of K (slot S t + range for the t-th of them). part == nullptr: every tile is a block.
+//  * Grouped: the tiles of all slots are laid end to end, super-block after super-block, and cut into G equal ranges, a
+//    block each, so that every CU gets the same work however the pairs fall on the slots; a tile weighs its number of
+//    32-row parts plus one (the weight side). A tile inside a range is stored directly; of a tile that is cut, every
+//    block leaves its part (slot 2 b + 1 for the part with the tile's first super-block, 2 b otherwise: a range has at
+//    most one of each) and the block with its start describes it in desc[b]. part == nullptr: a range takes the tiles
+//    that start in it, whole.
+struct KqWork {
     float* part;
-    int* tickets;
-    int full, S;
+    KqDesc* desc;
+    int full, S;  // grouped: full is unused, S is G
 };
 
 // The grouped (MoE) form: the activation rows are routed pairs in group order (slot s: rows offsets[s]..offsets[s + 1]),
 // slot s multiplies its own expert matrix (w + s expert_bytes; with w2, output columns from n_split on come from
-// w2 + s expert_bytes, row n - n_split), and output row p goes to y row out_rows[p] (or p). n_slots == 0: one matrix.
+// w2 + s expert_bytes, row n - n_split), and output row p goes to y row out_rows[p] (or p).
 struct KqMoe {
     const int32_t* offsets;
     const int32_t* out_rows;
@@ -95,447 +134,833 @@ struct KqMoe {
     int n_slots, n_split;
 };
 
-template <uint32_t TY, bool MOE>
-__global__ void __launch_bounds__(KQ_THREADS, 1) gemm_kq_kernel(const uint8_t* __restrict__ w, int64_t row_bytes,
-                                                                 const int8_t* __restrict__ xq, const _Float16* __restrict__ xa,
-                                                                 const float* __restrict__ xd32, const float* __restrict__ bias,
-                                                                 const float* __restrict__ res, float* __restrict__ y, int M, int N, int K,
-                                                                 KqTail tail_arg, KqMoe moe) {
-    const KqTail tail = MOE ? KqTail{nullptr, nullptr, 0, 1} : tail_arg;  // the dense form's tail split
-    // the grouped form splits K in two over every tile when its launcher passes the scratch (msplit)
-    const bool msplit = MOE && tail_arg.part != nullptr;
-    using G = KqGeo<TY>;
-    __shared__ __align__(16) uint8_t buf0[G::STAGE];
-    __shared__ __align__(16) uint8_t buf1[G::STAGE];
-    const int tid = threadIdx.x, lane = tid & 63;
+// kf_adma16 / kf_adma4 by the first LANES lanes only: the mask is set around the one instruction instead of by a branch,
+// which would cut the K loop's steps into small basic blocks (70 spilled registers). For uniform control flow of whole
+// waves.
+template <int LANES>
+__device__ __forceinline__ void kq_adma16(kf_arsrc_t r, int voff, int soff, const void* lds) {
+    static_assert(LANES > 0 && LANES < 64, "a part of the wave");
+    asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 exec, %4\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds\n\ts_mov_b64 exec, -1" ::"v"(voff),
+                 "s"(r), "s"(soff), "s"(kf_lds_addr(lds)), "s"((1ull << LANES) - 1)
+                 : "memory", "m0");
+}
+template <int LANES>
+__device__ __forceinline__ void kq_adma4(kf_arsrc_t r, int voff, int soff, const void* lds) {
+    static_assert(LANES > 0 && LANES < 64, "a part of the wave");
+    asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 exec, %4\n\tbuffer_load_dword %0, %1, %2 offen lds\n\ts_mov_b64 exec, -1" ::"v"(voff),
+                 "s"(r), "s"(soff), "s"(kf_lds_addr(lds)), "s"((1ull << LANES) - 1)
+                 : "memory", "m0");
+}
+
+// Grouped form: a block's arguments and the state of its range, parked in LDS while a K loop runs (kept in scalar registers
+// across the loop they would spill). Written by thread 0 between barriers, read as wave-uniform values.
+struct KqState {
+    const uint8_t *w, *w2;
+    const int8_t* xq;
+    const _Float16* xa;
+    const float* xd;
+    float* y;
+    const int32_t *offsets, *out_rows;
+    float* part;
+    KqDesc* desc;
+    int64_t row_bytes, expert_bytes;
+    int N, K, n_slots, n_split;
+    int b, G, U, u, u_end, slots_w;     // the range block, the ranges, their total, this block's position and end
+    int m0, m_end, n0, s0, s1, next;    // the tile in hand, its super-blocks here and where the next one starts
+    int count;                          // partial tiles of a tile that starts here and goes on
+};
+static_assert(sizeof(KqState) <= KQ_EPI, "the parked state fits");
+
+__device__ __forceinline__ int kq_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int64_t kq_uniform(int64_t v) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)v >> 32));
+    return (int64_t)((uint64_t)hi << 32 | lo);
+}
+template <typename T>
+__device__ __forceinline__ T* kq_uniform(T* p) {
+    return reinterpret_cast<T*>(kq_uniform((int64_t)reinterpret_cast<uint64_t>(p)));
+}
+
+// Grouped form: the weight of a slot of `rows` rows (per super-block and column tile) in tiles of TM 32-row parts
+template <int TM>
+__device__ __forceinline__ int kq_slot_w(int rows) {
+    const int full = rows / (32 * TM), rest = rows - full * 32 * TM;
+    return full * (TM + 1) + (rest > 0 ? (rest + 31) / 32 + 1 : 0);
+}
+
+// The sum of the slots' weights (every lane of the wave calls it)
+template <int TM>
+__device__ int kq_slots_w(const int32_t* __restrict__ offsets, int n_slots) {
+    int t = 0;
+    for (int s = threadIdx.x & 63; s < n_slots; s += 64) t += kq_slot_w<TM>(offsets[s + 1] - offsets[s]);
+    return kq_uniform(kf_wave_isum(t));
+}
+
+// The slot whose weight range holds position q, and the position inside it
+template <int TM>
+__device__ int kq_find_slot(const int32_t* __restrict__ offsets, int n_slots, int& q) {
+    const int lane = threadIdx.x & 63;
+    for (int base = 0;; base += 64) {
+        const int s = base + lane;
+        int v = s < n_slots ? kq_slot_w<TM>(offsets[s + 1] - offsets[s]) : 0;
+        const int own = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(v, o, 64);
+            if (lane >= o) v += u;
+        }
+        const uint64_t hit = __ballot(v > q);
+        if (hit || base + 64 >= n_slots) {
+            const int l = hit ? __builtin_ctzll(hit) : 63;
+            q -= __builtin_amdgcn_readlane(v, l) - __builtin_amdgcn_readlane(own, l);
+            return min(base + l, n_slots - 1);
+        }
+        q -= __builtin_amdgcn_readlane(v, 63);
+    }
+}
+
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t kq_pk_mul(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b)));
+}
+__device__ __forceinline__ uint32_t kq_pk_mad(uint32_t a, uint32_t b, uint32_t c) {
+    return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b) + __builtin_bit_cast(u16x2, c)));
+}
+
+// Byte B of v in both 16-bit halves, zero- or sign-extended
+template <int B>
+__device__ __forceinline__ uint32_t kq_pair(uint32_t v) {
+    return __builtin_amdgcn_perm(v, v, 0x0c000c00u | (uint32_t)B << 16 | B);
+}
+template <int B>
+__device__ __forceinline__ uint32_t kq_pair_signed(uint32_t v) {
+    typedef short i16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, (i16x2)(__builtin_bit_cast(i16x2, __builtin_amdgcn_perm(v, v, 0x000c000cu | (uint32_t)B << 24 | B << 8)) >> (short)8));
+}
+
+// The two int8 operand planes of one group for a lane: its 16 columns' products v = scale x value, v = lo + (hi << SHIFT)
+struct KqPlanes {
+    v4i lo, hi;
+};
+
+// Four products v + 128 as 16-bit pairs (e: bytes 0 and 2, o: bytes 1 and 3 of the four), split into the signed low byte
+// and the rest: v + 128 = 256 hi + b, v = 256 hi + (b - 128)
+__device__ __forceinline__ int kq_low16(uint32_t e, uint32_t o) { return (int)(__builtin_amdgcn_perm(o, e, 0x06020400u) ^ 0x80808080u); }
+__device__ __forceinline__ int kq_high16(uint32_t e, uint32_t o) { return (int)__builtin_amdgcn_perm(o, e, 0x07030501u); }
+
+// A wave's weight column (32 lanes a tile, each lane half the group's columns) being expanded, one super-block at a time
+template <uint32_t TY, int TM>
+struct KqWeight {
+    using G = KqGeo<TY, TM>;
+    uint32_t sc[2], sh[2], mn[2];  // q4_K / q5_K: the eight 6-bit scales (q4_K: their low and high three bits) and mins
+    uint32_t sw[4];               // q6_K: the sixteen int8 scales, shifted so that group g's is byte 2 (g % 2) of word g / 2
+    uint32_t d16;                 // d (low), dmin (high)
+    uint4 raw, raw2, qh;
+
+    // the header, and the first group's bytes
+    __device__ __forceinline__ void begin(const uint8_t* wr, int half) {
+        if constexpr (G::Q6) {
+            const u32x4_a2 s = *reinterpret_cast<const u32x4_a2*>(wr + 192);
+#pragma unroll
+            for (int k = 0; k < 4; k++) sw[k] = s[k] >> (8 * half);
+            d16 = *reinterpret_cast<const uint16_t*>(wr + 208);
+        } else {
+            const uint4 hd = *reinterpret_cast<const uint4*>(wr);
+            kf_q4k_scales8(hd.y, hd.z, hd.w, sc, mn);
+            if constexpr (G::Q4) {
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    sh[k] = (sc[k] >> 3) & 0x07070707u;
+                    sc[k] &= 0x07070707u;
+                }
+            }
+            d16 = hd.x;
+            if constexpr (G::Q5) qh = *reinterpret_cast<const uint4*>(wr + 16 + 16 * half);
+        }
+        fetch<0>(wr, half);
+    }
+
+    // group g's bytes into registers (q4_K / q5_K: a pair of groups shares its 16 bytes; q6_K: four groups share 48)
+    template <int g>
+    __device__ __forceinline__ void fetch(const uint8_t* wr, int half) {
+        if constexpr (G::Q6) {
+            if constexpr (g % 4 == 0) {
+                const u32x4_a2 a = *reinterpret_cast<const u32x4_a2*>(wr + 16 * g + 16 * half);
+                const u32x4_a2 b = *reinterpret_cast<const u32x4_a2*>(wr + 16 * g + 32 + 16 * half);
+                const u32x4_a2 h = *reinterpret_cast<const u32x4_a2*>(wr + 128 + 8 * g + 16 * half);
+                raw = make_uint4(a.x, a.y, a.z, a.w);
+                raw2 = make_uint4(b.x, b.y, b.z, b.w);
+                qh = make_uint4(h.x, h.y, h.z, h.w);
+            }
+        } else if constexpr (g % 2 == 0) {
+            raw = *reinterpret_cast<const uint4*>(wr + G::QS + 16 * g + 16 * half);
+        }
+    }
+
+    template <int g>
+    __device__ __forceinline__ KqPlanes planes() const {
+        KqPlanes p;
+        const uint32_t m4 = 0x0f0f0f0fu, mb = 0x00ff00ffu;
+        if constexpr (G::Q4) {
+            // 6-bit scale 8 sh + sl: the nibble products q sl and q sh (at most 105) are bytes, two to a 16-bit product
+            const uint32_t v[4] = {raw.x, raw.y, raw.z, raw.w};
+            const uint32_t s0 = kq_pair<g & 3>(sc[g >> 2]), s1 = kq_pair<g & 3>(sh[g >> 2]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t q = ((g & 1) ? v[e] >> 4 : v[e]) & m4;
+                p.lo[e] = (int)kq_pk_mul(q, s0);
+                p.hi[e] = (int)kq_pk_mul(q, s1);
+            }
+        } else if constexpr (G::Q5) {
+            const uint32_t v[4] = {raw.x, raw.y, raw.z, raw.w}, h[4] = {qh.x, qh.y, qh.z, qh.w};
+            const uint32_t s = kq_pair<g & 3>(sc[g >> 2]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t q = (((g & 1) ? v[e] >> 4 : v[e]) & m4) | (((h[e] >> g) & 0x01010101u) << 4);
+                const uint32_t ev = kq_pk_mad(q & mb, s, 0x00800080u), ov = kq_pk_mad((q >> 8) & mb, s, 0x00800080u);
+                p.lo[e] = kq_low16(ev, ov);
+                p.hi[e] = kq_high16(ev, ov);
+            }
+        } else {
+            // q6_K group 4 h + k: the low (k < 2) or high nibbles of run k % 2 and bits 2 k.. of qh; v = sc (q - 32)
+            const uint32_t v[4] = {(g & 1) ? raw2.x : raw.x, (g & 1) ? raw2.y : raw.y, (g & 1) ? raw2.z : raw.z, (g & 1) ? raw2.w : raw.w};
+            const uint32_t h[4] = {qh.x, qh.y, qh.z, qh.w};
+            const uint32_t s = kq_pair_signed<2 * (g & 1)>(sw[g >> 1]);
+            const uint32_t c = kq_pk_mad(s, 0xffe0ffe0u, 0x00800080u);  // 128 - 32 sc
+            constexpr int k = g & 3;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t lo = ((k & 2) ? v[e] >> 4 : v[e]) & m4;
+                const uint32_t q = lo | (((h[e] >> (2 * k)) & 0x03030303u) << 4);
+                const uint32_t ev = kq_pk_mad(q & mb, s, c), ov = kq_pk_mad((q >> 8) & mb, s, c);
+                p.lo[e] = kq_low16(ev, ov);
+                p.hi[e] = kq_high16(ev, ov);
+            }
+        }
+        return p;
+    }
+
+    // the mins operand: per lane the eight mins, times 64 for the lanes that meet the high parts of the group sums
+    __device__ __forceinline__ v8h mins(int half) const {
+        // 1024 + m as f16 bits, less 1024, times f: exact
+        typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+        const _Float16 f = half ? (_Float16)1.0f : (_Float16)64.0f;
+        v8h mo;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint32_t u = __builtin_amdgcn_perm(0x64646464u, mn[k >> 1], (k & 1) ? 0x04030402u : 0x04010400u);
+            const v2h m = __builtin_bit_cast(v2h, u) - (v2h){(_Float16)1024.0f, (_Float16)1024.0f};
+            mo[2 * k] = m[0] * f;
+            mo[2 * k + 1] = m[1] * f;
+        }
+        return mo;
+    }
+};
+
+template <uint32_t TY, int TM, bool MOE>
+__global__ void __launch_bounds__(KQ_THREADS, 2) gemm_kq_kernel(const uint8_t* w_, int64_t row_bytes_, const int8_t* xq_, const _Float16* xa_,
+                                                                 const float* xd_, const float* bias_, const float* res_, float* y_, int M_, int N_,
+                                                                 int K_, KqWork work, KqMoe moe) {
+    using G = KqGeo<TY, TM>;
+    constexpr int BM = G::BM;
+    extern __shared__ __align__(256) uint8_t lds[];
+    KqState& st = *reinterpret_cast<KqState*>(lds + G::LDS);
+    if constexpr (MOE) {
+        // positions are super-blocks times tile weights, from the first tile of all
+        const int nsb = K_ >> 8, NT = (N_ + KQ_BN - 1) / KQ_BN;
+        const int sw = kq_slots_w<TM>(moe.offsets, moe.n_slots), U = NT * nsb * sw;
+        const int Gr = max(min(work.S, U / (4 * (TM + 1))), U > 0 ? 1 : 0);  // at least a few super-blocks a range
+        const bool idle = (int)blockIdx.x >= Gr;
+        const int b = idle ? blockIdx.x : kq_order(Gr, blockIdx.x);
+        if (threadIdx.x == 0 && work.desc) work.desc[b].count = 0;
+        if (idle) return;  // nothing to do: whole block, before any barrier
+        if (threadIdx.x == 0)
+            st = KqState{w_, moe.w2, xq_, xa_, xd_, y_, moe.offsets, moe.out_rows, work.part, work.desc, row_bytes_, moe.expert_bytes, N_, K_,
+                         moe.n_slots, moe.n_split, b, Gr, U, (int)((int64_t)U * b / Gr), (int)((int64_t)U * (b + 1) / Gr), sw, 0, 0, 0, 0, 0, 0, 0};
+    }
+    for (;;) {  // grouped: a range's tiles; otherwise one pass
+    if constexpr (MOE) __syncthreads();  // the state is written, and every wave is done with the LDS of the tile before
+    // the thread's indices, made anew for each tile: what derives from them is not kept from tile to tile
+    int tid = threadIdx.x;
+    if constexpr (MOE) __asm__ volatile("" : "+v"(tid));
+    const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int half = lane >> 5, r32 = lane & 31;
-    __shared__ int last;
-    const int mt = (M + KQ_BM - 1) / KQ_BM;
-    const int kg = K >> 5;
-    const int nsb = K >> 8;
-    int tm, tn;
-    int s0 = 0, s1 = nsb, sp = -1, tt = 0;  // super-blocks [s0, s1); a tail block's split and tail tile
-    if (!MOE && tail.part && (int)blockIdx.x >= tail.full) {
-        const int b = blockIdx.x - tail.full;
-        tt = b / tail.S;
-        sp = b - tt * tail.S;
-        const int t = tail.full + tt;
-        tn = t / mt;
-        tm = t - tn * mt;
-        s0 = nsb * sp / tail.S;
-        s1 = nsb * (sp + 1) / tail.S;
-    } else if (msplit) {
-        // the two K halves of tile tt, in XCD order: XCD x (blocks go to the eight XCDs round-robin) takes a contiguous
-        // range of tiles, both halves of each, so the blocks of an expert's weight tiles share them in its L2
-        const int T = ((N + KQ_BN - 1) / KQ_BN) * mt, b = blockIdx.x;
-        if ((T & 7) == 0) {
-            tt = (b & 7) * (T >> 3) + (b >> 4);
-            sp = (b >> 3) & 1;
-        } else {
-            tt = b >> 1;
-            sp = b & 1;
+    const int N = MOE ? kq_uniform(st.N) : N_, K = MOE ? kq_uniform(st.K) : K_;
+    const int64_t row_bytes = MOE ? kq_uniform(st.row_bytes) : row_bytes_;
+    const int kg = K >> 5, nsb = K >> 8;
+    int s0 = 0, s1 = nsb, m0, m_end, n0, nr0, n_rows = N, slot = -1;  // slot: the partial tile's place (-1: a whole tile)
+    const uint8_t* wt = MOE ? kq_uniform(st.w) : w_;
+    if constexpr (MOE) {
+        // the tile at the range's position
+        const int u = kq_uniform(st.u), u_end = kq_uniform(st.u_end);
+        const int sw = kq_uniform(st.slots_w), per = sw * nsb;
+        const int tn = u / per;
+        const int q = u - tn * per, q0 = q / nsb;
+        int qs = q0;
+        const int32_t* offsets = kq_uniform(st.offsets);
+        const int sl = kq_find_slot<TM>(offsets, kq_uniform(st.n_slots), qs);
+        const int r0 = kq_uniform(offsets[sl]), r1 = kq_uniform(offsets[sl + 1]);
+        const int slot_pos = (q0 - qs) * nsb;  // the slot's first position in the column tile
+        const int i = min((q - slot_pos) / (nsb * (TM + 1)), (r1 - r0) / BM);
+        m0 = r0 + i * BM;
+        m_end = r1;
+        const int wgt = (min(r1 - m0, BM) + 31) / 32 + 1;
+        const int start = tn * per + slot_pos + i * nsb * (TM + 1), end = start + nsb * wgt;
+        n0 = tn * KQ_BN;
+        nr0 = n0;
+        const uint8_t* w2 = kq_uniform(st.w2);
+        if (w2) {
+            const int split = kq_uniform(st.n_split);
+            n_rows = split;
+            if (n0 >= split) {
+                wt = w2;
+                nr0 = n0 - split;
+                n_rows = N - split;
+            }
         }
-        tn = tt / mt;
-        tm = tt - tn * mt;
-        s0 = nsb * sp / 2;
-        s1 = nsb * (sp + 1) / 2;
+        wt += sl * kq_uniform(st.expert_bytes);
+        s0 = (u - start) / wgt;
+        s1 = u_end >= end ? nsb : (u_end - start) / wgt;
+        if (!kq_uniform(st.part)) s1 = u > start ? s0 : nsb;  // no scratch: whole tiles
+        int count = 0;
+        if (s0 == 0 && s1 < nsb) {
+            // the blocks after this one, up to the one that reaches the tile's end
+            const int b = kq_uniform(st.b), Gr = kq_uniform(st.G), U = kq_uniform(st.U);
+            count = 2;
+            while ((int64_t)U * (b + count) / Gr < end) count++;
+        }
+        s0 = kq_uniform(s0);
+        s1 = kq_uniform(s1);
+        m0 = kq_uniform(m0);
+        m_end = kq_uniform(m_end);
+        n0 = kq_uniform(n0);
+        __syncthreads();  // every wave has read the position
+        if (tid == 0) {
+            st.m0 = m0;
+            st.m_end = m_end;
+            st.n0 = n0;
+            st.s0 = s0;
+            st.s1 = s1;
+            st.next = end;
+            st.count = count;
+        }
     } else {
-        kq_tile(tail.part ? tail.full : ((N + KQ_BN - 1) / KQ_BN) * mt, mt, blockIdx.x, tm, tn);
-    }
-    int m0 = tm * KQ_BM;
-    const int n0 = tn * KQ_BN;
-    int m_end = M;  // rows of the block's slot end here
-    const uint8_t* wt = w + (int64_t)n0 * row_bytes;
-    int n_end = N;  // columns of the block's matrix end here (as output columns)
-    if (MOE) {
-        // M counts the grid's row tiles over all slots (an upper bound): tile tm is the slot's tile tm - (the tiles of
-        // the slots before it); past the last slot's tiles the block has nothing to do
-        int sl = 0, t0 = 0;
-        for (; sl < moe.n_slots; sl++) {
-            const int rows = moe.offsets[sl + 1] - moe.offsets[sl], t = (rows + KQ_BM - 1) / KQ_BM;
-            if (tm < t0 + t) break;
-            t0 += t;
-        }
-        if (sl == moe.n_slots) return;  // whole block, before any barrier
-        m0 = moe.offsets[sl] + (tm - t0) * KQ_BM;
-        m_end = moe.offsets[sl + 1];
-        if (moe.w2 && n0 >= moe.n_split) {
-            wt = moe.w2 + sl * moe.expert_bytes + (int64_t)(n0 - moe.n_split) * row_bytes;
+        const int mt = (M_ + BM - 1) / BM;
+        int t;
+        if (work.part && (int)blockIdx.x >= work.full) {
+            slot = blockIdx.x - work.full;
+            const int tt = slot / work.S, sp = slot - tt * work.S;
+            t = work.full + tt;
+            s0 = nsb * sp / work.S;
+            s1 = nsb * (sp + 1) / work.S;
         } else {
-            wt = w + sl * moe.expert_bytes + (int64_t)n0 * row_bytes;
-            if (moe.w2) n_end = moe.n_split;
+            t = kq_order(work.full, blockIdx.x);
         }
+        const int tn = t / mt;
+        m0 = (t - tn * mt) * BM;
+        m_end = M_;
+        n0 = tn * KQ_BN;
+        nr0 = n0;
+        s0 = kq_uniform(s0);
+        s1 = kq_uniform(s1);
     }
-
-    const kf_arsrc_t rw = kf_arsrc(wt, (uint64_t)(n_end - n0) * row_bytes);
-    const kf_arsrc_t rx = kf_arsrc(xq + (int64_t)m0 * K, (uint64_t)(m_end - m0) * K);
-    const kf_arsrc_t rs = kf_arsrc(xa + (int64_t)m0 * nsb * 16, (uint64_t)(m_end - m0) * nsb * 32);
-    const kf_arsrc_t rd = kf_arsrc(xd32 + (int64_t)m0 * kg, (uint64_t)(m_end - m0) * kg * 4);
-    // activation instruction i (rows 4 i..) is wave i % 8's: lane l takes chunk (l % 16) ^ (row % 16) of row
-    // 4 i + l / 16 and writes it at position l % 16, so the MFMA operand reads below hit distinct banks
-    int va[G::NA / KQ_WAVES];
-#pragma unroll
-    for (int k = 0; k < G::NA / KQ_WAVES; k++) {
-        const int row = 4 * (wave + KQ_WAVES * k) + (lane >> 4);
-        va[k] = row * K + 16 * ((lane & 15) ^ (row & 15));
-    }
-    // weight piece q = 64 i + l of a stage: row q / PR, piece q % PR
-    auto wpiece = [&](int i) __attribute__((always_inline)) {
-        const int q = min(64 * i + lane, KQ_BN * G::PR - 1), row = q / G::PR;
-        return row * (int)row_bytes + 16 * (q - G::PR * row);
+    if (!MOE || s0 < s1) {
+    // The wave's weight rows: a buffer from the 16-byte piece its first row starts in to the piece the matrix ends in
+    // (reads stay inside that piece's 16 bytes; rows past the matrix read as zeros through the hardware range check).
+    // Waves wholly past the matrix get an empty one.
+    const int wr0 = nr0 + 32 * wave;
+    const int64_t wb0 = (int64_t)wr0 * row_bytes;
+    const int wsh = (int)(wb0 & 15);  // q6_K rows start at any even byte
+    const int64_t wlen = ((int64_t)n_rows * row_bytes + 15) / 16 * 16 - (wb0 - wsh);
+    const kf_arsrc_t rw = kf_arsrc(wt + (wr0 < n_rows ? wb0 - wsh : 0), wr0 < n_rows ? (uint64_t)wlen : 0);
+    const kf_arsrc_t rx = kf_arsrc((MOE ? kq_uniform(st.xq) : xq_) + (int64_t)m0 * K, (uint64_t)(m_end - m0) * K);
+    const kf_arsrc_t rs = kf_arsrc((MOE ? kq_uniform(st.xa) : xa_) + (int64_t)m0 * nsb * 16, (uint64_t)(m_end - m0) * nsb * 32);
+    const kf_arsrc_t rd = kf_arsrc((MOE ? kq_uniform(st.xd) : xd_) + (int64_t)m0 * kg, (uint64_t)(m_end - m0) * kg * 4);
+    // past the range's end the loads run with an empty buffer: no traffic, and the counts of the waits hold
+    auto off = [](kf_arsrc_t r, bool on) __attribute__((always_inline)) {
+        if (!on) r[2] = 0;
+        return r;
     };
-    auto dma = [&](uint8_t* buf, int sb) __attribute__((always_inline)) {
-#pragma unroll
-        for (int k = 0; k < G::NA / KQ_WAVES; k++) kf_adma16(rx, va[k], sb * 256, buf + G::A + (wave + KQ_WAVES * k) * 1024);
-        const int wo = G::Q6 ? (sb * G::SBB) & ~15 : sb * G::SBB;
-#pragma unroll
-        for (int k = 0; k < (G::NW + KQ_WAVES - 1) / KQ_WAVES; k++) {
-            const int i = wave + KQ_WAVES * k;
-            if (i < G::NW) kf_adma16(rw, wpiece(i), wo, buf + G::W + i * 1024);
-        }
-        if (wave == 0) kf_adma4(rd, lane * kg * 4, sb * 32, buf + G::DX);
-        if (!G::Q6 && (wave == 1 || wave == 2))
-            kf_adma16(rs, ((wave - 1) * 32 + (lane >> 1)) * nsb * 32 + (lane & 1) * 16, sb * 32, buf + G::XS + (wave - 1) * 1024);
-    };
-
-    v16f acc[KQ_TM];
-#pragma unroll
-    for (int i = 0; i < KQ_TM; i++) acc[i] = v16f{};
-    const int wcol = (wave * 32 + r32) * G::WROW;  // the wave's weight row (tile column) for this lane
-    const int sw = r32 & 15;
-
-    // group g's activation operand of tile i: chunk 2 g + half of the lane's row, stored at (2 g + half) ^ (row % 16)
-    auto aop = [&](const uint8_t* cur, int g, int i) __attribute__((always_inline)) {
-        return *reinterpret_cast<const v4i*>(cur + G::A + (i * 32 + r32) * 256 + 16 * ((2 * g + half) ^ sw));
-    };
-
-    // TLC: the 32-row tiles of the block that hold rows (a grouped tile with at most 32 rows skips its second)
-    auto stage = [&](auto tlc, const uint8_t* cur, int sb) __attribute__((always_inline)) {
-        constexpr int TL = decltype(tlc)::value;
-        v16i S[KQ_TM];
-#pragma unroll
-        for (int i = 0; i < TL; i++) S[i] = v16i{};
-        float d, dm = 0.0f;
-        v8h mo;
-        if constexpr (!G::Q6) {
-            // q5_K: d, dmin, 12 bytes of 6-bit scales / mins, qh[32], qs[128]; the lane's 16 columns of group g are
-            // bytes 16 half.. of qs[32 (g / 2)..] (low nibbles: g even) with bit g of qh[16 half..]
-            const uint8_t* wr = cur + G::W + wcol;
-            const uint4 hd = *reinterpret_cast<const uint4*>(wr);
-            const uint4 qh = G::Q4 ? make_uint4(0u, 0u, 0u, 0u) : *reinterpret_cast<const uint4*>(wr + 16 + 16 * half);
-            const uint32_t qhv[4] = {qh.x, qh.y, qh.z, qh.w};
-            const uint32_t m4 = 0x0f0f0f0fu, m1 = 0x01010101u;
-            uint4 raw[4];
-            uint32_t sc2[4], scv[2], mnv[2];
-            kf_q4k_scales8(hd.y, hd.z, hd.w, scv, mnv);
-#pragma unroll
-            for (int p = 0; p < 4; p++) {
-                raw[p] = *reinterpret_cast<const uint4*>(wr + G::QS + 32 * p + 16 * half);
-                sc2[p] = kf_pair(scv, p);
-                const uint32_t m2 = kf_pair(mnv, p);
-                mo[2 * p] = (_Float16)(float)((half ? 1u : 64u) * (m2 & 0xffu));
-                mo[2 * p + 1] = (_Float16)(float)((half ? 1u : 64u) * (m2 >> 8));
-            }
-            // group g's MFMAs (operand: 0..31 per byte, the fifth bit from qh)
-            auto issue = [&](auto gc, v16i (&I)[KQ_TM]) __attribute__((always_inline)) {
-                constexpr int g = decltype(gc)::value;
-                const uint32_t v[4] = {raw[g / 2].x, raw[g / 2].y, raw[g / 2].z, raw[g / 2].w};
-                v4i b;
-#pragma unroll
-                for (int e = 0; e < 4; e++) b[e] = (int)((((g & 1) ? v[e] >> 4 : v[e]) & m4) | (((qhv[e] >> g) & m1) << 4));
-#pragma unroll
-                for (int i = 0; i < TL; i++) I[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(aop(cur, g, i), b, v16i{}, 0, 0, 0);
-            };
-            // Software-pipelined by one group: group g + 1's MFMAs are issued before group g's multiply-adds, which
-            // depend on none of them, so the adds run while the matrix core works. The running sums are
-            // materialized after each group (left free, the compiler reassociates the integer adds across groups
-            // and holds every product), and the sched barriers keep the groups in this order.
-            v16i Ia[KQ_TM], Ib[KQ_TM];
-            auto mads = [&](int g, const v16i (&I)[KQ_TM]) __attribute__((always_inline)) {
-                const int sc = (int)((g & 1) ? sc2[g / 2] >> 8 : sc2[g / 2] & 0xffu);
-#pragma unroll
-                for (int i = 0; i < TL; i++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) S[i][r] += __mul24(sc, I[i][r]);  // |sc I| < 2^22
-#pragma unroll
-                for (int i = 0; i < TL; i++) __asm__ volatile("" : "+v"(S[i]));
-            };
-            issue(std::integral_constant<int, 0>{}, Ia);
-            __builtin_amdgcn_sched_barrier(0);
-            issue(std::integral_constant<int, 1>{}, Ib);
-            mads(0, Ia);
-            __builtin_amdgcn_sched_barrier(0);
-            issue(std::integral_constant<int, 2>{}, Ia);
-            mads(1, Ib);
-            __builtin_amdgcn_sched_barrier(0);
-            issue(std::integral_constant<int, 3>{}, Ib);
-            mads(2, Ia);
-            __builtin_amdgcn_sched_barrier(0);
-            issue(std::integral_constant<int, 4>{}, Ia);
-            mads(3, Ib);
-            __builtin_amdgcn_sched_barrier(0);
-            issue(std::integral_constant<int, 5>{}, Ib);
-            mads(4, Ia);
-            __builtin_amdgcn_sched_barrier(0);
-            issue(std::integral_constant<int, 6>{}, Ia);
-            mads(5, Ib);
-            __builtin_amdgcn_sched_barrier(0);
-            issue(std::integral_constant<int, 7>{}, Ib);
-            mads(6, Ia);
-            __builtin_amdgcn_sched_barrier(0);
-            mads(7, Ib);
-            __builtin_amdgcn_sched_barrier(0);
-            d = kf_h2f(hd.x & 0xffffu);
-            dm = kf_h2f(hd.x >> 16);
+    // record part k: the activation scales, the mins operands; each wave moves its eighth of the block's rows
+    auto dma_rec = [&](int sb, int k) __attribute__((always_inline)) {
+        uint8_t* rec = lds + G::R + (sb % G::NS) * G::REC;
+        constexpr int RW = BM / KQ_WAVES;
+        if (k == 0) {
+            kq_adma4<RW>(off(rd, sb < s1), (wave * RW + lane) * kg * 4, sb * 32, rec + wave * RW * 4);
         } else {
-            // q6_K: ql[128], qh[64], int8 scales[16], d; the super-block starts at the window's shift (sb * 210) % 16,
-            // 2-byte aligned. Group g = 4 h + gg (columns 128 h + 32 gg..): the lane's 16 columns l = 16 half.. take
-            // the low (gg < 2) or high nibbles of ql[64 h + 32 (gg % 2) + l] and bits 2 gg.. of qh[32 h + l]; scales
-            // 8 h + 2 gg (columns 0-15 of the group) and 8 h + 2 gg + 1 (16-31)
-            const uint8_t* wr = cur + G::W + wcol + ((sb * G::SBB) & 15);
-            const u32x4_a2 scv = *reinterpret_cast<const u32x4_a2*>(wr + 192);
-            const uint32_t scw[4] = {scv.x, scv.y, scv.z, scv.w};
-            const uint32_t m4 = 0x0f0f0f0fu, m3 = 0x03030303u, hb = 0x80808080u, k32 = 0x20202020u;
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const u32x4_a2 la = *reinterpret_cast<const u32x4_a2*>(wr + 64 * h + 16 * half);
-                const u32x4_a2 lb = *reinterpret_cast<const u32x4_a2*>(wr + 64 * h + 32 + 16 * half);
-                const u32x4_a2 qq = *reinterpret_cast<const u32x4_a2*>(wr + 128 + 32 * h + 16 * half);
-#pragma unroll
-                for (int gg = 0; gg < 4; gg++) {
-                    const u32x4_a2 src = (gg & 1) ? lb : la;
-                    v4i bw;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const uint32_t lo = (gg >> 1) ? (src[e] >> 4) & m4 : src[e] & m4;
-                        const uint32_t v = lo | (((qq[e] >> (2 * gg)) & m3) << 4);  // q in [0, 63] per byte
-                        bw[e] = (int)(((v | hb) - k32) ^ hb);                         // q - 32 per byte, no borrows
-                    }
-                    const v4i b0 = half ? v4i{} : bw, b1 = half ? bw : v4i{};  // columns 0-15, then 16-31
-                    const int si = 8 * h + 2 * gg;
-                    const int s0 = (int)(int8_t)(uint8_t)(scw[si >> 2] >> (8 * (si & 3)));
-                    const int s1 = (int)(int8_t)(uint8_t)(scw[(si + 1) >> 2] >> (8 * ((si + 1) & 3)));
-#pragma unroll
-                    for (int i = 0; i < TL; i++) {
-                        const v4i a = aop(cur, 4 * h + gg, i);
-                        const v16i I0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b0, v16i{}, 0, 0, 0);
-                        const v16i I1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b1, v16i{}, 0, 0, 0);
-                        // |dot| <= 16 * 128 * 32 and |sc| <= 128: the 24-bit products are exact
-#pragma unroll
-                        for (int r = 0; r < 16; r++) S[i][r] += __mul24(s0, I0[r]) + __mul24(s1, I1[r]);
-                    }
-#pragma unroll
-                    for (int i = 0; i < TL; i++) __asm__ volatile("" : "+v"(S[i]));
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-            d = kf_h2f(*reinterpret_cast<const uint16_t*>(wr + 208));
-        }
-        // acc += dx (d S - dmin mins); accumulator register r holds row (r % 4) + 8 (r / 4) + 4 (lane / 32)
-#pragma unroll
-        for (int i = 0; i < TL; i++) {
-            v16f mins = v16f{};
-            if constexpr (!G::Q6) {
-                const v8h xo = *reinterpret_cast<const v8h*>(cur + G::XS + (i * 32 + r32) * 32 + half * 16);
-                mins = __builtin_amdgcn_mfma_f32_32x32x16_f16(xo, mo, v16f{}, 0, 0, 0);
-            }
-            const float* dxp = reinterpret_cast<const float*>(cur + G::DX) + i * 32 + half * 4;
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const v4f dx = *reinterpret_cast<const v4f*>(dxp + 8 * q);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int r = 4 * q + e;
-                    const float t = G::Q6 ? d * (float)S[i][r] : fmaf(-dm, mins[r], d * (float)S[i][r]);
-                    acc[i][r] = fmaf(t, dx[e], acc[i][r]);
-                }
-            }
+            kq_adma16<2 * RW>(off(rs, sb < s1), (wave * RW + (lane >> 1)) * nsb * 32 + (lane & 1) * 16, sb * 32, rec + BM * 4 + wave * RW * 32);
         }
     };
+    // The wave's rows 4 w.. of activation tile i: lane l takes chunk (l % 16) ^ (row % 16) of row 4 w + l / 16 and writes
+    // it at position l % 16, so the MFMA operand reads below hit distinct banks. With four tiles the addresses are made
+    // anew each time (an opaque lane index): kept across the K loop they would spill.
+    auto dma_a = [&](int sb, int i) __attribute__((always_inline)) {
+        int ln = lane;
+        if constexpr (TM > 2) __asm__("" : "+v"(ln));
+        const int arow = 4 * wave + (ln >> 4);
+        kf_adma16(off(rx, sb < s1), (arow + 32 * i) * K + 16 * ((ln & 15) ^ (arow & 15)), sb * 256,
+                  lds + G::A + (sb % G::NA) * G::ABUF + wave * 1024 + i * 8192);
+    };
+    // 64 of the pieces of the wave's 32 weight rows
+    auto dma_w = [&](int sb, int k) __attribute__((always_inline)) {
+        int ln = lane;
+        if constexpr (TM > 2) __asm__("" : "+v"(ln));
+        const int q = 64 * k + ln, row = q / G::PR, piece = q - G::PR * row;
+        const int start = row * (int)row_bytes + (G::Q6 ? wsh + sb * G::SBB : 0);
+        const int vo = (G::Q6 ? start & ~15 : start) + 16 * piece;
+        uint8_t* buf = lds + G::W + (sb % G::NW * KQ_WAVES + wave) * G::WBUF;
+        if (64 * k + 64 <= G::PW)
+            kf_adma16(off(rw, sb < s1), vo, G::Q6 ? 0 : sb * G::SBB, buf + k * 1024);
+        else
+            kq_adma16<(G::PW & 63) ? (G::PW & 63) : 1>(off(rw, sb < s1), vo, G::Q6 ? 0 : sb * G::SBB, buf + k * 1024);
+    };
 
-    // stage sb multiplies one buffer while sb + 1 lands in the other; every DMA wait is explicit
+    v16f acc[TM];
+#pragma unroll
+    for (int i = 0; i < TM; i++) acc[i] = v16f{};
+
+    // The K loop over TLC 32-row tiles (a grouped tile with fewer rows skips the empty ones). Per super-block the tiles
+    // run one after another, each as eight group steps: the step's two MFMAs, one eighth of the previous tile's rescale
+    // and, in the last tile, the expansion of the same group of the next super-block into the operand registers the
+    // step has just used. So every step mixes matrix-core and vector work and no phase of a wave is without MFMAs.
     auto kloop = [&](auto tlc) __attribute__((always_inline)) {
-        dma(buf0, s0);
-        __builtin_amdgcn_s_waitcnt(KF_WAITCNT_VM(0));
-        __syncthreads();
-#pragma unroll 1
-        for (int sb = s0; sb < s1; sb += 2) {
-            if (sb + 1 < s1) dma(buf1, sb + 1);
-            stage(tlc, buf0, sb);
-            __builtin_amdgcn_s_waitcnt(KF_WAITCNT_VM(0));
-            __syncthreads();
-            if (sb + 1 < s1) {
-                if (sb + 2 < s1) dma(buf0, sb + 2);
-                stage(tlc, buf1, sb + 1);
-                __builtin_amdgcn_s_waitcnt(KF_WAITCNT_VM(0));
-                __syncthreads();
-            }
-        }
-    };
-    // a grouped slot's last tile often holds a few rows: with at most 32 the second 32-row tile's MFMAs, adds and
-    // rescale are skipped (its accumulators stay zero and its rows are not stored)
-    if (MOE && m_end - m0 <= 32)
-        kloop(std::integral_constant<int, 1>{});
-    else
-        kloop(std::integral_constant<int, KQ_TM>{});
-
-    if (!MOE && sp >= 0) {
-        // a split: its partial tile through system-scope stores (they write through to memory, so the other splits'
-        // blocks see them from any XCD without an L2 write-back), a ticket, and the last to arrive adds all S
-        constexpr int R = KQ_TM * 16;
-        float* pp = tail.part + (size_t)(tail.S * tt + sp) * R * KQ_THREADS + tid;
-#pragma unroll
-        for (int i = 0; i < KQ_TM; i++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) __hip_atomic_store(pp + (i * 16 + r) * KQ_THREADS, acc[i][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __builtin_amdgcn_s_waitcnt(KF_WAITCNT_VM(0));
-        __syncthreads();
-        if (tid == 0) last = __hip_atomic_fetch_add(&tail.tickets[tt], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == tail.S - 1;
-        __syncthreads();
-        if (!last) return;
-        const float* p0 = tail.part + (size_t)tail.S * tt * R * KQ_THREADS + tid;
-#pragma unroll
-        for (int i = 0; i < KQ_TM; i++) acc[i] = v16f{};
-        for (int k = 0; k < tail.S; k++) {
-            float part[R];
-#pragma unroll
-            for (int e = 0; e < R; e++) part[e] = __hip_atomic_load(p0 + ((size_t)k * R + e) * KQ_THREADS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-#pragma unroll
-            for (int i = 0; i < KQ_TM; i++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[i][r] += part[i * 16 + r];
-        }
-        if (tid == 0) __hip_atomic_store(&tail.tickets[tt], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-
-    const int n = n0 + wave * 32 + r32;
-    if (MOE && msplit) {
-        // The two K halves of a grouped tile. The first half leaves its partial in y (the tile's output rows) and the
-        // second in the scratch, each with system-scope stores, which write through to memory, then each takes the
-        // tile's ticket; the second to arrive reads the other's partial from its place and stores the sum. A sum of
-        // two is the same in either order, so the result does not depend on which half arrives last.
-        constexpr int R = KQ_TM * 16;
-        float* pp = tail_arg.part + (size_t)tt * R * KQ_THREADS + tid;
-        auto yo = [&](int i, int r) __attribute__((always_inline)) {
-            const int m = m0 + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * half;
-            return m >= m_end ? (int64_t)-1 : (int64_t)(moe.out_rows ? moe.out_rows[m] : m) * N + n;
+        constexpr int TL = decltype(tlc)::value;
+        // An even number of tiles carries the last tile's rescale over into the next super-block's first tile; an odd
+        // one, whose parities would alternate, rescales it at the super-block's end.
+        constexpr bool LAG = TL % 2 == 0;
+        constexpr bool SLOTS = TL > 1;
+        constexpr int SPER = (G::NSI + TL + G::NWI + 8 * (TL - 1) - 1) / (8 * (TL > 1 ? TL - 1 : 1));  // loads a step, done before the last tile
+        KqPlanes B[8];
+        KqWeight<TY, TM> kw;
+        float d = 0.0f, dm = 0.0f, dp = 0.0f, dmp = 0.0f;  // this super-block's column scales, and the previous one's
+        v8h mo = v8h{};
+        auto wrow = [&](int sb) __attribute__((always_inline)) {
+            const uint8_t* p = lds + G::W + (sb % G::NW * KQ_WAVES + wave) * G::WBUF + r32 * G::WROW;
+            return G::Q6 ? p + ((r32 * (int)row_bytes + wsh + sb * G::SBB) & 15) : p;
         };
-        if (sp == 1) {
+        auto take = [&]() __attribute__((always_inline)) {
+            d = kf_h2f(kw.d16 & 0xffffu);
+            if constexpr (!G::Q6) {
+                dm = kf_h2f(kw.d16 >> 16);
+                __asm__("" : "+v"(dm));  // kept in f32: mixed-precision multiply-adds need wait states here
+            }
+        };
+        // group g's activation operand of tile i: chunk 2 g + half of the lane's row, stored at (2 g + half) ^ (row % 16),
+        // i.e. 32 g exclusive-or'ed into the address of group 0's
+        const uint32_t a0 = kf_lds_addr(lds + G::A) + r32 * 256 + 16 * (half ^ (r32 & 15));
+        auto aop = [&](uint32_t at, int g, int i) __attribute__((always_inline)) {
+            const uint32_t p = ((at + a0) ^ (32u * g)) + i * 8192;
+            return *reinterpret_cast<const __attribute__((address_space(3))) v4i*>(p);
+        };
+        v16i S[2][2];  // [tile parity][lo, hi]; lo becomes S once a tile is done
+        v16f mins = v16f{};
+        // The rescale of tile i in eight parts: S = lo + (hi << SHIFT) in the first two, the mins product, then rows
+        // rat[g].. of acc += dx (d S - dmin mins); accumulator register r holds row (r % 4) + 8 (r / 4) + 4 (lane / 32). The
+        // LDS operands of part g are read by load(g) one step earlier.
+        constexpr int rat[9] = {0, 0, 0, 4, 6, 8, 12, 14, 16};
+        float dxn[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        auto load = [&](auto gc, const uint8_t* rec, int i) __attribute__((always_inline)) {
+            constexpr int g = decltype(gc)::value;
+            if constexpr (g >= 2 && g < 8) {
 #pragma unroll
-            for (int i = 0; i < KQ_TM; i++)
+                for (int r = rat[g]; r < rat[g + 1]; r++) dxn[r - rat[g]] = reinterpret_cast<const float*>(rec)[i * 32 + half * 4 + 8 * (r >> 2) + (r & 3)];
+            }
+        };
+        auto rescale = [&](auto pc, auto gc, v16f& a, const float (&dx)[4], const uint8_t* rec, int i, float ds, float dms) __attribute__((always_inline)) {
+            constexpr int p = decltype(pc)::value, g = decltype(gc)::value;
+            if constexpr (g < 2) {
 #pragma unroll
-                for (int r = 0; r < 16; r++) __hip_atomic_store(pp + (i * 16 + r) * KQ_THREADS, acc[i][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        } else if (n < N) {
-#pragma unroll
-            for (int i = 0; i < KQ_TM; i++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int64_t o = yo(i, r);
-                    if (o >= 0) __hip_atomic_store(y + o, acc[i][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                for (int r = 8 * g; r < 8 * g + 8; r++) S[p][0][r] += (int)((uint32_t)S[p][1][r] << G::SHIFT);
+                if constexpr (g == 1 && !G::Q6) {
+                    const v8h xo = *reinterpret_cast<const v8h*>(rec + BM * 4 + (i * 32 + r32) * 32 + half * 16);
+                    mins = __builtin_amdgcn_mfma_f32_32x32x16_f16(xo, mo, v16f{}, 0, 0, 0);
                 }
-        }
-        __builtin_amdgcn_s_waitcnt(KF_WAITCNT_VM(0));
-        __syncthreads();
-        if (tid == 0) last = __hip_atomic_fetch_add(&tail_arg.tickets[tt], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == 1;
-        __syncthreads();
-        if (!last) return;
-        if (sp == 0) {
-            float other[R];
+            } else {
 #pragma unroll
-            for (int e = 0; e < R; e++) other[e] = __hip_atomic_load(pp + e * KQ_THREADS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-#pragma unroll
-            for (int i = 0; i < KQ_TM; i++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[i][r] = acc[i][r] + other[i * 16 + r];
-        } else if (n < N) {
-            float other[R];
-#pragma unroll
-            for (int i = 0; i < KQ_TM; i++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int64_t o = yo(i, r);
-                    other[i * 16 + r] = o >= 0 ? __hip_atomic_load(y + o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) : 0.0f;
+                for (int r = rat[g]; r < rat[g + 1]; r++) {
+                    const float sf = (float)S[p][0][r];
+                    const float t = G::Q6 ? ds * sf : fmaf(-dms, mins[r], ds * sf);
+                    a[r] = fmaf(t, dx[r - rat[g]], a[r]);
                 }
+            }
+        };
+        // one tile's eight steps; `prev`: the tile rescaled meanwhile (its index and parity), sbn: the super-block
+        // expanded meanwhile (EXP)
+        auto tile = [&](auto ic, auto pc, auto expc, auto firstc, uint32_t at, const uint8_t* prec, const uint8_t* wn, auto issue)
+            __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value, p = decltype(pc)::value;
+            constexpr bool EXP = decltype(expc)::value, FIRST = decltype(firstc)::value;
+            constexpr int pi = i == 0 ? TL - 1 : i - 1;  // the tile before this one
+            if constexpr (i == 0 && !LAG && !G::Q6) mo = kw.mins(half);
+            if constexpr (EXP) kw.begin(wn, half);
+            v4i a = aop(at, 0, i);
+            auto step = [&](auto gc) __attribute__((always_inline)) {
+                constexpr int g = decltype(gc)::value;
+                // the next step's LDS reads go first, this step's matrix and vector work hides their latency
+                v4i an = a;
+                if constexpr (g < 7) an = aop(at, g + 1, i);
+                const float dx[4] = {dxn[0], dxn[1], dxn[2], dxn[3]};
+                if constexpr (!FIRST && g < 7) load(std::integral_constant<int, g + 1>{}, prec, pi);
+                if constexpr (SLOTS) {
 #pragma unroll
-            for (int i = 0; i < KQ_TM; i++)
+                    for (int k = SPER * (8 * i + g); k < SPER * (8 * i + g + 1); k++) issue(k);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                const KqPlanes b = B[g];
+                S[p][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b.lo, g == 0 ? v16i{} : S[p][0], 0, 0, 0);
+                S[p][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b.hi, g == 0 ? v16i{} : S[p][1], 0, 0, 0);
+                if constexpr (!FIRST) rescale(std::integral_constant<int, 1 - p>{}, gc, acc[pi], dx, prec, pi, i == 0 ? dp : d, i == 0 ? dmp : dm);
+                if constexpr (EXP) {
+                    B[g] = kw.template planes<g>();
+                    if constexpr (g < 7) kw.template fetch<g + 1>(wn, half);
+                }
+                // the previous super-block's mins operand has had its last use
+                if constexpr (i == 0 && g == 2 && LAG && !G::Q6) mo = kw.mins(half);
+                a = an;
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            step(std::integral_constant<int, 0>{});
+            step(std::integral_constant<int, 1>{});
+            step(std::integral_constant<int, 2>{});
+            step(std::integral_constant<int, 3>{});
+            step(std::integral_constant<int, 4>{});
+            step(std::integral_constant<int, 5>{});
+            step(std::integral_constant<int, 6>{});
+            step(std::integral_constant<int, 7>{});
+        };
+        // the rescale of a super-block's last tile by itself
+        auto finish = [&](int sb) __attribute__((always_inline)) {
+            const uint8_t* rec = lds + G::R + (sb % G::NS) * G::REC;
+            auto all = [&](auto gc) __attribute__((always_inline)) {
+                load(gc, rec, TL - 1);
+                rescale(std::integral_constant<int, (TL - 1) & 1>{}, gc, acc[TL - 1], dxn, rec, TL - 1, dp, dmp);
+            };
+            all(std::integral_constant<int, 0>{});
+            all(std::integral_constant<int, 1>{});
+            all(std::integral_constant<int, 2>{});
+            all(std::integral_constant<int, 3>{});
+            all(std::integral_constant<int, 4>{});
+            all(std::integral_constant<int, 5>{});
+            all(std::integral_constant<int, 6>{});
+            all(std::integral_constant<int, 7>{});
+        };
+        // One super-block (FIRST: no tile before it to rescale)
+        auto sblock = [&](auto firstc, int sbv) __attribute__((always_inline)) {
+            constexpr bool FIRST = decltype(firstc)::value || !LAG;
+            const int sb = __builtin_amdgcn_readfirstlane(sbv);
+            // The loads ahead: all at once with one tile, which waits for them right away; with more, SPER of them a step
+            // from the first, so that the eight waves' requests do not queue in front of each other.
+            auto issue = [&](int k) __attribute__((always_inline)) {
+                if (k < G::NSI)
+                    dma_rec(sb + G::NA - 1, k);
+                else if (k < G::NSI + TL)
+                    dma_a(sb + G::NA - 1, k - G::NSI);
+                else if (k < G::NSI + TL + G::NWI)
+                    dma_w(sb + G::NW, k - G::NSI - TL);
+            };
+            if constexpr (!SLOTS) {
 #pragma unroll
-                for (int r = 0; r < 16; r++) acc[i][r] = other[i * 16 + r] + acc[i][r];
+                for (int k = 0; k < G::NSI + TL + G::NWI; k++) issue(k);
+            }
+            const uint32_t at = (sb % G::NA) * G::ABUF;
+            const uint8_t* rec = lds + G::R + (sb % G::NS) * G::REC;
+            const uint8_t* prec = FIRST ? rec : lds + G::R + ((sb - 1) % G::NS) * G::REC;
+            const uint8_t* wn = wrow(sb + 1);
+            auto one = [&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value;
+                if constexpr (i < TL) {
+                    if constexpr (i == TL - 1) __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(G::wait(TL)) : "memory");
+                    tile(ic, std::integral_constant<int, i & 1>{}, std::integral_constant<bool, i == TL - 1>{},
+                         std::integral_constant<bool, FIRST && i == 0>{}, at, i == 0 ? prec : rec, wn, issue);
+                }
+            };
+            one(std::integral_constant<int, 0>{});
+            one(std::integral_constant<int, 1>{});
+            one(std::integral_constant<int, 2>{});
+            one(std::integral_constant<int, 3>{});
+            dp = d;
+            dmp = dm;
+            take();
+            if constexpr (!LAG) finish(sb);
+            __syncthreads();
+        };
+#pragma unroll
+        for (int b = 0; b < G::NA - 1; b++) {
+#pragma unroll
+            for (int k = 0; k < G::NSI; k++) dma_rec(s0 + b, k);
+#pragma unroll
+            for (int i = 0; i < TL; i++) dma_a(s0 + b, i);
         }
-        if (tid == 0) __hip_atomic_store(&tail_arg.tickets[tt], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+#pragma unroll
+        for (int b = 0; b < G::NW; b++)
+#pragma unroll
+            for (int k = 0; k < G::NWI; k++) dma_w(s0 + b, k);
+        __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        {
+            const uint8_t* wr = wrow(s0);
+            kw.begin(wr, half);
+            auto ex = [&](auto gc) __attribute__((always_inline)) {
+                constexpr int g = decltype(gc)::value;
+                B[g] = kw.template planes<g>();
+                if constexpr (g < 7) kw.template fetch<g + 1>(wr, half);
+            };
+            ex(std::integral_constant<int, 0>{});
+            ex(std::integral_constant<int, 1>{});
+            ex(std::integral_constant<int, 2>{});
+            ex(std::integral_constant<int, 3>{});
+            ex(std::integral_constant<int, 4>{});
+            ex(std::integral_constant<int, 5>{});
+            ex(std::integral_constant<int, 6>{});
+            ex(std::integral_constant<int, 7>{});
+            take();
+            __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+        using std::false_type;
+        using std::true_type;
+        sblock(true_type{}, s0);
+#pragma unroll 1
+        for (int sb = s0 + 1; sb < s1; sb++) sblock(false_type{}, sb);
+        if constexpr (LAG) finish(s1 - 1);
+    };
+    if constexpr (MOE) {
+        const int tl = (min(m_end - m0, BM) + 31) / 32;
+        if (TM >= 4 && tl == 4)
+            kloop(std::integral_constant<int, TM < 4 ? TM : 4>{});
+        else if (TM >= 4 && tl == 3)
+            kloop(std::integral_constant<int, TM < 3 ? TM : 3>{});
+        else if (TM >= 2 && tl == 2)
+            kloop(std::integral_constant<int, TM < 2 ? TM : 2>{});
+        else
+            kloop(std::integral_constant<int, 1>{});
+    } else {
+        kloop(std::integral_constant<int, TM>{});
     }
-    if (n < N) {
-        const float bn = bias ? bias[n] : 0.0f;
+
+    // the tile, or the part of it that is this block's
+    float* y = y_;
+    float* part = work.part;
+    const float *bias = bias_, *res = res_;
+    const int32_t* out_rows = nullptr;
+    int Nn = N_, me = m_end, mb = m0, n = n0;
+    if constexpr (MOE) {
+        const bool starts = kq_uniform(st.s0) == 0, ends = kq_uniform(st.s1) == kq_uniform(st.K) >> 8;
+        if (!starts || !ends) {
+            const int b = kq_uniform(st.b);
+            slot = 2 * b + (starts ? 1 : 0);
+            if (starts && tid == 0) kq_uniform(st.desc)[b] = KqDesc{st.m0, st.m_end, st.n0, st.count};
+        }
+        y = kq_uniform(st.y);
+        part = kq_uniform(st.part);
+        out_rows = kq_uniform(st.out_rows);
+        bias = res = nullptr;
+        Nn = kq_uniform(st.N);
+        me = kq_uniform(st.m_end);
+        mb = kq_uniform(st.m0);
+        n = kq_uniform(st.n0);
+    }
+    if (slot >= 0) {
+        float* pp = part + (size_t)slot * (TM * 16) * KQ_THREADS + tid;
 #pragma unroll
-        for (int i = 0; i < KQ_TM; i++)
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) pp[(i * 16 + r) * KQ_THREADS] = acc[i][r];
+    } else {
+        n += wave * 32 + r32;
+        const float bn = bias && n < Nn ? bias[n] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                const int m = m0 + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * half;
-                if (m >= m_end) continue;
-                const int64_t o = (int64_t)(MOE && moe.out_rows ? moe.out_rows[m] : m) * N + n;
+                const int m = mb + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * half;
+                if (m >= me || n >= Nn) continue;
+                const int64_t o = (int64_t)(out_rows ? out_rows[m] : m) * Nn + n;
                 y[o] = acc[i][r] + bn + (res ? res[o] : 0.0f);
             }
+    }
+    }
+    if constexpr (!MOE) return;
+    __syncthreads();  // the state is written (an empty part runs no K loop, whose barriers would order it)
+    if (kq_uniform(st.next) >= kq_uniform(st.u_end)) return;
+    __syncthreads();  // every wave has read the state
+    if (threadIdx.x == 0) st.u = st.next;
+    }
+}
+
+// Adds the partial tiles of the tiles that several blocks shared, in K order, with bias and residual. One thread an output;
+// a block takes RED of the TM * 16 (register, 512 threads) slices of a tile, so every load and store is a run of whole
+// lines: one slice with one matrix, whose few tiles have many parts (four made 32 rows of 4096 x 4096 14.2 us, 12.7 with
+// one), four in the grouped form, where most blocks have nothing to add. A launch of its own: the last block to arrive adding them by itself took 10-40 us with 16 partial tiles, as
+// one CU reads them all.
+template <int TM, bool MOE, int RED>
+__global__ void __launch_bounds__(KQ_THREADS) kq_reduce_kernel(KqWork work, const float* __restrict__ bias, const float* __restrict__ res,
+                                                                const int32_t* __restrict__ out_rows, float* __restrict__ y, int M, int N) {
+    constexpr int R = TM * 16;
+    const int b = blockIdx.x / (R / RED), e0 = (blockIdx.x - b * (R / RED)) * RED, tid = threadIdx.x;
+    KqDesc d;
+    size_t first, step;  // the first partial tile's slot, and from the second on the distance
+    if constexpr (MOE) {
+        d = work.desc[b];
+        if (d.count == 0) return;
+        first = 2 * b + 1;  // then range block b + 1's slot 2 (b + 1), b + 2's ...
+        step = 2;
+    } else {
+        const int mt = (M + 32 * TM - 1) / (32 * TM), t = work.full + b, tn = t / mt;
+        d = KqDesc{(t - tn * mt) * 32 * TM, M, tn * KQ_BN, work.S};
+        first = (size_t)b * work.S;
+        step = 1;
+    }
+    const int n = d.n0 + (tid >> 6) * 32 + (tid & 31);
+    // registers 4 q.. hold rows 8 q..
+    const int mb = d.m0 + (e0 >> 4) * 32 + 8 * ((e0 & 15) >> 2) + (e0 & 3) + 4 * ((tid >> 5) & 1);
+    if (mb >= d.m_end || n >= N) return;
+    const float* p = work.part + (first * R + e0) * KQ_THREADS + tid;
+    float v[RED];
+#pragma unroll
+    for (int e = 0; e < RED; e++) v[e] = p[e * KQ_THREADS];
+    p += (size_t)R * KQ_THREADS;
+    for (int k = 1; k < d.count; k += 4, p += 4 * step * R * KQ_THREADS) {
+        float a[4][RED];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int e = 0; e < RED; e++) a[u][e] = k + u < d.count ? p[(u * step * R + e) * KQ_THREADS] : 0.0f;
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int e = 0; e < RED; e++) v[e] += a[u][e];
+    }
+    const float bn = bias ? bias[n] : 0.0f;
+#pragma unroll
+    for (int e = 0; e < RED; e++) {
+        if (mb + e >= d.m_end) break;
+        const int64_t o = (int64_t)(out_rows ? out_rows[mb + e] : mb + e) * N + n;
+        y[o] = v[e] + bn + (res ? res[o] : 0.0f);
     }
 }
 
 }  // namespace
 
-// Whether the q5_K / q6_K GEMM takes these weights: K a multiple of 256 with 16-byte aligned rows (q5_K: always, 176-byte
-// super-blocks), q6_K rows that start 16-byte aligned (210-byte super-blocks: K a multiple of 2048), matrices below
-// 2 GB (row offsets travel as 32-bit values)
+// Whether the GEMM takes these weights: K a multiple of 256, rows of whole super-blocks from a 16-byte aligned base
 bool kf_gemm_kq_ok(uint32_t ty, const void* w, int64_t row_bytes, int K, int N) {
-    if (K % 256 != 0 || (int64_t)N * row_bytes >= (1ll << 31) || (reinterpret_cast<uintptr_t>(w) & 15) != 0) return false;
-    if (ty == KF_TYPE_Q4_K || ty == KF_TYPE_Q5_K) return row_bytes % 16 == 0;
-    if (ty == KF_TYPE_Q6_K) return row_bytes % 16 == 0;
-    return false;
+    (void)N;
+    return (ty == KF_TYPE_Q4_K || ty == KF_TYPE_Q5_K || ty == KF_TYPE_Q6_K) && K % 256 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 &&
+           row_bytes == (int64_t)(K / 256) * (ty == KF_TYPE_Q4_K ? KF_Q4_K_BYTES : ty == KF_TYPE_Q5_K ? KF_Q5_K_BYTES : KF_Q6_K_BYTES);
 }
 
-// The tail split of an M x N x K launch: the number of K ranges the last round's tiles run as (1: none) and the rounds'
-// length in super-blocks (full rounds of nsb, plus nsb / S for a split tail), as the launcher plans them
-static int kq_splits(int T, int nsb, int cus) {
-    const int rem = T % cus;
-    int S = 1;
-    while (S < 4 && rem * S * 2 <= cus && nsb / (S * 2) >= 2) S *= 2;
-    return S;
+namespace {
+
+// Descriptors and partial tiles in the split scratch
+constexpr size_t KQ_DESC_BYTES = 16384;
+static_assert(KF_SPLIT_SCRATCH >= KF_SPLIT_TICKETS * 4 + KQ_DESC_BYTES, "room for the descriptors");
+
+// Most blocks with a partial tile of their own (grouped: with two): one a CU, within the scratch
+int kq_max_ranges(int tm, int cus) {
+    const size_t room = (KF_SPLIT_SCRATCH - (size_t)KF_SPLIT_TICKETS * 4 - KQ_DESC_BYTES) / ((size_t)2 * tm * 16 * KQ_THREADS * 4);
+    int G = kf_knob_or(KF_KNOB_KQ_G, cus);
+    if ((size_t)G > room) G = (int)room;
+    if (G > (int)(KQ_DESC_BYTES / sizeof(KqDesc))) G = (int)(KQ_DESC_BYTES / sizeof(KqDesc));
+    return G;
 }
 
-double kf_gemm_kq_sb_rounds(int M, int N, int K) {
-    const int T = ((N + KQ_BN - 1) / KQ_BN) * ((M + KQ_BM - 1) / KQ_BM), nsb = K / 256, cus = kf_cu_count();
-    const int rem = T % cus, S = kq_splits(T, nsb, cus);
-    return (double)(T / cus) * nsb + (rem == 0 ? 0.0 : (double)nsb / S);
+struct KqPlan {
+    int tm, T, full, S;
+    double us;
+};
+
+KqPlan kq_plan_tm(uint32_t ty, int tm, int M, int N, int K) {
+    KqPlan p;
+    p.tm = tm;
+    const int cus = kf_cu_count(), nsb = K / 256;
+    p.T = ((N + KQ_BN - 1) / KQ_BN) * ((M + 32 * tm - 1) / (32 * tm));
+    const int rem = p.T % cus, t = tm >> 1, max_g = kq_max_ranges(tm, cus);
+    const double sb = KQ_SB_US[ty == KF_TYPE_Q4_K ? 0 : ty == KF_TYPE_Q5_K ? 1 : 2][t];
+    p.full = p.T;
+    p.S = 1;
+    // the tiles of the last round as S blocks each, S the cheapest that fits the CUs with two super-blocks a block or more
+    double tail = rem ? KQ_ROUND_US[t] + sb * nsb : 0.0;
+    for (int S = 2; rem && rem * S <= max_g && 2 * S <= nsb; S++) {
+        const double us = KQ_ROUND_US[t] + sb * ((nsb + S - 1) / S) + KQ_PART_US[t] * tm * rem * S / cus;
+        if (us < tail) {
+            tail = us;
+            p.full = p.T - rem;
+            p.S = S;
+        }
+    }
+    p.us = 1.8 + (p.T / cus) * (KQ_ROUND_US[t] + sb * nsb) + tail;
+    return p;
 }
+
+KqPlan kq_plan(uint32_t ty, int M, int N, int K) {
+    const int forced = ty == KF_TYPE_Q4_K && kf_knob_on(KF_KNOB_Q4K_KQ) ? (kf_knob(KF_KNOB_Q4K_KQ) ? 2 : 4) : kf_knob_or(KF_KNOB_KQ_TM, 0);
+    if (forced) return kq_plan_tm(ty, forced == 1 || forced == 2 ? forced : 4, M, N, K);
+    KqPlan best = kq_plan_tm(ty, 1, M, N, K);
+    for (int tm = 2; tm <= 4; tm *= 2) {
+        const KqPlan p = kq_plan_tm(ty, tm, M, N, K);
+        if (p.us < best.us) best = p;
+    }
+    return best;
+}
+
+// The scratch's range area, null when the stream has none
+KqWork kq_work(hipStream_t s, int full, int S) {
+    KqWork w{nullptr, nullptr, full, S};
+    if (char* scr = static_cast<char*>(kf_split_scratch(s))) {
+        w.desc = reinterpret_cast<KqDesc*>(scr + (size_t)KF_SPLIT_TICKETS * 4);
+        w.part = reinterpret_cast<float*>(scr + (size_t)KF_SPLIT_TICKETS * 4 + KQ_DESC_BYTES);
+    }
+    return w;
+}
+
+template <uint32_t TY, int TM, bool MOE>
+hipError_t kq_run(int blocks, hipStream_t s, const uint8_t* w, int64_t row_bytes, const int8_t* xq, const _Float16* xa, const float* xd,
+                  const float* bias, const float* res, float* y, int M, int N, int K, KqWork work, KqMoe moe) {
+    const auto fn = gemm_kq_kernel<TY, TM, MOE>;
+    constexpr int bytes = KqGeo<TY, TM>::LDS + KQ_EPI;
+    const hipError_t e = kf_raise_lds(reinterpret_cast<const void*>(fn), bytes);
+    if (e != hipSuccess) return e;
+    fn<<<blocks, KQ_THREADS, bytes, s>>>(w, row_bytes, xq, xa, xd, bias, res, y, M, N, K, work, moe);
+    const int shared = MOE ? work.S : (blocks - work.full) / work.S;  // tiles that may have partial ones
+    constexpr int RED = MOE ? 4 : 1;
+    if (work.part) kq_reduce_kernel<TM, MOE, RED><<<shared * (TM * 16 / RED), KQ_THREADS, 0, s>>>(work, bias, res, moe.out_rows, y, M, N);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+double kf_gemm_kq_us(uint32_t ty, int M, int N, int K) { return kq_plan(ty, M, N, K).us; }
 
 // Host launcher, validated by the caller (kf_gemm_kq_ok; Q8K-kind activations in `act`)
 hipError_t kf_launch_gemm_kq(uint32_t ty, const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y,
                              int M, int N, int K, hipStream_t s) {
     const kf_act_offsets o = kf_act_layout((size_t)M, (size_t)K);
     const char* base = static_cast<const char*>(act);
-    const int T = ((N + KQ_BN - 1) / KQ_BN) * ((M + KQ_BM - 1) / KQ_BM);
-    // the tail split (one block a CU): the tiles of a last round at most half full run as S = 2 or 4 blocks over K
-    // ranges of at least two super-blocks, S as large as the round holds (KF_GEMM_NO_TAIL turns it off, a comparison
-    // knob); it needs the split scratch
-    KqTail tail{nullptr, nullptr, T, 1};
-    int blocks = T;
-    const int cus = kf_cu_count(), rem = T % cus;
-    const int S = kq_splits(T, K / 256, cus);
-    const size_t part_bytes = (size_t)rem * S * KQ_TM * 16 * KQ_THREADS * 4;
-    if (S > 1 && rem <= KF_SPLIT_TICKETS && part_bytes <= KF_SPLIT_SCRATCH - (size_t)KF_SPLIT_TICKETS * 4 && !kf_knob_on(KF_KNOB_GEMM_NO_TAIL)) {
-        if (char* scr = static_cast<char*>(kf_split_scratch(s))) {
-            tail = KqTail{reinterpret_cast<float*>(scr + (size_t)KF_SPLIT_TICKETS * 4), reinterpret_cast<int*>(scr), T - rem, S};
-            blocks = T - rem + rem * S;
-        }
+    // whole rounds of the CUs, then the split tiles (KF_GEMM_NO_TAIL: a block a tile, a comparison knob); these need the scratch
+    const KqPlan p = kq_plan(ty, M, N, K);
+    KqWork work{nullptr, nullptr, p.T, 1};
+    if (p.S > 1 && !kf_knob_on(KF_KNOB_GEMM_NO_TAIL)) {
+        const KqWork r = kq_work(s, p.full, p.S);
+        if (r.part) work = r;
     }
+    const int blocks = work.full + (p.T - work.full) * work.S;
     const auto* wb = static_cast<const uint8_t*>(w);
     const auto* xq = reinterpret_cast<const int8_t*>(base + o.q);
     const auto* xa = reinterpret_cast<const _Float16*>(base + o.xa);
     const auto* xd = reinterpret_cast<const float*>(base + o.d32);
-    if (ty == KF_TYPE_Q4_K)
-        gemm_kq_kernel<KF_TYPE_Q4_K, false><<<blocks, KQ_THREADS, 0, s>>>(wb, row_bytes, xq, xa, xd, bias, res, y, M, N, K, tail, KqMoe{});
-    else if (ty == KF_TYPE_Q5_K)
-        gemm_kq_kernel<KF_TYPE_Q5_K, false><<<blocks, KQ_THREADS, 0, s>>>(wb, row_bytes, xq, xa, xd, bias, res, y, M, N, K, tail, KqMoe{});
-    else
-        gemm_kq_kernel<KF_TYPE_Q6_K, false><<<blocks, KQ_THREADS, 0, s>>>(wb, row_bytes, xq, xa, xd, bias, res, y, M, N, K, tail, KqMoe{});
-    return hipGetLastError();
+#define KQ_GO(TY, TM) return kq_run<TY, TM, false>(blocks, s, wb, row_bytes, xq, xa, xd, bias, res, y, M, N, K, work, KqMoe{})
+#define KQ_TMS(TY)               \
+    {                            \
+        if (p.tm == 1) KQ_GO(TY, 1); \
+        if (p.tm == 2) KQ_GO(TY, 2); \
+        KQ_GO(TY, 4);            \
+    }
+    if (ty == KF_TYPE_Q4_K) KQ_TMS(KF_TYPE_Q4_K)
+    if (ty == KF_TYPE_Q5_K) KQ_TMS(KF_TYPE_Q5_K)
+    KQ_TMS(KF_TYPE_Q6_K)
+#undef KQ_TMS
+#undef KQ_GO
 }
 
 // Grouped (MoE) form on q4_K experts: `act` holds `pairs` activation rows in group order (slot s: rows
@@ -546,24 +971,20 @@ hipError_t kf_launch_gemm_kq_moe(const void* w, const void* w2, int64_t expert_b
                                  int n_slots, const int32_t* offsets, const int32_t* out_rows, float* y, int N, int K, hipStream_t s) {
     const kf_act_offsets o = kf_act_layout((size_t)pairs, (size_t)K);
     const char* base = static_cast<const char*>(act);
-    // row tiles over all slots: each slot adds at most one partial tile
-    const int mt = (pairs + KQ_BM - 1) / KQ_BM + n_slots;
+    // The tile height by the pairs a slot gets on average (KF_MOE_KQ = 0 / 1: 128- or 64-row tiles, a comparison knob)
+    const int avg = pairs / n_slots;
+    int tm = kf_knob_on(KF_KNOB_MOE_KQ) ? (kf_knob(KF_KNOB_MOE_KQ) ? 2 : 4) : kf_knob_or(KF_KNOB_KQ_TM, avg <= 24 ? 1 : avg <= 64 ? 2 : 4);
     const KqMoe moe{offsets, out_rows, static_cast<const uint8_t*>(w2), expert_bytes, n_slots, n_split};
-    // Grids of at most two rounds of the CUs (by the tile bound; down at 512 tokens top-2: 384 tiles, about 320 live)
-    // run every tile as two K halves: a second round a quarter full would otherwise take as long as a full one. It
-    // needs the split scratch, one partial tile per tile (KF_GEMM_NO_TAIL turns it off, a comparison knob)
-    const int T = ((N + KQ_BN - 1) / KQ_BN) * mt;
-    KqTail split{nullptr, nullptr, 0, 1};
-    int blocks = T;
-    if (T <= 2 * kf_cu_count() && K / 256 >= 4 && T <= KF_SPLIT_TICKETS &&
-        (size_t)T * KQ_TM * 16 * KQ_THREADS * 4 <= KF_SPLIT_SCRATCH - (size_t)KF_SPLIT_TICKETS * 4 && !kf_knob_on(KF_KNOB_GEMM_NO_TAIL)) {
-        if (char* scr = static_cast<char*>(kf_split_scratch(s))) {
-            split = KqTail{reinterpret_cast<float*>(scr + (size_t)KF_SPLIT_TICKETS * 4), reinterpret_cast<int*>(scr), 0, 2};
-            blocks = 2 * T;
-        }
-    }
-    gemm_kq_kernel<KF_TYPE_Q4_K, true><<<blocks, KQ_THREADS, 0, s>>>(
-        static_cast<const uint8_t*>(w), row_bytes, reinterpret_cast<const int8_t*>(base + o.q), reinterpret_cast<const _Float16*>(base + o.xa),
-        reinterpret_cast<const float*>(base + o.d32), nullptr, nullptr, y, mt * KQ_BM, N, K, split, moe);
-    return hipGetLastError();
+    // every CU takes an equal range of the tiles (without the scratch: the tiles that start in it)
+    const int G = kq_max_ranges(tm, kf_cu_count());
+    // KF_GEMM_NO_TAIL: without the scratch (a comparison knob)
+    const KqWork work = kf_knob_on(KF_KNOB_GEMM_NO_TAIL) ? KqWork{nullptr, nullptr, 0, G} : kq_work(s, 0, G);
+#define KQ_GO(TM)                                                                                                                             \
+    return kq_run<KF_TYPE_Q4_K, TM, true>(G, s, static_cast<const uint8_t*>(w), row_bytes, reinterpret_cast<const int8_t*>(base + o.q),      \
+                                          reinterpret_cast<const _Float16*>(base + o.xa), reinterpret_cast<const float*>(base + o.d32),      \
+                                          nullptr, nullptr, y, pairs, N, K, work, moe)
+    if (tm == 1) KQ_GO(1);
+    if (tm == 2) KQ_GO(2);
+    KQ_GO(4);
+#undef KQ_GO
 }

@@ -46,7 +46,7 @@ inline int kf_cu_count() {
 // at the same time. A slot starts with KF_SPLIT_TICKETS int32 tickets, which the kernels leave at zero when they end.
 // Null (and the products take their scratch-free form) for a stream that finds every stream slot held by other
 // streams, and under capture when KF_CAPTURE_NO_SPLIT is set.
-constexpr size_t KF_SPLIT_SCRATCH = 40u << 20;
+constexpr size_t KF_SPLIT_SCRATCH = 68u << 20;
 constexpr int KF_SPLIT_STREAM_SLOTS = 2;
 constexpr int KF_SPLIT_SLOTS = KF_SPLIT_STREAM_SLOTS + 1;
 constexpr int KF_SPLIT_TICKETS = 1 << 16;

@@ -17,9 +17,9 @@ enum KfKnob : int {
     KF_KNOB_RM_NB,           // value: stage buffers of the grouped matrix-core product
     KF_KNOB_RM_WHOLE,        // value: whole tiles a wave in the grouped matrix-core product
     KF_KNOB_RM1_TILES,       // value: tiles a block of the one-matrix few-row product
-    KF_KNOB_Q4K_KQ,          // value: 0 / 1 forces the q4_K prefill GEMM kernel
-    KF_KNOB_KQ_GEMM,         // value: 0 / 1 forces q5_K / q6_K few-row product or GEMM
-    KF_KNOB_MOE_KQ,          // value: 0 selects the split-scale grouped MoE GEMM
+    KF_KNOB_Q4K_KQ,          // value: 0 / 1 forces 128- / 64-row tiles in the q4_K GEMM
+    KF_KNOB_KQ_GEMM,         // value: 0 / 1 forces the K types' few-row product or GEMM
+    KF_KNOB_MOE_KQ,          // value: 0 / 1 forces 128- / 64-row tiles in the grouped MoE GEMM
     KF_KNOB_GEMM_NO_TAIL,    // flag: no K-split tail rounds in the tile GEMMs
     KF_KNOB_GEMM_TILE,       // flag: q8_0 always on the tile GEMM
     KF_KNOB_GEMM_SLICE,      // value: 0 / 1 forces 64-row slices for 65.. q8_0 rows
@@ -32,6 +32,8 @@ enum KfKnob : int {
     KF_KNOB_GEMM_SMALL_TN,   // value: 16-column tiles a wave of the small-batch kernel
     KF_KNOB_CAPTURE_NO_SPLIT,  // flag: products under graph capture take the scratch-free forms
     KF_KNOB_GEMV_BURST,      // value: the burst GEMV takes grids of up to this many rows a wave (0: none; default 1)
+    KF_KNOB_KQ_TM,           // value: 1 / 2 / 4 forces the K-quant GEMM's 32-row tiles a block
+    KF_KNOB_KQ_G,            // value: range blocks of the K-quant GEMM's last tiles
     KF_KNOB_COUNT
 };
 

@@ -1,0 +1,90 @@
+"""The K-quant tile GEMM (gemm_kq.hip) at the sizes where its tiling can go wrong: super-block counts that start q6_K rows
+at every even byte offset, row counts around the 32-row tiles of a block, output columns around the 256-column tiles, split
+and unsplit, and the grouped form's ranges over uneven slots. Outputs against the CPU backend's int8 path (the same
+integers; the f32 sums of at most 56 super-blocks differ by their order only)."""
+import numpy as np
+import pytest
+
+import kungfu_amd as kf
+import oracle
+
+pytestmark = pytest.mark.gpu
+K_TYPES = [kf.TYPE_Q4_K, kf.TYPE_Q5_K, kf.TYPE_Q6_K]
+
+
+def _t(a, dev):
+    import torch
+
+    return torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+
+
+def _blocks(ty, n_out, n, seed):
+    return kf.quantize(ty, kf.synth_normal(seed, 0.02, n_out * n).reshape(n_out, n))
+
+
+def _close(got, want):
+    # 2^-24 for each of a row's sums of up to 56 super-block terms of magnitude below 8
+    err = np.abs(got.astype(np.float64) - want.astype(np.float64))
+    assert err.max() <= 56 * 2.0**-24 * 8, f"max err {err.max():.3e}"
+
+
+@pytest.mark.parametrize("tm", [1, 2, 4])
+@pytest.mark.parametrize("ty", K_TYPES)
+@pytest.mark.parametrize("rows,n,n_out", [(2, 256, 1), (31, 768, 255), (33, 1280, 257), (65, 1792, 40), (129, 2304, 300), (96, 2560, 33),
+                                          (128, 3328, 256), (40, 14336, 70)])
+def test_tile_edges(cuda, knobs, ty, tm, rows, n, n_out):
+    import torch
+
+    w = _blocks(ty, n_out, n, rows + n + n_out)
+    x = kf.synth_normal(rows + n, 1.0, rows * n).reshape(rows, n)
+    bias, res = kf.synth_normal(3, 1.0, n_out), kf.synth_normal(4, 1.0, rows * n_out).reshape(rows, n_out)
+    want = oracle.matmul_i8(ty, w, n, n_out, x, bias) + res
+    knobs.setenv("KF_KQ_GEMM", 1)
+    knobs.setenv("KF_KQ_TM", tm)
+    # a guard row behind the matrix: reads past its last 16-byte piece would meet it
+    wt = torch.full((w.size + 4096,), 255, dtype=torch.uint8, device=cuda)
+    wt[: w.size] = _t(w.reshape(-1), cuda)
+    act = kf.alloc_act(rows, n, cuda)
+    got = []
+    for _ in range(2):
+        y = torch.full((rows, n_out), float("nan"), device=cuda)
+        kf.matmul(ty, wt, _t(x, cuda), act, y, n_out, bias=_t(bias, cuda), res=_t(res, cuda))
+        torch.cuda.synchronize()
+        got.append(y.cpu().numpy())
+    _close(got[0], want)
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    knobs.setenv("KF_GEMM_NO_TAIL", 1)
+    kf.matmul(ty, wt, _t(x, cuda), act, y, n_out, bias=_t(bias, cuda), res=_t(res, cuda))
+    torch.cuda.synchronize()
+    _close(y.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("scratch", [True, False])
+@pytest.mark.parametrize("tm", [1, 2, 4])
+@pytest.mark.parametrize("counts", [(1,), (0, 33, 0, 128, 5), (97, 96, 95, 64, 1, 0, 0, 31), tuple((7 * i) % 41 for i in range(70))])
+def test_grouped_ranges(cuda, knobs, counts, tm, scratch):
+    """Slots of no, few and many rows (more than 64 of them: two steps of the slot search) cut into ranges that start and end
+    inside tiles; the output rows through a permutation, and the two-matrix form's columns past the split."""
+    import torch
+
+    ty, n, half = kf.TYPE_Q4_K, 512, 256
+    pairs, n_slots = sum(counts), len(counts)
+    offs = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    wa, wb = (_blocks(ty, n_slots * half, n, s) for s in (11, 12))
+    x = kf.synth_normal(pairs, 1.0, pairs * n).reshape(pairs, n)
+    rows = np.random.default_rng(pairs).permutation(pairs).astype(np.int32)
+    knobs.setenv("KF_KQ_TM", tm)
+    if not scratch:
+        knobs.setenv("KF_GEMM_NO_TAIL", 1)
+    act = kf.alloc_act(pairs, n, cuda)
+    kf.quant_act(_t(x, cuda), act, kf.ACT_Q8K)
+    y = torch.full((pairs, 2 * half), float("nan"), device=cuda)
+    kf.moe_gemm(ty, _t(wa, cuda), act, pairs, n, 2 * half, _t(offs, cuda), n_slots, y, half * kf.row_bytes(ty, n), w2=_t(wb, cuda), n_split=half,
+                out_rows=_t(rows, cuda))
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()[rows]
+    for s in range(n_slots):
+        r0, r1 = offs[s], offs[s + 1]
+        if r1 > r0:
+            for at, w in ((0, wa), (half, wb)):
+                _close(got[r0:r1, at : at + half], oracle.matmul_i8(ty, w[s * half : (s + 1) * half], n, half, x[r0:r1], None))
