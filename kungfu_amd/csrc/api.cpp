@@ -45,8 +45,13 @@ hipError_t kf_launch_gemm_q8_0(const void* w, int64_t row_bytes, const void* act
                                int N, int K, hipStream_t s);
 int kf_gemm_k_multiple();
 
+bool kf_gemm_q8_below(int M, int N, int K, double us);
+hipError_t kf_launch_gemm_q8(const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y, int M, int N, int K,
+                             hipStream_t s);
+static bool q8_gemm_pays(int rows, int n_in, int n_out, int64_t row_bytes, bool multi);
+
 bool kf_gemm_kq_ok(uint32_t ty, const void* w, int64_t row_bytes, int K, int N);
-double kf_gemm_kq_us(uint32_t ty, int M, int N, int K);
+bool kf_gemm_kq_below(uint32_t ty, int M, int N, int K, double us);
 hipError_t kf_launch_gemm_kq_moe(const void* w, const void* w2, int64_t expert_bytes, int64_t row_bytes, int n_split, const void* act, int pairs,
                                  int n_slots, const int32_t* offsets, const int32_t* out_rows, float* y, int N, int K, hipStream_t s);
 static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes);
@@ -211,6 +216,10 @@ int kf_hip_gemv(uint32_t ty, const void* w, int64_t row_bytes, const void* act, 
     const int rc = check_product(ty, w, row_bytes, act, y, rows, n, n_out);
     if (rc != KF_OK) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (ty == KF_TYPE_Q8_0 && n_out > 0 && q8_gemm_pays(rows, n, n_out, row_bytes, false)) {
+        const hipError_t e = kf_launch_gemm_q8(w, row_bytes, act, bias, res, y, rows, n_out, n, s);
+        return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
+    }
     // the K types: the tile GEMM where its cost is below the few-row product's
     if (ty != KF_TYPE_Q8_0 && n_out > 0 && kq_gemm_pays(ty, w, rows, n, n_out, row_bytes)) {
         const hipError_t e = kf_launch_gemm_kq(ty, w, row_bytes, act, bias, res, y, rows, n_out, n, s);
@@ -260,6 +269,10 @@ int kf_hip_gemm_i8(uint32_t ty, const void* w, int64_t row_bytes, const void* ac
     }
     if (ty != KF_TYPE_Q8_0) return fail(KF_E_UNSUPPORTED, "the int8 GEMM runs q8_0, q4_K, q5_K and q6_K weights (type %u given)", ty);
     if (n % kf_gemm_k_multiple() != 0) return fail(KF_E_INVALID, "%d columns, the GEMM needs a multiple of %d", n, kf_gemm_k_multiple());
+    if (n_out > 0 && q8_gemm_pays(rows, n, n_out, row_bytes, true)) {
+        const hipError_t e = kf_launch_gemm_q8(w, row_bytes, act, bias, res, y, rows, n_out, n, static_cast<hipStream_t>(stream));
+        return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
+    }
     const hipError_t e = kf_launch_gemm_q8_0(w, row_bytes, act, bias, res, y, rows, n_out, n, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
 }
@@ -310,12 +323,12 @@ int kf_hip_rms_norm_matmul(uint32_t ty, const void* w, int n_in, int n_out, cons
 
 // The few-row products' cost on the K types (MI355X, us; fitted over 4-128 rows at 4096 -> 4096, 4096 -> 14336 and
 // 14336 -> 4096): about 5.5 plus, per 16 activation rows and MB of weights, 0.22 (q4_K), 0.20 (q5_K) or 0.32 (q6_K). q6_K
-// rows that start off a dword (an odd number of super-blocks) run the per-lane product, 1.35 us per MB and eight rows;
-// q4_K rows wider than the few-row product stages run as one GEMV launch per row.
+// rows that start off a dword (an odd number of super-blocks) run the per-lane product, whose cost grows with each row
+// (1792 -> 3584, 6400 -> 2304 and 13056 -> 2048 at 2-16 rows: 7.1-36.6, 11.7-53.3 and 15.8-69.8 us); q4_K rows wider than the few-row product stages run as one GEMV launch per row.
 static double kq_few_rows_us(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes) {
     const double mb = (double)n_out * row_bytes / 1e6;
     if (ty == KF_TYPE_Q4_K && n_in > kf_rows_max_n(ty)) return rows * (2.5 + 0.22 * mb);
-    if (!kf_rows_mma_1_ok(ty, w, row_bytes, n_in, n_out, rows)) return 5.5 + (rows + 7) / 8 * (1.35 * mb + 2.0);
+    if (!kf_rows_mma_1_ok(ty, w, row_bytes, n_in, n_out, rows)) return 2.0 + (rows + 7) / 8 * (1.0 + 0.3 * mb) + rows * (0.9 + 0.13 * mb);
     return 5.5 + (rows + 15) / 16 * mb * (ty == KF_TYPE_Q4_K ? 0.22 : ty == KF_TYPE_Q5_K ? 0.20 : 0.32);
 }
 
@@ -323,7 +336,34 @@ static double kq_few_rows_us(uint32_t ty, const void* w, int rows, int n_in, int
 static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes) {
     if (rows < 2 || !kf_gemm_kq_ok(ty, w, row_bytes, n_in, n_out)) return false;
     if (kf_knob_on(KF_KNOB_KQ_GEMM)) return kf_knob(KF_KNOB_KQ_GEMM) != 0;
-    return kf_gemm_kq_us(ty, rows, n_out, n_in) < kq_few_rows_us(ty, w, rows, n_in, n_out, row_bytes);
+    return kf_gemm_kq_below(ty, rows, n_out, n_in, kq_few_rows_us(ty, w, rows, n_in, n_out, row_bytes));
+}
+
+// The older q8_0 products' cost (MI355X, us; fitted over 4-2048 rows at the shapes of gemm_q8.hip's model). kf_hip_gemv's
+// multi-row product costs so much a row (1888 -> 1774: 9.3 us at 9 rows, 14.2 at 16; 4128 -> 2048: 16.4 and 25.0), and past the
+// width it stages is one GEMV a row. kf_hip_gemm_i8's: up to 64 rows the small-batch kernels by the weights' MB, past that the
+// 128 x 128 tile kernel (two blocks a CU) by its tiles and 128-column stages, or 64-row slices through the small-batch
+// kernels; these need rows of whole 256-column steps, and other widths have only the tile GEMM.
+static double q8_old_us(int rows, int n_in, int n_out, int64_t row_bytes, bool multi) {
+    const double mb = (double)n_out * row_bytes / 1e6;
+    if (!multi) return n_in > kf_rows_max_n(KF_TYPE_Q8_0) ? rows * (3.0 + 0.22 * mb) : 1.7 + 0.26 * mb + rows * (0.33 + 0.11 * mb);
+    if (n_in % 256 != 0) return 1e30;
+    if (rows <= 64) return rows <= 16 ? 4.5 + 0.2 * mb : rows <= 32 ? 7.5 + 0.20 * mb : 10.5 + 0.33 * mb;
+    const double t = (double)((n_out + 127) / 128) * ((rows + 127) / 128), st = n_in / 128;
+    return std::min(6.0 + st * (t > 256 ? 3.2 * t / 512 : 0.75 + t / 224), ((rows + 63) / 64) * (9.0 + 0.45 * mb));
+}
+
+// Whether the q8_0 tile GEMM of any width (gemm_q8.hip) beats the product the entry point took before it (multi:
+// kf_hip_gemm_i8's). kf_hip_gemv keeps its one-pass product up to eight rows. The knobs that force an older kernel keep
+// forcing it; KF_Q8_V = 0-2 forces this one, 3 the older ones (a comparison knob)
+static bool q8_gemm_pays(int rows, int n_in, int n_out, int64_t row_bytes, bool multi) {
+    if (rows < 2) return false;
+    if (kf_knob_on(KF_KNOB_Q8_V)) return kf_knob(KF_KNOB_Q8_V) < 3;
+    if (!multi && rows <= 8) return false;
+    for (KfKnob k : {KF_KNOB_GEMM_TILE, KF_KNOB_GEMM_SLICE, KF_KNOB_GEMM_SK, KF_KNOB_GEMM_SK_S, KF_KNOB_GEMM_SK_V, KF_KNOB_GEMM_NO_MR, KF_KNOB_GEMM_MR,
+                     KF_KNOB_GEMM_SMALL_W, KF_KNOB_GEMM_SMALL_TN})
+        if (kf_knob_on(k)) return false;
+    return kf_gemm_q8_below(rows, n_out, n_in, q8_old_us(rows, n_in, n_out, row_bytes, multi));
 }
 
 namespace {
@@ -335,6 +375,12 @@ int product(uint32_t ty, const void* w, int64_t rb, const void* act, const float
     // several q8_0 rows are the int8 GEMM, which reads each weight byte once per 128 rows
     if (rows > 1 && ty == KF_TYPE_Q8_0 && n_in % kf_gemm_k_multiple() == 0 && n_out > 0)
         return kf_hip_gemm_i8(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream);
+    // other widths of q8_0: no older product but the multi-row one, which the tile GEMM beats from a few rows on
+    if (rows > 1 && ty == KF_TYPE_Q8_0 && n_out > 0 && !kf_knob_on(KF_KNOB_Q8_V) &&
+        kf_gemm_q8_below(rows, n_out, n_in, q8_old_us(rows, n_in, n_out, rb, false))) {
+        const hipError_t e = kf_launch_gemm_q8(w, rb, act, bias, res, y, rows, n_out, n_in, static_cast<hipStream_t>(stream));
+        return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
+    }
     // the K types: kf_hip_gemv picks the tile GEMM or the few-row product
     return kf_hip_gemv(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream);
 }

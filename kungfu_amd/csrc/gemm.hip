@@ -5,14 +5,10 @@
 // first unpacks native bytes into an int8 + f32-scale form; here the q8_0 rows are read unchanged (a q8_0 block is
 // already int8 with one f16 scale per 32) and only their 32 weight bytes are moved into LDS tiles.
 //
+// The tile kernel here (128 x 128, two blocks a CU, K a multiple of 256) stays for the grids that gemm_q8.hip's 256-column
+// tiles fill badly; other widths and most row counts run there.
+//
 // gfx950 design:
-//   * Four waves per block in a WM x WN grid, each computing TM x TN tiles of 32 x 32, so a block tile is
-//     (32 WM TM) x (32 WN TN): 128 x 128 for prefill, 32 x 128 / 64 x 128 for small batches.
-//   * K advances 128 columns (four groups) per stage. The next stage's global loads are in flight in registers while
-//     the current one is multiplied from LDS; LDS is double-buffered with one barrier per stage.
-//   * An operand tile of 32 rows x 32 bytes sits in LDS as two halves of 32 slots of 16 bytes, in the order the MFMA
-//     consumes (lane l reads slot l % 32 of half l / 32), with the slot XOR-swizzled by the piece's (group, half) so
-//     that both the row-contiguous stores and the operand reads hit 16 distinct bank quads per 16 lanes.
 //   * Per group and 32 x 32 tile: one v_mfma_i32_32x32x32_i8 gives the exact int32 dots I_g; one
 //     v_mfma_f32_32x32x16_f16 with a single non-zero k slot gives the exact outer product d_x (x) d_w of the group's
 //     f16 scales (q8_0 weight scales are f16, Q8_0-kind activation scales are f16-rounded); the VALU converts I_g and
@@ -38,205 +34,20 @@
 #error "the split-K fixups assume gfx950's cache and counter behaviour"
 #endif
 
+hipError_t kf_launch_gemm_q8(const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y, int M, int N, int K,
+                             hipStream_t s);
+
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int GM_BK = 128;  // columns per stage: four 32-column groups
 constexpr int GM_G = GM_BK / 32;
-constexpr int GM_THREADS = 256;
-
-template <int WM, int WN, int TM, int TN>
-struct GmCfg {
-    static_assert(WM * WN == 4, "four waves");
-    static constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
-    static constexpr int A_BYTES = BM * GM_BK, B_BYTES = BN * GM_BK;
-    static constexpr int SA = A_BYTES + B_BYTES;          // f16 activation scales [g][BM]
-    static constexpr int SB = SA + GM_G * BM * 2;         // f16 weight scales [g][BN]
-    static constexpr int STAGE = SB + GM_G * BN * 2;
-    static constexpr int PA = BM * 8 / GM_THREADS;        // 16-byte pieces a thread moves per stage
-    static constexpr int PB = BN * 8 / GM_THREADS;
-    static constexpr int QA = (BM * GM_G + GM_THREADS - 1) / GM_THREADS;  // scales a thread moves per stage
-    static constexpr int QB = (BN * GM_G + GM_THREADS - 1) / GM_THREADS;
-    static_assert(PA >= 1 && PB >= 1, "a block tile spans at least 32 rows");
-};
-
-// Byte offset of the 16-byte piece (group g, tile row r, half h) in an operand tile of `tiles` 32-row tiles
-__device__ __forceinline__ int gm_slot(int tiles, int g, int r, int h) {
-    return (((g * tiles + (r >> 5)) * 2 + h) * 32 + ((r & 31) ^ ((g * 2 + h) << 1))) * 16;
-}
-
-// The piece a lane reads for the MFMA operand of tile t, group g: row lane % 32, half lane / 32
-__device__ __forceinline__ int gm_operand(int tiles, int g, int t, int lane) {
-    const int h = lane >> 5;
-    return (((g * tiles + t) * 2 + h) * 32 + ((lane & 31) ^ ((g * 2 + h) << 1))) * 16;
-}
-
-template <class C>
-struct GmStage {
-    uint4 a[C::PA], b[C::PB];
-    float dx[C::QA];
-    uint32_t dw[C::QB];
-
-    __device__ __forceinline__ void load(const uint8_t* __restrict__ w, int64_t row_bytes, const int8_t* __restrict__ xq,
-                                         const float* __restrict__ xd32, int m0, int n0, int M, int N, int K, int st, int tid) {
-        const int gb = st * GM_G;
-        const int kg = K >> 5;
-#pragma unroll
-        for (int i = 0; i < C::PA; i++) {
-            const int c = tid + GM_THREADS * i;  // eight consecutive threads read one row's 128 bytes
-            const int m = min(m0 + (c >> 3), M - 1);
-            a[i] = *reinterpret_cast<const uint4*>(xq + (int64_t)m * K + gb * 32 + (c & 7) * 16);
-        }
-#pragma unroll
-        for (int i = 0; i < C::PB; i++) {
-            const int c = tid + GM_THREADS * i;
-            const int n = min(n0 + (c >> 3), N - 1);
-            const int p = c & 7;
-            const u32x4_a2 v = *reinterpret_cast<const u32x4_a2*>(w + (int64_t)n * row_bytes + (int64_t)(gb + (p >> 1)) * KF_Q8_0_BYTES + 2 +
-                                                                  16 * (p & 1));
-            b[i] = make_uint4(v.x, v.y, v.z, v.w);
-        }
-#pragma unroll
-        for (int i = 0; i < C::QA; i++) {
-            const int c = min(tid + GM_THREADS * i, C::BM * GM_G - 1);  // row c / 4, group c % 4
-            const int m = min(m0 + (c >> 2), M - 1);
-            dx[i] = xd32[(int64_t)m * kg + gb + (c & 3)];
-        }
-#pragma unroll
-        for (int i = 0; i < C::QB; i++) {
-            const int c = min(tid + GM_THREADS * i, C::BN * GM_G - 1);
-            const int n = min(n0 + (c >> 2), N - 1);
-            dw[i] = *reinterpret_cast<const uint16_t*>(w + (int64_t)n * row_bytes + (int64_t)(gb + (c & 3)) * KF_Q8_0_BYTES);
-        }
-    }
-
-    __device__ __forceinline__ void store(uint8_t* buf, int tid) const {
-#pragma unroll
-        for (int i = 0; i < C::PA; i++) {
-            const int c = tid + GM_THREADS * i;
-            const int p = c & 7;
-            *reinterpret_cast<uint4*>(buf + gm_slot(C::BM / 32, p >> 1, c >> 3, p & 1)) = a[i];
-        }
-#pragma unroll
-        for (int i = 0; i < C::PB; i++) {
-            const int c = tid + GM_THREADS * i;
-            const int p = c & 7;
-            *reinterpret_cast<uint4*>(buf + C::A_BYTES + gm_slot(C::BN / 32, p >> 1, c >> 3, p & 1)) = b[i];
-        }
-#pragma unroll
-        for (int i = 0; i < C::QA; i++) {
-            const int c = tid + GM_THREADS * i;
-            // Q8_0-kind activation scales are f16-rounded values, so this conversion is exact
-            if (C::QA * GM_THREADS == C::BM * GM_G || c < C::BM * GM_G)
-                reinterpret_cast<_Float16*>(buf + C::SA)[(c & 3) * C::BM + (c >> 2)] = (_Float16)dx[i];
-        }
-#pragma unroll
-        for (int i = 0; i < C::QB; i++) {
-            const int c = tid + GM_THREADS * i;
-            if (C::QB * GM_THREADS == C::BN * GM_G || c < C::BN * GM_G)
-                reinterpret_cast<uint16_t*>(buf + C::SB)[(c & 3) * C::BN + (c >> 2)] = (uint16_t)dw[i];
-        }
-    }
-};
-
-// One block: output tile (blockIdx.y, blockIdx.x) over all of K
-template <int WM, int WN, int TM, int TN>
-__global__ void __launch_bounds__(GM_THREADS, 2) gemm_q8_0_kernel(const uint8_t* __restrict__ w, int64_t row_bytes, const int8_t* __restrict__ xq,
-                                                                  const float* __restrict__ xd32, const float* __restrict__ bias,
-                                                                  const float* __restrict__ res, float* __restrict__ y, int M, int N, int K) {
-    using C = GmCfg<WM, WN, TM, TN>;
-    extern __shared__ __align__(16) uint8_t smem[];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WN, wn = wave % WN;
-    const int m0 = blockIdx.y * C::BM, n0 = blockIdx.x * C::BN;
-    const int st0 = 0, st1 = K / GM_BK;
-
-    v16f acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = v16f{};
-
-    GmStage<C> pf;
-    pf.load(w, row_bytes, xq, xd32, m0, n0, M, N, K, st0, tid);
-    pf.store(smem, tid);
-    __syncthreads();
-    for (int st = st0; st < st1; st++) {
-        const uint8_t* buf = smem + ((st - st0) & 1) * C::STAGE;
-        // the last stage reloads itself: an unconditional load keeps the prefetch registers out of any phi
-        pf.load(w, row_bytes, xq, xd32, m0, n0, M, N, K, min(st + 1, st1 - 1), tid);
-        // the operands of group g + 1 are read from LDS while group g is multiplied and rescaled; the scale operands
-        // of the outer-product MFMA carry one f16 in k slot 0 (lanes < 32; lanes >= 32 hold k slots 8..15) and
-        // zeros elsewhere, and only their first dword changes from group to group
-        struct Ops {
-            v4i a[TM], b[TN];
-            uint32_t sa[TM], sb[TN];
-        };
-        auto read_ops = [&](Ops& o, int g) {
-#pragma unroll
-            for (int t = 0; t < TM; t++) {
-                o.a[t] = *reinterpret_cast<const v4i*>(buf + gm_operand(C::BM / 32, g, wm * TM + t, lane));
-                const uint16_t v = reinterpret_cast<const uint16_t*>(buf + C::SA)[g * C::BM + (wm * TM + t) * 32 + (lane & 31)];
-                o.sa[t] = lane < 32 ? v : 0u;
-            }
-#pragma unroll
-            for (int t = 0; t < TN; t++) {
-                o.b[t] = *reinterpret_cast<const v4i*>(buf + C::A_BYTES + gm_operand(C::BN / 32, g, wn * TN + t, lane));
-                o.sb[t] = reinterpret_cast<const uint16_t*>(buf + C::SB)[g * C::BN + (wn * TN + t) * 32 + (lane & 31)];
-            }
-        };
-        Ops cur;
-        read_ops(cur, 0);
-#pragma unroll 1
-        for (int g = 0; g < GM_G; g++) {
-            Ops nxt;
-            read_ops(nxt, min(g + 1, GM_G - 1));
-#pragma unroll
-            for (int i = 0; i < TM; i++) {
-                v16i c[TN];
-                v16f s[TN];
-#pragma unroll
-                for (int j = 0; j < TN; j++) {
-                    c[j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur.a[i], cur.b[j], v16i{}, 0, 0, 0);
-                    const v4u sa = {cur.sa[i], 0u, 0u, 0u}, sb = {cur.sb[j], 0u, 0u, 0u};
-                    s[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, sa), __builtin_bit_cast(v8h, sb), v16f{}, 0, 0, 0);
-                }
-#pragma unroll
-                for (int j = 0; j < TN; j++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) acc[i][j][r] = fmaf((float)c[j][r], s[j][r], acc[i][j][r]);
-            }
-            cur = nxt;
-        }
-        if (st + 1 < st1) pf.store(smem + ((st + 1 - st0) & 1) * C::STAGE, tid);
-        __syncthreads();
-    }
-
-    // 32 x 32 accumulator layout: lane l holds column l % 32; register r holds row (r % 4) + 8 * (r / 4) + 4 * (l / 32)
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int n = n0 + (wn * TN + j) * 32 + (lane & 31);
-            if (n >= N) continue;
-            const float bn = bias ? bias[n] : 0.0f;
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int m = m0 + (wm * TM + i) * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
-                if (m >= M) continue;
-                const int64_t o = (int64_t)m * N + n;
-                y[o] = acc[i][j][r] + bn + (res ? res[o] : 0.0f);
-            }
-        }
-}
 
 // Decode-batch product (up to MR activation rows). Block x owns 32 output columns [32 x, +32); its W waves take the
 // 8-group chunks of K round-robin. A chunk is 272 bytes of each of the 32 weight rows (17 aligned 16-byte pieces, so a
@@ -1203,19 +1014,6 @@ hipError_t gemm_q8_0_dma_launch(const uint8_t* w, int64_t row_bytes, const int8_
     return hipGetLastError();
 }
 
-template <int WM, int WN, int TM, int TN>
-hipError_t gemm_launch(const uint8_t* w, int64_t row_bytes, const int8_t* xq, const float* xd32, const float* bias, const float* res, float* y,
-                       int M, int N, int K, hipStream_t s) {
-    using C = GmCfg<WM, WN, TM, TN>;
-    auto* fn = gemm_q8_0_kernel<WM, WN, TM, TN>;
-    // the double-buffered stage needs more than the default 64 KB of LDS
-    const hipError_t e = kf_raise_lds(reinterpret_cast<const void*>(fn), 2 * C::STAGE);
-    if (e != hipSuccess) return e;
-    dim3 grid((N + C::BN - 1) / C::BN, (M + C::BM - 1) / C::BM);
-    fn<<<grid, GM_THREADS, 2 * C::STAGE, s>>>(w, row_bytes, xq, xd32, bias, res, y, M, N, K);
-    return hipGetLastError();
-}
-
 template <int MR, int TN>
 hipError_t gemm_small_launch(const uint8_t* w, int64_t row_bytes, const int8_t* xq, const float* xd32, const float* bias, const float* res,
                              float* y, int M, int N, int K, int W, hipStream_t s) {
@@ -1245,9 +1043,6 @@ int small_waves(int M, int N, int K, int rows_per_block) {
 
 int kf_gemm_k_multiple() { return GM_BK; }
 
-
-
-// Host launcher, validated by the caller (api.cpp): K a multiple of 128, Q8_0-kind activations in `act`
 // Whether 65.. q8_0 rows run faster as 64-row slices through the small-batch products than on the tile GEMM
 // (MI355X, Llama-3-8B shapes at 96-512 rows; the model picks the faster form at all 24 measured points): a 64-row
 // slice costs about 9 us + 0.45 us per weight MB, the tile GEMM about 3 us per 128-column stage per round of one
@@ -1318,6 +1113,7 @@ static hipError_t small_q8_0(const uint8_t* wb, int64_t row_bytes, const int8_t*
     return hipErrorNotSupported;
 }
 
+// Host launcher, validated by the caller (api.cpp): K a multiple of 128, Q8_0-kind activations in `act`
 hipError_t kf_launch_gemm_q8_0(const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y, int M,
                                int N, int K, hipStream_t s) {
     const kf_act_offsets o = kf_act_layout((size_t)M, (size_t)K);
@@ -1341,5 +1137,5 @@ hipError_t kf_launch_gemm_q8_0(const void* w, int64_t row_bytes, const void* act
         }
     }
     if (K % 256 == 0 && row_bytes % 16 == 0) return gemm_q8_0_dma_launch<2, 4, 2, 1>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, s);
-    return gemm_launch<2, 2, 2, 2>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, s);
+    return kf_launch_gemm_q8(w, row_bytes, act, bias, res, y, M, N, K, s);
 }

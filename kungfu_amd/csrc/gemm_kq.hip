@@ -882,7 +882,8 @@ KqPlan kq_plan_tm(uint32_t ty, int tm, int M, int N, int K) {
     // the tiles of the last round as S blocks each, S the cheapest that fits the CUs with two super-blocks a block or more
     double tail = rem ? KQ_ROUND_US[t] + sb * nsb : 0.0;
     for (int S = 2; rem && rem * S <= max_g && 2 * S <= nsb; S++) {
-        const double us = KQ_ROUND_US[t] + sb * ((nsb + S - 1) / S) + KQ_PART_US[t] * tm * rem * S / cus;
+        const double part = KQ_ROUND_US[t] + KQ_PART_US[t] * tm * rem * S / cus, us = part + sb * ((nsb + S - 1) / S);
+        if (part + 2 * sb >= tail) break;
         if (us < tail) {
             tail = us;
             p.full = p.T - rem;
@@ -930,7 +931,13 @@ hipError_t kq_run(int blocks, hipStream_t s, const uint8_t* w, int64_t row_bytes
 
 }  // namespace
 
-double kf_gemm_kq_us(uint32_t ty, int M, int N, int K) { return kq_plan(ty, M, N, K).us; }
+// Whether the product costs less than `us`. What no plan goes below comes first: the plan's search would cost the shortest
+// products a noticeable part of their launch.
+bool kf_gemm_kq_below(uint32_t ty, int M, int N, int K, double us) {
+    if (1.8 + KQ_ROUND_US[0] + std::min(K / 256, 2) * KQ_SB_US[0][0] >= us) return false;
+    const KqPlan p = kq_plan(ty, M, N, K);
+    return p.us + (p.S > 1 ? 2.0 : 0.0) < us;  // the second launch's host work, which a short product does not hide
+}
 
 // Host launcher, validated by the caller (kf_gemm_kq_ok; Q8K-kind activations in `act`)
 hipError_t kf_launch_gemm_kq(uint32_t ty, const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y,

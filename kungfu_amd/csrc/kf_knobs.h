@@ -34,6 +34,7 @@ enum KfKnob : int {
     KF_KNOB_GEMV_BURST,      // value: the burst GEMV takes grids of up to this many rows a wave (0: none; default 1)
     KF_KNOB_KQ_TM,           // value: 1 / 2 / 4 forces the K-quant GEMM's 32-row tiles a block
     KF_KNOB_KQ_G,            // value: range blocks of the K-quant GEMM's last tiles
+    KF_KNOB_Q8_V,            // value: 0 / 1 / 2 forces 32- / 64- / 128-row tiles in the q8_0 GEMM; 3 the older q8_0 products
     KF_KNOB_COUNT
 };
 
