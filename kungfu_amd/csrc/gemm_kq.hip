@@ -934,7 +934,8 @@ hipError_t kq_run(int blocks, hipStream_t s, const uint8_t* w, int64_t row_bytes
 // Whether the product costs less than `us`. What no plan goes below comes first: the plan's search would cost the shortest
 // products a noticeable part of their launch.
 bool kf_gemm_kq_below(uint32_t ty, int M, int N, int K, double us) {
-    if (1.8 + KQ_ROUND_US[0] + std::min(K / 256, 2) * KQ_SB_US[0][0] >= us) return false;
+    const double least = std::min(K / 256 * KQ_SB_US[0][0], 2.0 + 2 * KQ_SB_US[0][0]);  // unsplit, split
+    if (1.8 + KQ_ROUND_US[0] + least >= us) return false;
     const KqPlan p = kq_plan(ty, M, N, K);
     return p.us + (p.S > 1 ? 2.0 : 0.0) < us;  // the second launch's host work, which a short product does not hide
 }

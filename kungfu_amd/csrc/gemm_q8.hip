@@ -27,6 +27,7 @@
 #include "kf_knobs.h"
 #include "kf_layout.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -383,7 +384,8 @@ Q8Plan q8_plan(int M, int N, int K) {
 // Whether the product costs less than `us`. What no plan goes below comes first: the plan's search would cost the shortest
 // products a noticeable part of their launch.
 bool kf_gemm_q8_below(int M, int N, int K, double us) {
-    if (Q8_LAUNCH_US[0] + Q8_ROUND_US[0] + Q8_ST_US[0] >= us) return false;
+    const double least = std::min((K / 32 + Q8_G - 1) / Q8_G * Q8_ST_US[0], 2.0 + 2 * Q8_ST_US[0]);  // unsplit, split
+    if (Q8_LAUNCH_US[0] + Q8_ROUND_US[0] + least >= us) return false;
     const Q8Plan p = q8_plan(M, N, K);
     return p.us + (p.S > 1 ? 2.0 : 0.0) < us;  // the second launch's host work, which a short product does not hide
 }
