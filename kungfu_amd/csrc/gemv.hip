@@ -1110,10 +1110,14 @@ hipError_t launch_gemv(const uint8_t* w, int64_t row_bytes, const int8_t* xq, co
     // row iterations per block: enough blocks that the chip is full, each block's waves holding the loads of all
     // their rows at once
     const int want = maxit_env > 0 ? maxit_env : KF_GV_MAXIT;
-    // the DMA variant needs 16-byte aligned rows and activation pieces
-    const bool dma = row_bytes % 16 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 &&
-                     (reinterpret_cast<uintptr_t>(fused ? static_cast<const void*>(xf) : xq) & 15) == 0 && !kf_knob_on(KF_KNOB_GEMV_NO_DMA);
-    if (fused && (SPW != 1 || !dma)) return hipErrorNotSupported;
+    // the DMA variants need 16-byte aligned rows and activation pieces. The pipelined one loads q8_0 rows at their 2-byte
+    // alignment, so widths that are no multiple of 256 (rows that start off a 16-byte piece) run it too and quantize
+    // their activation row in the same launch (us, before -> now, the product and its quantization: 1056 -> 1760 8.2 -> 4.0, 4064 ->
+    // 14000 25.8 -> 13.7; past the fused width 14368 -> 4096 30.5 -> 17.1)
+    const bool xa = (reinterpret_cast<uintptr_t>(fused ? static_cast<const void*>(xf) : xq) & 15) == 0 && !kf_knob_on(KF_KNOB_GEMV_NO_DMA);
+    const bool dma = row_bytes % 16 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0 && xa;
+    const bool pipe = TY == KF_TYPE_Q8_0 ? xa : dma;
+    if (fused && (SPW != 1 || !pipe)) return hipErrorNotSupported;
     // one-shot waves, each fetching its row straight into LDS, the whole matrix requested at launch (KF_GEMV_ONESHOT=1,
     // a comparison knob: one row a wave and every block resident at once). The persistent variant below measured
     // faster on q4_K QKV and O (5.34 / 4.25 us against 5.44 / 4.71) and level on q8_0, so it takes them too
@@ -1152,7 +1156,7 @@ hipError_t launch_gemv(const uint8_t* w, int64_t row_bytes, const int8_t* xq, co
         }
     }
     // the pipelined persistent variant: a resident grid, every wave walking its rows two in flight
-    if (SPW == 1 && dma && (fused || !kf_knob_on(KF_KNOB_GEMV_NO_PIPE))) {
+    if (SPW == 1 && pipe && (fused || !kf_knob_on(KF_KNOB_GEMV_NO_PIPE))) {
         const int dv = kf_knob(KF_KNOB_GEMV_DEPTH);
         const int depth = dv >= 2 && dv <= 4 ? dv : KF_GV_DEPTH;
         GvKernel k = fused ? gv_fused_pipe<TY, WPR>(qx, norm != nullptr)
@@ -1244,7 +1248,7 @@ int kf_gemv_fused_max_n() { return 2 * GV_WAVES * 256; }
 
 // The single-row GEMV quantizing its f32 activation row x itself (one launch in place of quant_act + GEMV; the same
 // integers and scales, so the same outputs bit for bit). hipErrorNotSupported when no fused variant fits (n above
-// kf_gemv_fused_max_n, rows or x not 16-byte aligned, a type other than q8_0 / q4_K): the caller quantizes first.
+// kf_gemv_fused_max_n, x or q4_K rows not 16-byte aligned, a type other than q8_0 / q4_K): the caller quantizes first.
 hipError_t kf_launch_gemv1_fused(uint32_t ty, const void* wv, int64_t row_bytes, const float* x, const float* bias, const float* res, float* y,
                                  int n, int n_out, const KfSegs* segs, hipStream_t s, const float* norm_w, const float* norm_b, float norm_eps,
                                  bool norm) {
