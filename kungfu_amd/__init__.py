@@ -210,10 +210,14 @@ def _ptr(t) -> int | None:
 
 
 def _stream(stream) -> int | None:
+    """The stream given, or torch's current one. Asking torch for the handle alone costs 0.2 us; its stream object, which a
+    process that has not used the GPU yet still needs, 2.9."""
     if stream is not None:
         return stream
     import torch
 
+    if torch.cuda.is_initialized():
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
     return torch.cuda.current_stream().cuda_stream
 
 
@@ -260,32 +264,44 @@ SEG_NONE = -(1 << 63)
 MAX_SEGMENTS = 4
 
 
+def _segments(members):
+    """The members' segment words as an int64 array of C, lead w, lead y."""
+    lead_w, lead_y = _ptr(members[0][0]), _ptr(members[0][1])
+    words, start = [], 0
+    for w, y, bias, res in members:
+        n_out = y.shape[-1]
+        words += (
+            _ptr(w) - lead_w,
+            _ptr(y) - lead_y,
+            SEG_NONE if bias is None else _ptr(bias) - lead_y,
+            SEG_NONE if res is None else _ptr(res) - lead_y,
+            start,
+            n_out,
+        )
+        start += n_out
+    return (ctypes.c_int64 * len(words))(*words), lead_w, lead_y
+
+
 def segment_table(members):
     """The reference's segment words (six int64 per member, offsets from the first member's weights and output) for
     members given as (w, y, bias, res) device tensors, bias/res None or a tensor. Returns (words, lead w, lead y)."""
     import numpy as np
 
-    lead_w, lead_y = _ptr(members[0][0]), _ptr(members[0][1])
-    words, start = [], 0
-    for w, y, bias, res in members:
-        n_out = y.shape[-1]
-        off = lambda t: SEG_NONE if t is None else _ptr(t) - lead_y
-        words += [_ptr(w) - lead_w, _ptr(y) - lead_y, off(bias), off(res), start, n_out]
-        start += n_out
-    return np.asarray(words, dtype=np.int64), lead_w, lead_y
+    words, lead_w, lead_y = _segments(members)
+    return np.array(words, dtype=np.int64), lead_w, lead_y
 
 
 def gemv_group(ty: int, members, act, rows: int, n: int, stream=None) -> None:
     """Grouped product of members (w, y, bias, res) sharing the quantized activations act (kf_hip_gemv_group)."""
-    words, lw, ly = segment_table(members)
-    check(lib().kf_hip_gemv_group(ty, lw, row_bytes(ty, n), _ptr(act), ly, rows, n, words.ctypes.data, len(members), _stream(stream)))
+    words, lw, ly = _segments(members)
+    check(lib().kf_hip_gemv_group(ty, lw, row_bytes(ty, n), _ptr(act), ly, rows, n, words, len(members), _stream(stream)))
 
 
 def matmul_group(ty: int, members, x, act, stream=None) -> None:
     """Grouped Op::MatMul of members (w, y, bias, res) on one f32 input x [rows][n] (kf_hip_matmul_group)."""
     rows, n = x.shape
-    words, lw, ly = segment_table(members)
-    check(lib().kf_hip_matmul_group(ty, lw, n, _ptr(x), rows, _ptr(act), ly, words.ctypes.data, len(members), _stream(stream)))
+    words, lw, ly = _segments(members)
+    check(lib().kf_hip_matmul_group(ty, lw, n, _ptr(x), rows, _ptr(act), ly, words, len(members), _stream(stream)))
 
 
 def block_ints(ty: int, w, act, out, rows: int, n: int, n_out: int, stream=None) -> None:
