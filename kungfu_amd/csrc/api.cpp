@@ -332,11 +332,17 @@ static double kq_few_rows_us(uint32_t ty, const void* w, int rows, int n_in, int
     return 5.5 + (rows + 15) / 16 * mb * (ty == KF_TYPE_Q4_K ? 0.22 : ty == KF_TYPE_Q5_K ? 0.20 : 0.32);
 }
 
+// Up to here the products of a decoded batch keep the few-row kernels' order of the f32 sums, one for every row count: layers
+// chained through int8 turn another order's last bits into differences of 2e-3 to 4e-3 after three of them (3840 -> 11008 at 12
+// rows, 10240 at 26), though either order is equally far from the exact result. It costs the q6_K rows of an odd number of
+// super-blocks most (6400 -> 2304 at 16 rows: 53 us against 18).
+constexpr int KF_FEW_ROWS = 32;
+
 // Whether the tile GEMM beats the few-row product (KF_KQ_GEMM=0 / 1 forces the choice, a comparison knob)
 static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes) {
     if (rows < 2 || !kf_gemm_kq_ok(ty, w, row_bytes, n_in, n_out)) return false;
     if (kf_knob_on(KF_KNOB_KQ_GEMM)) return kf_knob(KF_KNOB_KQ_GEMM) != 0;
-    return kf_gemm_kq_below(ty, rows, n_out, n_in, kq_few_rows_us(ty, w, rows, n_in, n_out, row_bytes));
+    return rows > KF_FEW_ROWS && kf_gemm_kq_below(ty, rows, n_out, n_in, kq_few_rows_us(ty, w, rows, n_in, n_out, row_bytes));
 }
 
 // The older q8_0 products' cost (MI355X, us; fitted over 4-2048 rows at the shapes of gemm_q8.hip's model). kf_hip_gemv's
@@ -354,12 +360,13 @@ static double q8_old_us(int rows, int n_in, int n_out, int64_t row_bytes, bool m
 }
 
 // Whether the q8_0 tile GEMM of any width (gemm_q8.hip) beats the product the entry point took before it (multi:
-// kf_hip_gemm_i8's). kf_hip_gemv keeps its one-pass product up to eight rows. The knobs that force an older kernel keep
-// forcing it; KF_Q8_V = 0-2 forces this one, 3 the older ones (a comparison knob)
+// kf_hip_gemm_i8's). Rows of whole 256-column steps keep the older products up to KF_FEW_ROWS, others kf_hip_gemv's one-pass
+// product up to eight rows. The knobs that force an older kernel keep forcing it; KF_Q8_V = 0-2 forces this one, 3 the older
+// ones (a comparison knob)
 static bool q8_gemm_pays(int rows, int n_in, int n_out, int64_t row_bytes, bool multi) {
     if (rows < 2) return false;
     if (kf_knob_on(KF_KNOB_Q8_V)) return kf_knob(KF_KNOB_Q8_V) < 3;
-    if (!multi && rows <= 8) return false;
+    if (rows <= (n_in % 256 == 0 ? KF_FEW_ROWS : multi ? 1 : 8)) return false;
     for (KfKnob k : {KF_KNOB_GEMM_TILE, KF_KNOB_GEMM_SLICE, KF_KNOB_GEMM_SK, KF_KNOB_GEMM_SK_S, KF_KNOB_GEMM_SK_V, KF_KNOB_GEMM_NO_MR, KF_KNOB_GEMM_MR,
                      KF_KNOB_GEMM_SMALL_W, KF_KNOB_GEMM_SMALL_TN})
         if (kf_knob_on(k)) return false;
