@@ -15,6 +15,7 @@
 #include "kf_blocks.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -111,6 +112,88 @@ __global__ void __launch_bounds__(GK_THREADS) gemv_k_kernel(const uint8_t* __res
     }
 }
 
+// One activation row of up to 16 super-blocks on 16-byte aligned weight rows, several of these to a wave. The same lanes and
+// sums as the kernel above, two rows in flight a wave. What bounded that one is the order of its loads: the activations are
+// asked for after the next row's weights, and bias and residual at its end, and as loads complete in order each row then
+// waited for the next one's weights. Here the activations stay in registers and a row's bias and residual come with its
+// weights. Past the wave's last row the loads read an empty buffer (no traffic), so every pass issues the same loads and the
+// compiler's waits are exact.
+// Measured (MI355X, us, before -> now): q6_K 4096 -> 128256 102.5 -> 88.3, 4096 -> 28672 27.5 -> 24.1; q5_K 85.8 -> 63.6 and
+// 21.1 -> 17.5. It takes three rows a wave and more: at two it is level (q6_K 4096 -> 8192 9.7, both), at one slower (4096 ->
+// 4096 6.1 -> 6.6: the second request and the registers give nothing), and rows of half a pass lose (q6_K 2048 -> 16384 11.9 ->
+// 13.9).
+template <uint32_t TY>
+__global__ void __launch_bounds__(GK_THREADS) gemv_k1_kernel(const uint8_t* __restrict__ w, int64_t row_bytes, const int8_t* __restrict__ xq,
+                                                             const int32_t* __restrict__ xs, const float* __restrict__ xd16,
+                                                             const float* __restrict__ bias, const float* __restrict__ res, float* __restrict__ y,
+                                                             int n, int n_out) {
+    constexpr bool Q6 = TY == KF_TYPE_Q6_K;
+    constexpr int BYTES = Q6 ? KF_Q6_K_BYTES : KF_Q5_K_BYTES;
+    constexpr int D = 2;
+    using Unit = std::conditional_t<Q6, KfQ6Lane, KfQ5Lane>;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nsb = n / 256, j = lane & 3, len = nsb * BYTES;
+    __shared__ __align__(16) uint8_t park[GK_WAVES * GK_WBUF];
+    uint8_t* wbuf = park + wave * GK_WBUF;
+    const int stride = gridDim.x * GK_WAVES;
+    int row = blockIdx.x * GK_WAVES + wave;  // wave-uniform
+    if (row >= n_out) return;
+    int at[GK_PIECES];  // 16-byte pieces clamped onto the row's last 16 bytes
+#pragma unroll
+    for (int i = 0; i < GK_PIECES; i++) at[i] = min(16 * (lane + 64 * i), len - 16);
+    int zero = 0;
+    __asm__("" : "+v"(zero));  // vector loads of bias and residual: a scalar load in flight would hold up every LDS wait
+    uint4 v[D][GK_PIECES];
+    float bv[D], rv[D];
+    auto fetch = [&](int s, int rw) __attribute__((always_inline)) {
+        const bool own = rw < n_out;
+        const int o = own ? rw : row;
+        const auto r = kf_rsrc(w + (int64_t)o * row_bytes, own ? (uint64_t)len : 0);
+        bv[s] = (bias ? bias + o : xd16)[zero];
+        rv[s] = (res ? res + o : xd16)[zero];
+#pragma unroll
+        for (int i = 0; i < GK_PIECES; i++) {
+            const auto t = __builtin_amdgcn_raw_buffer_load_b128(r, at[i], 0, 2 /* nt */);
+            v[s][i] = make_uint4(t[0], t[1], t[2], t[3]);
+        }
+    };
+    const int sb = min(lane >> 2, nsb - 1);
+    const bool have = (lane >> 2) < nsb;
+    typename Unit::Act act;
+    act.load(xq + 256 * sb, xs + (Q6 ? 16 : 8) * sb, j);
+    const float dx = xd16[16 * sb];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < D; s++) fetch(s, row + s * stride);
+    for (; row < n_out; row += D * stride) {
+#pragma unroll
+        for (int s = 0; s < D; s++) {
+            const int o = row + s * stride;
+            if (s > 0 && o >= n_out) return;
+#pragma unroll
+            for (int i = 0; i < GK_PIECES; i++) *reinterpret_cast<uint4*>(wbuf + at[i]) = v[s][i];
+            const float b = bv[s], r = rv[s];
+            __builtin_amdgcn_wave_barrier();
+            fetch(s, o + D * stride);
+            Unit u;
+            u.template load<true>(wbuf + (lane >> 2) * BYTES, j);
+            float acc;
+            if constexpr (Q6) {
+                acc = fmaf(u.d * dx, (float)u.dot(act), 0.0f);
+            } else {
+                const float d = kf_h2f(u.hdr.x & 0xffffu), dmin = kf_h2f(u.hdr.x >> 16);
+                int isum, imin;
+                u.dot(act, j, isum, imin);
+                acc = fmaf(-(dmin * dx), (float)imin, fmaf(d * dx, (float)isum, 0.0f));
+            }
+            __builtin_amdgcn_wave_barrier();
+            const float vs = kf_wave_sum(have ? acc : 0.0f);
+            if (lane == 0) y[o] = vs + (bias ? b : 0.0f) + (res ? r : 0.0f);
+        }
+    }
+}
+
 int gk_cus() {
     static const int cus = [] {
         int dev = 0, v = 0;
@@ -127,6 +210,13 @@ hipError_t launch_k(const uint8_t* w, int64_t row_bytes, const int8_t* xq, const
     // a resident grid of four blocks per CU; each wave walks its rows with the next (row, pass) in flight
     const int grid = std::min((n_out + GK_WAVES - 1) / GK_WAVES, 4 * gk_cus());
     // rows of one launch: 1, 2, 4 or 8 (the kernel skips rows past `rows`)
+    if constexpr (PARK) {
+        // several rows a wave, each more than half a pass (figures at the kernel)
+        if (rows == 1 && n > 2048 && n <= 4096 && n_out >= 3 * GK_WAVES * grid) {
+            gemv_k1_kernel<TY><<<grid, GK_THREADS, 0, s>>>(w, row_bytes, xq, TY == KF_TYPE_Q6_K ? xs16 : xs32, xd16, bias, res, y, n, n_out);
+            return hipGetLastError();
+        }
+    }
     if (rows == 1)
         gemv_k_kernel<TY, 1, PARK><<<grid, GK_THREADS, 0, s>>>(w, row_bytes, xq, xs16, xs32, xd16, bias, res, y, rows, n, n_out, n_out);
     else if (rows == 2)

@@ -127,16 +127,33 @@ struct KfQ6Lane {
         d = kf_h2f(*reinterpret_cast<const uint16_t*>(blk + 208));
     }
 
-    // x: the super-block's 256 int8 activations (16-byte aligned); s16: its 16 per-16 integer sums
+    // the activations the lane multiplies by. x: the super-block's 256 int8 (16-byte aligned); s16: its 16 per-16 integer sums
+    struct Act {
+        uint4 x[4];
+        int s[4];
+        __device__ __forceinline__ void load(const int8_t* xq, const int32_t* s16, int j) {
+            const int hh = j >> 1, o = 16 * (j & 1);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                x[k] = *reinterpret_cast<const uint4*>(xq + 128 * hh + 32 * k + o);
+                s[k] = s16[8 * hh + (j & 1) + 2 * k];
+            }
+        }
+    };
+
     __device__ __forceinline__ int dot(const int8_t* x, const int32_t* s16, int j) const {
-        const int hh = j >> 1, o = 16 * (j & 1);
+        Act act;
+        act.load(x, s16, j);
+        return dot(act);
+    }
+
+    __device__ __forceinline__ int dot(const Act& act) const {
         const uint32_t m4 = 0x0f0f0f0fu, m30 = 0x30303030u;
         const uint32_t av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w}, hv[4] = {h.x, h.y, h.z, h.w};
         int isum = 0;
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            const uint4 xv = *reinterpret_cast<const uint4*>(x + 128 * hh + 32 * k + o);
-            const uint32_t xs[4] = {xv.x, xv.y, xv.z, xv.w};
+            const uint32_t xs[4] = {act.x[k].x, act.x[k].y, act.x[k].z, act.x[k].w};
             int dt = 0;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
@@ -148,7 +165,7 @@ struct KfQ6Lane {
                 dt = kf_dot4(wq, xs[e], dt);
             }
             // |dot| <= 63 * 128 * 16 and |sc| <= 128: 24-bit multiplies are exact
-            isum += __mul24(sc[k], dt - 32 * s16[8 * hh + (j & 1) + 2 * k]);
+            isum += __mul24(sc[k], dt - 32 * act.s[k]);
         }
         return isum;
     }
@@ -179,13 +196,30 @@ struct KfQ5Lane {
         }
     }
 
-    // x: the super-block's 256 int8 activations; s32: its 8 per-32 integer sums
+    // the activations the lane multiplies by. x: the super-block's 256 int8; s32: its 8 per-32 integer sums
+    struct Act {
+        uint4 x[4];
+        int s[2];
+        __device__ __forceinline__ void load(const int8_t* xq, const int32_t* s32, int j) {
+            const uint4* xl = reinterpret_cast<const uint4*>(xq + 64 * j);
+#pragma unroll
+            for (int k = 0; k < 4; k++) x[k] = xl[k];
+            s[0] = s32[2 * j];
+            s[1] = s32[2 * j + 1];
+        }
+    };
+
     __device__ __forceinline__ void dot(const int8_t* x, const int32_t* s32, int j, int& isum, int& imin) const {
+        Act act;
+        act.load(x, s32, j);
+        dot(act, j, isum, imin);
+    }
+
+    __device__ __forceinline__ void dot(const Act& act, int j, int& isum, int& imin) const {
         const uint32_t m4 = 0x0f0f0f0fu, m1 = 0x01010101u;
         const uint32_t q[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
         const uint32_t hq[8] = {ha.x, ha.y, ha.z, ha.w, hb.x, hb.y, hb.z, hb.w};
-        const uint4* xl = reinterpret_cast<const uint4*>(x + 64 * j);
-        const uint4 x0 = xl[0], x1 = xl[1], x2 = xl[2], x3 = xl[3];
+        const uint4 x0 = act.x[0], x1 = act.x[1], x2 = act.x[2], x3 = act.x[3];
         const uint32_t xlo[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
         const uint32_t xhi[8] = {x2.x, x2.y, x2.z, x2.w, x3.x, x3.y, x3.z, x3.w};
         int dlo = 0, dhi = 0;
@@ -197,6 +231,6 @@ struct KfQ5Lane {
         uint32_t sc2, m2;
         kf_q4k_scales(hdr.y, hdr.z, hdr.w, j, sc2, m2);
         isum = __mul24((int)(sc2 & 0xffu), dlo) + __mul24((int)(sc2 >> 8), dhi);
-        imin = __mul24((int)(m2 & 0xffu), s32[2 * j]) + __mul24((int)(m2 >> 8), s32[2 * j + 1]);
+        imin = __mul24((int)(m2 & 0xffu), act.s[0]) + __mul24((int)(m2 >> 8), act.s[1]);
     }
 };
