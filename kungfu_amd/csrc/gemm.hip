@@ -297,10 +297,10 @@ struct GmTail {
 };
 
 // ----------------------------------------------------------------------------------- q8_0 prefill GEMM, DMA staging
-// The product of gemm_q8_0_kernel (per group and 32 x 32 tile: the exact int32 dots I_g from v_mfma_i32_32x32x32_i8,
+// The q8_0 product (per group and 32 x 32 tile: the exact int32 dots I_g from v_mfma_i32_32x32x32_i8,
 // the outer product d_x (x) d_w of the f16 scales from one v_mfma_f32_32x32x16_f16 with a single non-zero k slot,
 // then a convert and an FMA per output) with all staging done by buffer_load ... lds DMA over buffer resources (per-lane
-// offsets fixed for the K loop, a stage adding a scalar offset), as in the q4_K GEMM:
+// offsets fixed for the K loop, a stage adding a scalar offset), as in the K types' GEMM:
 //   * activations: [group][32-row tile] 1 KB blocks in MFMA order, one DMA instruction each;
 //   * weights: a stage's four q8_0 blocks of a row are 136 bytes at row offset 136 st, 8-byte aligned; each row's
 //     16-byte aligned 144-byte window around them is copied whole ([row][144] in LDS: nine 16-byte pieces, the
@@ -312,7 +312,7 @@ struct GmTail {
 // double buffer never overlapped. The waits are explicit instead: each stage ends with vmcnt(0) and a barrier, after
 // which the other buffer's DMA (issued at the stage's start) has landed. Eight waves, each a 64 x 32 tile;
 // blocks in XCD order. Wave tiles of 2 x 2 measured slower (their 128 x 256 block halves the blocks per CU).
-// gemm_q8_0_kernel (register staging) remains for K % 256 != 0.
+// Other widths run gemm_q8.hip.
 template <int WM, int WN, int TM, int TN>
 struct GqCfg {
     static constexpr int W = WM * WN, THREADS = 64 * W;
