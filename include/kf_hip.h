@@ -166,14 +166,18 @@ int kf_hip_matmul_noalloc(uint32_t ty, const void* w, int n_in, int n_out, const
 /* KF_NOALLOC_SCRATCH_BYTES of the loaded library. No reference counterpart. */
 size_t kf_hip_noalloc_scratch_bytes(void);
 
-/* The split-K products and the tile GEMMs' tail splits keep partial tiles and tickets in a static per-GPU array of
- * three slots. Two are stream slots: one goes to each (device, stream) on its first such product and stays with it;
- * launches on one stream are ordered, so a stream's products never share their slot with a running product. A stream
- * that finds both stream slots held by other streams runs the scratch-free forms (same results within the bar). The
- * third is the graph slot: every product recorded under HIP graph capture on that GPU uses it, and direct launches
- * never do, so a replay (on any stream) never shares tickets or partials with a direct product. Rule: two replays of
- * graphs that hold such products must not run at the same time on one GPU (serialise them on one stream, or with
- * events); knob KF_CAPTURE_NO_SPLIT records the scratch-free forms instead. This call waits for `stream`'s work and
+/* Products that split K over blocks (the few-row q8_0 split-K product, the tile GEMMs where their tiles leave CUs idle,
+ * the grouped GEMM) keep partial tiles and tickets in a static per-GPU array of three 68 MiB slots. Two are stream
+ * slots: one goes to each (device, stream) on its first such product and stays with it; launches on one stream are
+ * ordered, so a stream's products never share their slot with a running product. A stream that finds both stream slots
+ * held by other streams runs the scratch-free forms (same results within the bar). The third is the graph slot, which
+ * direct launches never use, so a replay (on any stream) never shares tickets or partials with a direct product. It
+ * takes the products of several rows that kf_hip_matmul, kf_hip_gemm_i8 and the MoE entry points record under HIP graph
+ * capture, on weight rows of whole 16-byte pieces (q8_0: a multiple of 256 columns, q6_K: of 2048). Where branches of
+ * one capture run side by side, the branch that records first has it and the others run without scratch until the
+ * branches join. Rule: two replays of graphs that hold such products must not run at the same time on one GPU
+ * (serialise them on one stream, or with events); knob KF_CAPTURE_NO_SPLIT records the scratch-free forms instead.
+ * kf_hip_gemv and products on other widths use no scratch under capture, and no rule holds for them. This call waits for `stream`'s work and
  * returns its stream slot for other streams (a no-op if it holds none); call it before destroying a stream that ran
  * products. No reference counterpart. */
 int kf_hip_release_stream(void* stream);

@@ -47,8 +47,12 @@ int kf_gemm_k_multiple();
 
 bool kf_gemm_q8_below(int M, int N, int K, double us);
 hipError_t kf_launch_gemm_q8(const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y, int M, int N, int K,
-                             hipStream_t s);
+                             hipStream_t s, bool graph);
 static bool q8_gemm_pays(int rows, int n_in, int n_out, int64_t row_bytes, bool multi);
+// Whether kf_hip_matmul and kf_hip_gemm_i8 may use the split scratch's graph slot under capture: on rows of whole 16-byte
+// pieces only. On others (q8_0 widths that are no multiple of 256, q6_K ones that are none of 2048), and in kf_hip_gemv, every
+// captured product runs without scratch, so graphs that hold only these may be replayed at the same time.
+static bool graph_split(int64_t row_bytes) { return row_bytes % 16 == 0; }
 
 bool kf_gemm_kq_ok(uint32_t ty, const void* w, int64_t row_bytes, int K, int N);
 bool kf_gemm_kq_below(uint32_t ty, int M, int N, int K, double us);
@@ -56,7 +60,7 @@ hipError_t kf_launch_gemm_kq_moe(const void* w, const void* w2, int64_t expert_b
                                  int n_slots, const int32_t* offsets, const int32_t* out_rows, float* y, int N, int K, hipStream_t s);
 static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes);
 hipError_t kf_launch_gemm_kq(uint32_t ty, const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y,
-                             int M, int N, int K, hipStream_t s);
+                             int M, int N, int K, hipStream_t s, bool graph);
 int kf_rows_max_n(uint32_t ty);
 hipError_t kf_launch_rows(uint32_t ty, const void* w, const void* w2, int64_t expert_bytes, int64_t row_bytes, const void* act, int act_rows,
                           int n, int n_out, const int32_t* order, const int32_t* offsets, int n_slots, int pairs, int n_used, int per_slot,
@@ -211,18 +215,20 @@ int kf_hip_gated_act_q8(const float* gate, const float* up, int rows, int n, int
     return e == hipSuccess ? KF_OK : hip_fail(e, "gated_act_q8 launch");
 }
 
-int kf_hip_gemv(uint32_t ty, const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y, int rows,
-                int n, int n_out, void* stream) {
+// kf_hip_gemv, and the products kf_hip_matmul leaves to it. `graph`: under graph capture the product may use the graph slot
+// of the split scratch
+static int gemv_product(uint32_t ty, const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y, int rows,
+                        int n, int n_out, void* stream, bool graph) {
     const int rc = check_product(ty, w, row_bytes, act, y, rows, n, n_out);
     if (rc != KF_OK) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (ty == KF_TYPE_Q8_0 && n_out > 0 && q8_gemm_pays(rows, n, n_out, row_bytes, false)) {
-        const hipError_t e = kf_launch_gemm_q8(w, row_bytes, act, bias, res, y, rows, n_out, n, s);
+        const hipError_t e = kf_launch_gemm_q8(w, row_bytes, act, bias, res, y, rows, n_out, n, s, graph);
         return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
     }
     // the K types: the tile GEMM where its cost is below the few-row product's
     if (ty != KF_TYPE_Q8_0 && n_out > 0 && kq_gemm_pays(ty, w, rows, n, n_out, row_bytes)) {
-        const hipError_t e = kf_launch_gemm_kq(ty, w, row_bytes, act, bias, res, y, rows, n_out, n, s);
+        const hipError_t e = kf_launch_gemm_kq(ty, w, row_bytes, act, bias, res, y, rows, n_out, n, s, graph);
         return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
     }
     // q5_K / q6_K: several rows on the matrix cores (16 activation rows a weight pass), one row (or a layout the
@@ -257,6 +263,11 @@ int kf_hip_gemv(uint32_t ty, const void* w, int64_t row_bytes, const void* act, 
     return KF_OK;
 }
 
+int kf_hip_gemv(uint32_t ty, const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y, int rows,
+                int n, int n_out, void* stream) {
+    return gemv_product(ty, w, row_bytes, act, bias, res, y, rows, n, n_out, stream, false);
+}
+
 int kf_hip_gemm_i8(uint32_t ty, const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y,
                    int rows, int n, int n_out, void* stream) {
     const int rc = check_product(ty, w, row_bytes, act, y, rows, n, n_out);
@@ -264,13 +275,13 @@ int kf_hip_gemm_i8(uint32_t ty, const void* w, int64_t row_bytes, const void* ac
     if (ty == KF_TYPE_Q4_K || ty == KF_TYPE_Q5_K || ty == KF_TYPE_Q6_K) {
         if (ty != KF_TYPE_Q4_K && (row_bytes % 16 != 0 || (int64_t)n_out * row_bytes >= (1ll << 31)))
             return fail(KF_E_UNSUPPORTED, "the q5_K/q6_K GEMM needs 16-byte aligned weights and rows (q6_K: %d columns, a multiple of 2048) and a matrix below 2 GB; kf_hip_gemv takes any", n);
-        const hipError_t e = kf_launch_gemm_kq(ty, w, row_bytes, act, bias, res, y, rows, n_out, n, static_cast<hipStream_t>(stream));
+        const hipError_t e = kf_launch_gemm_kq(ty, w, row_bytes, act, bias, res, y, rows, n_out, n, static_cast<hipStream_t>(stream), true);
         return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
     }
     if (ty != KF_TYPE_Q8_0) return fail(KF_E_UNSUPPORTED, "the int8 GEMM runs q8_0, q4_K, q5_K and q6_K weights (type %u given)", ty);
     if (n % kf_gemm_k_multiple() != 0) return fail(KF_E_INVALID, "%d columns, the GEMM needs a multiple of %d", n, kf_gemm_k_multiple());
     if (n_out > 0 && q8_gemm_pays(rows, n, n_out, row_bytes, true)) {
-        const hipError_t e = kf_launch_gemm_q8(w, row_bytes, act, bias, res, y, rows, n_out, n, static_cast<hipStream_t>(stream));
+        const hipError_t e = kf_launch_gemm_q8(w, row_bytes, act, bias, res, y, rows, n_out, n, static_cast<hipStream_t>(stream), graph_split(row_bytes));
         return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
     }
     const hipError_t e = kf_launch_gemm_q8_0(w, row_bytes, act, bias, res, y, rows, n_out, n, static_cast<hipStream_t>(stream));
@@ -385,11 +396,11 @@ int product(uint32_t ty, const void* w, int64_t rb, const void* act, const float
     // other widths of q8_0: no older product but the multi-row one, which the tile GEMM beats from a few rows on
     if (rows > 1 && ty == KF_TYPE_Q8_0 && n_out > 0 && !kf_knob_on(KF_KNOB_Q8_V) &&
         kf_gemm_q8_below(rows, n_out, n_in, q8_old_us(rows, n_in, n_out, rb, false))) {
-        const hipError_t e = kf_launch_gemm_q8(w, rb, act, bias, res, y, rows, n_out, n_in, static_cast<hipStream_t>(stream));
+        const hipError_t e = kf_launch_gemm_q8(w, rb, act, bias, res, y, rows, n_out, n_in, static_cast<hipStream_t>(stream), graph_split(rb));
         return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
     }
     // the K types: kf_hip_gemv picks the tile GEMM or the few-row product
-    return kf_hip_gemv(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream);
+    return gemv_product(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream, graph_split(rb));
 }
 
 // A grouped product's members from the reference's segment words (quant.cuh:301-305): per member the byte offsets of

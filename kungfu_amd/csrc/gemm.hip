@@ -25,6 +25,7 @@
 #include "kf_device.h"
 
 #include <algorithm>
+#include <optional>
 #include <type_traits>
 #include <cstdlib>
 
@@ -35,7 +36,7 @@
 #endif
 
 hipError_t kf_launch_gemm_q8(const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y, int M, int N, int K,
-                             hipStream_t s);
+                             hipStream_t s, bool graph);
 
 namespace {
 
@@ -957,8 +958,7 @@ __global__ void __launch_bounds__(256) gemm_q8_0_sk_kernel(const uint8_t* __rest
 }
 
 // The split-K launch: S splits of K per weight tile, about BPC blocks a CU (as many as the stages' LDS lets a CU
-// hold, at most two), as many as the scratch holds; hipErrorNotSupported when the scratch cannot be had (a stream
-// under graph capture, or every slot held by other streams)
+// hold, at most two), as many as the scratch holds; hipErrorNotSupported when the scratch cannot be had (KfSplit)
 template <int TM, int TN, int G, int NS>
 hipError_t gemm_sk_launch(const uint8_t* w, int64_t row_bytes, const int8_t* xq, const float* xd32, const float* bias, const float* res,
                           float* y, int M, int N, int K, hipStream_t s) {
@@ -974,7 +974,8 @@ hipError_t gemm_sk_launch(const uint8_t* w, int64_t row_bytes, const int8_t* xq,
     const size_t room = (KF_SPLIT_SCRATCH - (size_t)KF_SPLIT_TICKETS * 4) / ((size_t)tiles * Geo::TILE * 4);
     S = std::min<int>(S, (int)std::min<size_t>(room, 1 << 20));
     if (tiles > KF_SPLIT_TICKETS || S < 1) return hipErrorNotSupported;
-    char* scr = static_cast<char*>(kf_split_scratch(s));
+    const KfSplit split(s, true);
+    char* scr = split.get();
     if (!scr) return hipErrorNotSupported;
     const hipError_t le = kf_raise_lds(reinterpret_cast<const void*>(fn), LDS);
     if (le != hipSuccess) return le;
@@ -1001,11 +1002,13 @@ hipError_t gemm_q8_0_dma_launch(const uint8_t* w, int64_t row_bytes, const int8_
     // off, a comparison knob)
     GmTail tail{nullptr, nullptr, T};
     int blocks = T;
+    std::optional<KfSplit> split;
     const int slots = kf_cu_count() * (8 / (WM * WN)), rem = T % slots;
     const size_t part_bytes = (size_t)rem * 2 * TM * TN * 16 * C::THREADS * 4;
     if (rem > 0 && rem <= slots / 2 && K % 512 == 0 && K / GM_BK >= 4 && rem <= KF_SPLIT_TICKETS &&
         part_bytes <= KF_SPLIT_SCRATCH - (size_t)KF_SPLIT_TICKETS * 4 && !kf_knob_on(KF_KNOB_GEMM_NO_TAIL)) {
-        if (char* scr = static_cast<char*>(kf_split_scratch(s))) {
+        split.emplace(s, true);
+        if (char* scr = split->get()) {
             tail = GmTail{reinterpret_cast<float*>(scr + (size_t)KF_SPLIT_TICKETS * 4), reinterpret_cast<int*>(scr), T - rem};
             blocks = T + rem;
         }
@@ -1137,5 +1140,5 @@ hipError_t kf_launch_gemm_q8_0(const void* w, int64_t row_bytes, const void* act
         }
     }
     if (K % 256 == 0 && row_bytes % 16 == 0) return gemm_q8_0_dma_launch<2, 4, 2, 1>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, s);
-    return kf_launch_gemm_q8(w, row_bytes, act, bias, res, y, M, N, K, s);
+    return kf_launch_gemm_q8(w, row_bytes, act, bias, res, y, M, N, K, s, false);
 }

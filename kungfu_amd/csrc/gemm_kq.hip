@@ -37,6 +37,7 @@
 #include "kf_device.h"
 #include "kf_host.h"
 
+#include <optional>
 #include <type_traits>
 
 // The K loop relies on gfx950's LDS DMA and vmcnt order: build for gfx950 only.
@@ -906,9 +907,9 @@ KqPlan kq_plan(uint32_t ty, int M, int N, int K) {
 }
 
 // The scratch's range area, null when the stream has none
-KqWork kq_work(hipStream_t s, int full, int S) {
+KqWork kq_work(const KfSplit& split, int full, int S) {
     KqWork w{nullptr, nullptr, full, S};
-    if (char* scr = static_cast<char*>(kf_split_scratch(s))) {
+    if (char* scr = split.get()) {
         w.desc = reinterpret_cast<KqDesc*>(scr + (size_t)KF_SPLIT_TICKETS * 4);
         w.part = reinterpret_cast<float*>(scr + (size_t)KF_SPLIT_TICKETS * 4 + KQ_DESC_BYTES);
     }
@@ -940,16 +941,18 @@ bool kf_gemm_kq_below(uint32_t ty, int M, int N, int K, double us) {
     return p.us + (p.S > 1 ? 2.0 : 0.0) < us;  // the second launch's host work, which a short product does not hide
 }
 
-// Host launcher, validated by the caller (kf_gemm_kq_ok; Q8K-kind activations in `act`)
+// Host launcher, validated by the caller (kf_gemm_kq_ok; Q8K-kind activations in `act`); `graph`: under graph capture the
+// product may use the graph slot of the split scratch
 hipError_t kf_launch_gemm_kq(uint32_t ty, const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y,
-                             int M, int N, int K, hipStream_t s) {
+                             int M, int N, int K, hipStream_t s, bool graph) {
     const kf_act_offsets o = kf_act_layout((size_t)M, (size_t)K);
     const char* base = static_cast<const char*>(act);
     // whole rounds of the CUs, then the split tiles (KF_GEMM_NO_TAIL: a block a tile, a comparison knob); these need the scratch
     const KqPlan p = kq_plan(ty, M, N, K);
     KqWork work{nullptr, nullptr, p.T, 1};
+    std::optional<KfSplit> split;
     if (p.S > 1 && !kf_knob_on(KF_KNOB_GEMM_NO_TAIL)) {
-        const KqWork r = kq_work(s, p.full, p.S);
+        const KqWork r = kq_work(split.emplace(s, graph), p.full, p.S);
         if (r.part) work = r;
     }
     const int blocks = work.full + (p.T - work.full) * work.S;
@@ -986,7 +989,8 @@ hipError_t kf_launch_gemm_kq_moe(const void* w, const void* w2, int64_t expert_b
     // every CU takes an equal range of the tiles (without the scratch: the tiles that start in it)
     const int G = kq_max_ranges(tm, kf_cu_count());
     // KF_GEMM_NO_TAIL: without the scratch (a comparison knob)
-    const KqWork work = kf_knob_on(KF_KNOB_GEMM_NO_TAIL) ? KqWork{nullptr, nullptr, 0, G} : kq_work(s, 0, G);
+    std::optional<KfSplit> split;
+    const KqWork work = kf_knob_on(KF_KNOB_GEMM_NO_TAIL) ? KqWork{nullptr, nullptr, 0, G} : kq_work(split.emplace(s, true), 0, G);
 #define KQ_GO(TM)                                                                                                                             \
     return kq_run<KF_TYPE_Q4_K, TM, true>(G, s, static_cast<const uint8_t*>(w), row_bytes, reinterpret_cast<const int8_t*>(base + o.q),      \
                                           reinterpret_cast<const _Float16*>(base + o.xa), reinterpret_cast<const float*>(base + o.d32),      \

@@ -28,6 +28,7 @@
 #include "kf_layout.h"
 
 #include <algorithm>
+#include <optional>
 #include <type_traits>
 
 namespace {
@@ -321,17 +322,18 @@ __global__ void __launch_bounds__(Q8_THREADS) q8_reduce_kernel(Q8Work work, cons
 
 template <int TM>
 hipError_t q8_run(const uint8_t* w, int64_t row_bytes, const int8_t* xq, const float* xd, const float* bias, const float* res, float* y, int M, int N,
-                  int K, int S, hipStream_t s) {
+                  int K, int S, hipStream_t s, bool graph) {
     using G = Q8Geo<TM>;
     const auto fn = gemm_q8_kernel<TM>;
     const hipError_t e = kf_raise_lds(reinterpret_cast<const void*>(fn), G::LDS);
     if (e != hipSuccess) return e;
     const int T = ((N + Q8_BN - 1) / Q8_BN) * ((M + G::BM - 1) / G::BM), rem = T % kf_cu_count();
     Q8Work work{nullptr, T, 1};
+    std::optional<KfSplit> scratch;
     if (S > 1 && rem > 0 && !kf_knob_on(KF_KNOB_GEMM_NO_TAIL)) {
         const size_t tile = (size_t)G::R * Q8_THREADS * 4;
-        char* scr = (size_t)rem * S * tile <= KF_SPLIT_SCRATCH - (size_t)KF_SPLIT_TICKETS * 4 ? static_cast<char*>(kf_split_scratch(s)) : nullptr;
-        if (scr) work = Q8Work{reinterpret_cast<float*>(scr + (size_t)KF_SPLIT_TICKETS * 4), T - rem, S};
+        if ((size_t)rem * S * tile <= KF_SPLIT_SCRATCH - (size_t)KF_SPLIT_TICKETS * 4) scratch.emplace(s, graph);
+        if (scratch && scratch->get()) work = Q8Work{reinterpret_cast<float*>(scratch->get() + (size_t)KF_SPLIT_TICKETS * 4), T - rem, S};
     }
     const int split = T - work.full;
     fn<<<work.full + split * work.S, Q8_THREADS, G::LDS, s>>>(w, row_bytes, xq, xd, bias, res, y, M, N, K, work);
@@ -390,16 +392,17 @@ bool kf_gemm_q8_below(int M, int N, int K, double us) {
     return p.us + (p.S > 1 ? 2.0 : 0.0) < us;  // the second launch's host work, which a short product does not hide
 }
 
-// Host launcher: K a multiple of 32, Q8_0-kind activations in `act`, weights 16-byte aligned
+// Host launcher: K a multiple of 32, Q8_0-kind activations in `act`, weights 16-byte aligned; `graph`: under graph capture
+// the product may use the graph slot of the split scratch
 hipError_t kf_launch_gemm_q8(const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y, int M, int N, int K,
-                             hipStream_t s) {
+                             hipStream_t s, bool graph) {
     const kf_act_offsets o = kf_act_layout((size_t)M, (size_t)K);
     const char* base = static_cast<const char*>(act);
     const auto* xq = reinterpret_cast<const int8_t*>(base + o.q);
     const auto* xd = reinterpret_cast<const float*>(base + o.d32);
     const auto* wb = static_cast<const uint8_t*>(w);
     const Q8Plan p = q8_plan(M, N, K);
-    if (p.v == 0) return q8_run<1>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, p.S, s);
-    if (p.v == 1) return q8_run<2>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, p.S, s);
-    return q8_run<4>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, p.S, s);
+    if (p.v == 0) return q8_run<1>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, p.S, s, graph);
+    if (p.v == 1) return q8_run<2>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, p.S, s, graph);
+    return q8_run<4>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, p.S, s, graph);
 }

@@ -10,7 +10,11 @@
 #include "kf_knobs.h"
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <deque>
 #include <mutex>
+#include <set>
+#include <vector>
 
 #include "../../include/kf_hip.h"
 #include "kf_layout.h"
@@ -74,28 +78,83 @@ extern "C" int kf_hip_matmul_noalloc(uint32_t ty, const void* w, int n_in, int n
 }
 
 // ------------------------------------------------------------------------------------------------ split-K scratch
-// The split-K products' partial tiles and tickets (kf_host.h): static, so nothing is allocated and the addresses never
+// The split products' partial tiles and tickets (kf_host.h): static, so nothing is allocated and the addresses never
 // change. Each device has its own copy, found with hipGetSymbolAddress once per device. Stream slots go to (device,
 // stream) pairs on first use and come back through kf_hip_release_stream. A stream under graph capture gets the
 // graph slot instead: a captured graph keeps the address it recorded and may be replayed on any stream, so it must
 // never share a slot with direct launches, which hold stream slots only.
+// Within one capture the slot goes from product to product only along the graph's own order: the nodes recorded at the
+// end of the last product that used it have to be ancestors of the next one. Branches forked over several streams of
+// a capture run at the same time in a replay, and two products there would write over each other's partials.
 static __device__ __align__(256) uint8_t split_scratch[KF_SPLIT_SLOTS * KF_SPLIT_SCRATCH];
 
 namespace {
+// A capture that has used the graph slot: its id, the nodes its last use ended with, and whether a product of it is
+// being recorded right now
+struct GraphUse {
+    unsigned long long id;
+    bool busy;
+    std::vector<hipGraphNode_t> last;
+};
+constexpr size_t KF_GRAPH_USES = 64;  // captures remembered per device; more of them at once are not expected
+
 std::mutex g_split_mu;
 std::map<int, uint8_t*> g_split_base;                       // per device
 std::map<std::pair<int, hipStream_t>, int> g_split_slot;    // per (device, stream)
 std::map<int, unsigned> g_split_free;                       // per device: bit i set when slot i is free
-}  // namespace
+std::map<int, std::deque<GraphUse>> g_graph_uses;           // per device, the newest last
 
-void* kf_split_scratch(hipStream_t s) {
+// A stream's capture: its id and the nodes that whatever it records next will depend on
+bool capture_front(hipStream_t s, unsigned long long* id, std::vector<hipGraphNode_t>* front) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const hipGraphNode_t* deps = nullptr;
+    size_t n = 0;
+    if (hipStreamGetCaptureInfo_v2(s, &cs, id, nullptr, &deps, &n) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (cs != hipStreamCaptureStatusActive) return false;
+    front->assign(deps, deps + (deps ? n : 0));
+    return true;
+}
+
+// Whether every node of `want` is in `front` or an ancestor of it. The search goes breadth first from the front: in a
+// capture on one stream the last use lies a few nodes back.
+bool all_before(const std::vector<hipGraphNode_t>& want, const std::vector<hipGraphNode_t>& front) {
+    std::set<hipGraphNode_t> left(want.begin(), want.end()), seen(front.begin(), front.end());
+    std::deque<hipGraphNode_t> at(front.begin(), front.end());
+    std::vector<hipGraphNode_t> deps;
+    while (!left.empty() && !at.empty()) {
+        const hipGraphNode_t node = at.front();
+        at.pop_front();
+        left.erase(node);
+        size_t n = 0;
+        if (hipGraphNodeGetDependencies(node, nullptr, &n) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (n == 0) continue;
+        deps.resize(n);
+        if (hipGraphNodeGetDependencies(node, deps.data(), &n) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        for (size_t i = 0; i < n; i++)
+            if (seen.insert(deps[i]).second) at.push_back(deps[i]);
+    }
+    return left.empty();
+}
+
+// The slot for a product on `s`, null if there is none for it. `take`: the product is launched next (under capture the
+// slot is then busy until split_done).
+void* split_slot(hipStream_t s, bool graph, bool take, bool* capturing) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
-    const bool capturing = cs != hipStreamCaptureStatusNone;
-    if (capturing && kf_knob_on(KF_KNOB_CAPTURE_NO_SPLIT)) return nullptr;
+    *capturing = cs != hipStreamCaptureStatusNone;
+    if (*capturing && (!graph || kf_knob_on(KF_KNOB_CAPTURE_NO_SPLIT))) return nullptr;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) {
         (void)hipGetLastError();
@@ -112,7 +171,23 @@ void* kf_split_scratch(hipStream_t s) {
         b = g_split_base.emplace(dev, static_cast<uint8_t*>(p)).first;
         g_split_free[dev] = (1u << KF_SPLIT_STREAM_SLOTS) - 1;
     }
-    if (capturing) return b->second + (size_t)KF_SPLIT_STREAM_SLOTS * KF_SPLIT_SCRATCH;
+    if (*capturing) {
+        unsigned long long id = 0;
+        std::vector<hipGraphNode_t> front;
+        if (!capture_front(s, &id, &front)) return nullptr;
+        auto& uses = g_graph_uses[dev];
+        auto u = std::find_if(uses.begin(), uses.end(), [&](const GraphUse& x) { return x.id == id; });
+        if (u != uses.end() && (u->busy || !all_before(u->last, front))) return nullptr;
+        if (take) {
+            if (u == uses.end()) {
+                if (uses.size() == KF_GRAPH_USES) uses.pop_front();
+                uses.push_back(GraphUse{id, true, {}});
+            } else {
+                u->busy = true;
+            }
+        }
+        return b->second + (size_t)KF_SPLIT_STREAM_SLOTS * KF_SPLIT_SCRATCH;
+    }
     auto it = g_split_slot.find({dev, s});
     if (it == g_split_slot.end()) {
         unsigned& fr = g_split_free[dev];
@@ -122,6 +197,28 @@ void* kf_split_scratch(hipStream_t s) {
         it = g_split_slot.emplace(std::make_pair(dev, s), i).first;
     }
     return b->second + (size_t)it->second * KF_SPLIT_SCRATCH;
+}
+}  // namespace
+
+KfSplit::KfSplit(hipStream_t s, bool graph) : stream_(s), capturing_(false), p_(static_cast<char*>(split_slot(s, graph, true, &capturing_))) {}
+
+// Under capture: the product is recorded, its nodes are the slot's last use. Where they cannot be read the slot stays
+// busy, and the rest of this capture runs without it.
+KfSplit::~KfSplit() {
+    if (!p_ || !capturing_) return;
+    int dev = 0;
+    unsigned long long id = 0;
+    std::vector<hipGraphNode_t> front;
+    if (hipGetDevice(&dev) != hipSuccess || !capture_front(stream_, &id, &front)) {
+        (void)hipGetLastError();
+        return;
+    }
+    std::lock_guard<std::mutex> g(g_split_mu);
+    for (GraphUse& u : g_graph_uses[dev])
+        if (u.id == id) {
+            u.last = front;
+            u.busy = false;
+        }
 }
 
 extern "C" int kf_hip_release_stream(void* stream) {

@@ -167,3 +167,91 @@ def test_graph_capture_without_split(cuda, case, knobs):
     for i, yg, yd in _replays(cuda, case, g, y_graph, n=3):
         assert np.array_equal(yg, plain), f"replay {i}"
         assert np.array_equal(yd, split), f"direct call {i}"
+
+
+def _graph(fn):
+    """fn captured; a second stream is forked off and joined inside it by fn."""
+    import torch
+
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        fn()
+    return g
+
+
+def _replay_equal(cuda, g, outs, wants, n=4):
+    """n replays with eager work and synchronisation between them; every output bit-equal to its want each time."""
+    import torch
+
+    for i in range(n):
+        for y in outs:
+            y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        for k, (y, want) in enumerate(zip(outs, wants)):
+            assert np.array_equal(_bits(y), want), f"replay {i}, output {k}"
+
+
+def test_forked_branches_of_one_capture(cuda, case, knobs):
+    """Two branches of one captured graph run at the same time in a replay, so only the branch that records first uses the
+    graph slot (the split result) and the other runs without scratch, whichever stream it is on; once the branches have
+    joined, the next product uses the slot again."""
+    import torch
+
+    split, plain = _refs(cuda, case, knobs)
+    assert not np.array_equal(split, plain)
+    side = torch.cuda.Stream()
+    ys = [torch.full((ROWS, N_OUT), float("nan"), device=cuda) for _ in range(6)]
+
+    def run(side_first):
+        cur = torch.cuda.current_stream()
+        _run(cuda, case, y=ys[0])
+        side.wait_stream(cur)
+        with torch.cuda.stream(side):
+            if side_first:
+                _run(cuda, case, y=ys[1])
+        _run(cuda, case, y=ys[2])
+        _run(cuda, case, y=ys[3])
+        with torch.cuda.stream(side):
+            if not side_first:
+                _run(cuda, case, y=ys[1])
+        cur.wait_stream(side)
+        _run(cuda, case, y=ys[4])
+        _run(cuda, case, y=ys[5])
+
+    torch.cuda.synchronize()
+    for side_first in (True, False):
+        g = _graph(lambda: run(side_first))
+        on_main, on_side = (plain, split) if side_first else (split, plain)
+        _replay_equal(cuda, g, ys, [split, on_side, on_main, on_main, split, split])
+
+
+@pytest.mark.parametrize("ty,rows,n,n_out", [(kf.TYPE_Q4_K, 64, 4096, 4096), (kf.TYPE_Q6_K, 64, 6400, 1000), (kf.TYPE_Q8_0, 64, 4128, 1000)])
+def test_captured_products_without_the_graph_slot(cuda, knobs, ty, rows, n, n_out):
+    """kf_hip_gemv, and kf_hip_matmul on rows that are not whole 16-byte pieces, use no scratch under capture (so two such
+    graphs may be replayed at once): the scratch-free result, where a direct call splits K."""
+    import torch
+
+    w = _tensor(kf.quantize(ty, kf.synth_normal(105, 0.02, n_out * n).reshape(n_out, n)), cuda)
+    x = _tensor(kf.synth_normal(106, 1.0, rows * n).reshape(rows, n), cuda)
+    act = kf.alloc_act(rows, n, cuda)
+    kf.quant_act(x, act, kf.act_kind(ty))
+    knobs.setenv("KF_Q8_V" if ty == kf.TYPE_Q8_0 else "KF_KQ_GEMM", 1)  # the tile GEMM, whatever the cost model says
+    calls = [lambda y: kf.gemv(ty, w, act, y, rows, n, n_out)]
+    if ty != kf.TYPE_Q4_K:
+        calls.append(lambda y: kf.matmul(ty, w, x, act, y, n_out))
+    ys = [torch.full((rows, n_out), float("nan"), device=cuda) for _ in calls]
+    for call in calls:
+        call(ys[0])
+        torch.cuda.synchronize()
+        direct = _bits(ys[0])
+        knobs.setenv("KF_GEMM_NO_TAIL", 1)
+        call(ys[0])
+        torch.cuda.synchronize()
+        plain = _bits(ys[0])
+        knobs.delenv("KF_GEMM_NO_TAIL")
+        assert not np.array_equal(direct, plain)
+        y = torch.full((rows, n_out), float("nan"), device=cuda)
+        g = _graph(lambda: call(y))
+        _replay_equal(cuda, g, [y], [plain])
