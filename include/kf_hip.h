@@ -167,10 +167,12 @@ int kf_hip_matmul_noalloc(uint32_t ty, const void* w, int n_in, int n_out, const
 size_t kf_hip_noalloc_scratch_bytes(void);
 
 /* Products that split K over blocks (the few-row q8_0 split-K product, the tile GEMMs where their tiles leave CUs idle,
- * the grouped GEMM) keep partial tiles and tickets in a static per-GPU array of three 68 MiB slots. Two are stream
- * slots: one goes to each (device, stream) on its first such product and stays with it; launches on one stream are
- * ordered, so a stream's products never share their slot with a running product. A stream that finds both stream slots
- * held by other streams runs the scratch-free forms (same results within the bar). The third is the graph slot, which
+ * the grouped GEMM) keep partial tiles and tickets in a static per-GPU array of 272 MiB: three slots of 68 MiB and two
+ * spare ones of 34. Two are stream slots: one goes to each (device, stream) on its first such product and stays with it;
+ * launches on one stream are ordered, so a stream's products never share their slot with a running product. A stream
+ * that finds both stream slots held by other streams runs the scratch-free forms, chosen by their own cost (same results
+ * within the bar). kf_hip_gemv, and products on weight rows that are not whole 16-byte pieces, use the stream's slot if
+ * it has one and otherwise a spare slot, handed out in the same way. The third is the graph slot, which
  * direct launches never use, so a replay (on any stream) never shares tickets or partials with a direct product. It
  * takes the products of several rows that kf_hip_matmul, kf_hip_gemm_i8 and the MoE entry points record under HIP graph
  * capture, on weight rows of whole 16-byte pieces (q8_0: a multiple of 256 columns, q6_K: of 2048). Where branches of

@@ -45,20 +45,20 @@ hipError_t kf_launch_gemm_q8_0(const void* w, int64_t row_bytes, const void* act
                                int N, int K, hipStream_t s);
 int kf_gemm_k_multiple();
 
-bool kf_gemm_q8_below(int M, int N, int K, double us);
+bool kf_gemm_q8_below(int M, int N, int K, double us, hipStream_t s, bool graph);
 hipError_t kf_launch_gemm_q8(const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y, int M, int N, int K,
                              hipStream_t s, bool graph);
-static bool q8_gemm_pays(int rows, int n_in, int n_out, int64_t row_bytes, bool multi);
+static bool q8_gemm_pays(int rows, int n_in, int n_out, int64_t row_bytes, bool multi, hipStream_t s, bool graph);
 // Whether kf_hip_matmul and kf_hip_gemm_i8 may use the split scratch's graph slot under capture: on rows of whole 16-byte
 // pieces only. On others (q8_0 widths that are no multiple of 256, q6_K ones that are none of 2048), and in kf_hip_gemv, every
 // captured product runs without scratch, so graphs that hold only these may be replayed at the same time.
 static bool graph_split(int64_t row_bytes) { return row_bytes % 16 == 0; }
 
 bool kf_gemm_kq_ok(uint32_t ty, const void* w, int64_t row_bytes, int K, int N);
-bool kf_gemm_kq_below(uint32_t ty, int M, int N, int K, double us);
+bool kf_gemm_kq_below(uint32_t ty, int M, int N, int K, double us, hipStream_t s, bool graph);
 hipError_t kf_launch_gemm_kq_moe(const void* w, const void* w2, int64_t expert_bytes, int64_t row_bytes, int n_split, const void* act, int pairs,
                                  int n_slots, const int32_t* offsets, const int32_t* out_rows, float* y, int N, int K, hipStream_t s);
-static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes);
+static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes, hipStream_t s, bool graph);
 hipError_t kf_launch_gemm_kq(uint32_t ty, const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y,
                              int M, int N, int K, hipStream_t s, bool graph);
 int kf_rows_max_n(uint32_t ty);
@@ -222,12 +222,12 @@ static int gemv_product(uint32_t ty, const void* w, int64_t row_bytes, const voi
     const int rc = check_product(ty, w, row_bytes, act, y, rows, n, n_out);
     if (rc != KF_OK) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (ty == KF_TYPE_Q8_0 && n_out > 0 && q8_gemm_pays(rows, n, n_out, row_bytes, false)) {
+    if (ty == KF_TYPE_Q8_0 && n_out > 0 && q8_gemm_pays(rows, n, n_out, row_bytes, false, s, graph)) {
         const hipError_t e = kf_launch_gemm_q8(w, row_bytes, act, bias, res, y, rows, n_out, n, s, graph);
         return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
     }
     // the K types: the tile GEMM where its cost is below the few-row product's
-    if (ty != KF_TYPE_Q8_0 && n_out > 0 && kq_gemm_pays(ty, w, rows, n, n_out, row_bytes)) {
+    if (ty != KF_TYPE_Q8_0 && n_out > 0 && kq_gemm_pays(ty, w, rows, n, n_out, row_bytes, s, graph)) {
         const hipError_t e = kf_launch_gemm_kq(ty, w, row_bytes, act, bias, res, y, rows, n_out, n, s, graph);
         return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
     }
@@ -280,7 +280,7 @@ int kf_hip_gemm_i8(uint32_t ty, const void* w, int64_t row_bytes, const void* ac
     }
     if (ty != KF_TYPE_Q8_0) return fail(KF_E_UNSUPPORTED, "the int8 GEMM runs q8_0, q4_K, q5_K and q6_K weights (type %u given)", ty);
     if (n % kf_gemm_k_multiple() != 0) return fail(KF_E_INVALID, "%d columns, the GEMM needs a multiple of %d", n, kf_gemm_k_multiple());
-    if (n_out > 0 && q8_gemm_pays(rows, n, n_out, row_bytes, true)) {
+    if (n_out > 0 && q8_gemm_pays(rows, n, n_out, row_bytes, true, static_cast<hipStream_t>(stream), graph_split(row_bytes))) {
         const hipError_t e = kf_launch_gemm_q8(w, row_bytes, act, bias, res, y, rows, n_out, n, static_cast<hipStream_t>(stream), graph_split(row_bytes));
         return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
     }
@@ -350,10 +350,10 @@ static double kq_few_rows_us(uint32_t ty, const void* w, int rows, int n_in, int
 constexpr int KF_FEW_ROWS = 32;
 
 // Whether the tile GEMM beats the few-row product (KF_KQ_GEMM=0 / 1 forces the choice, a comparison knob)
-static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes) {
+static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes, hipStream_t s, bool graph) {
     if (rows < 2 || !kf_gemm_kq_ok(ty, w, row_bytes, n_in, n_out)) return false;
     if (kf_knob_on(KF_KNOB_KQ_GEMM)) return kf_knob(KF_KNOB_KQ_GEMM) != 0;
-    return rows > KF_FEW_ROWS && kf_gemm_kq_below(ty, rows, n_out, n_in, kq_few_rows_us(ty, w, rows, n_in, n_out, row_bytes));
+    return rows > KF_FEW_ROWS && kf_gemm_kq_below(ty, rows, n_out, n_in, kq_few_rows_us(ty, w, rows, n_in, n_out, row_bytes), s, graph);
 }
 
 // The older q8_0 products' cost (MI355X, us; fitted over 4-2048 rows at the shapes of gemm_q8.hip's model). kf_hip_gemv's
@@ -374,14 +374,14 @@ static double q8_old_us(int rows, int n_in, int n_out, int64_t row_bytes, bool m
 // kf_hip_gemm_i8's). Rows of whole 256-column steps keep the older products up to KF_FEW_ROWS, others kf_hip_gemv's one-pass
 // product up to eight rows. The knobs that force an older kernel keep forcing it; KF_Q8_V = 0-2 forces this one, 3 the older
 // ones (a comparison knob)
-static bool q8_gemm_pays(int rows, int n_in, int n_out, int64_t row_bytes, bool multi) {
+static bool q8_gemm_pays(int rows, int n_in, int n_out, int64_t row_bytes, bool multi, hipStream_t s, bool graph) {
     if (rows < 2) return false;
     if (kf_knob_on(KF_KNOB_Q8_V)) return kf_knob(KF_KNOB_Q8_V) < 3;
     if (rows <= (n_in % 256 == 0 ? KF_FEW_ROWS : multi ? 1 : 8)) return false;
     for (KfKnob k : {KF_KNOB_GEMM_TILE, KF_KNOB_GEMM_SLICE, KF_KNOB_GEMM_SK, KF_KNOB_GEMM_SK_S, KF_KNOB_GEMM_SK_V, KF_KNOB_GEMM_NO_MR, KF_KNOB_GEMM_MR,
                      KF_KNOB_GEMM_SMALL_W, KF_KNOB_GEMM_SMALL_TN})
         if (kf_knob_on(k)) return false;
-    return kf_gemm_q8_below(rows, n_out, n_in, q8_old_us(rows, n_in, n_out, row_bytes, multi));
+    return kf_gemm_q8_below(rows, n_out, n_in, q8_old_us(rows, n_in, n_out, row_bytes, multi), s, graph);
 }
 
 namespace {
@@ -395,7 +395,7 @@ int product(uint32_t ty, const void* w, int64_t rb, const void* act, const float
         return kf_hip_gemm_i8(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream);
     // other widths of q8_0: no older product but the multi-row one, which the tile GEMM beats from a few rows on
     if (rows > 1 && ty == KF_TYPE_Q8_0 && n_out > 0 && !kf_knob_on(KF_KNOB_Q8_V) &&
-        kf_gemm_q8_below(rows, n_out, n_in, q8_old_us(rows, n_in, n_out, rb, false))) {
+        kf_gemm_q8_below(rows, n_out, n_in, q8_old_us(rows, n_in, n_out, rb, false), static_cast<hipStream_t>(stream), graph_split(rb))) {
         const hipError_t e = kf_launch_gemm_q8(w, rb, act, bias, res, y, rows, n_out, n_in, static_cast<hipStream_t>(stream), graph_split(rb));
         return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
     }

@@ -857,7 +857,7 @@ namespace {
 constexpr size_t KQ_DESC_BYTES = 16384;
 static_assert(KF_SPLIT_SCRATCH >= KF_SPLIT_TICKETS * 4 + KQ_DESC_BYTES, "room for the descriptors");
 
-// Most blocks with a partial tile of their own (grouped: with two): one a CU, within the scratch
+// Grouped: most range blocks, each with two partial tiles: one a CU, within the scratch
 int kq_max_ranges(int tm, int cus) {
     const size_t room = (KF_SPLIT_SCRATCH - (size_t)KF_SPLIT_TICKETS * 4 - KQ_DESC_BYTES) / ((size_t)2 * tm * 16 * KQ_THREADS * 4);
     int G = kf_knob_or(KF_KNOB_KQ_G, cus);
@@ -866,23 +866,29 @@ int kq_max_ranges(int tm, int cus) {
     return G;
 }
 
+// One matrix: most partial tiles, one a CU, within the smaller of the scratch's slots
+int kq_max_parts(int tm, int cus) {
+    const size_t room = (std::min(KF_SPLIT_SCRATCH, KF_SPLIT_SPARE) - (size_t)KF_SPLIT_TICKETS * 4 - KQ_DESC_BYTES) / ((size_t)tm * 16 * KQ_THREADS * 4);
+    return (int)std::min((size_t)kf_knob_or(KF_KNOB_KQ_G, cus), room);
+}
+
 struct KqPlan {
     int tm, T, full, S;
     double us;
 };
 
-KqPlan kq_plan_tm(uint32_t ty, int tm, int M, int N, int K) {
+KqPlan kq_plan_tm(uint32_t ty, int tm, int M, int N, int K, bool split) {
     KqPlan p;
     p.tm = tm;
     const int cus = kf_cu_count(), nsb = K / 256;
     p.T = ((N + KQ_BN - 1) / KQ_BN) * ((M + 32 * tm - 1) / (32 * tm));
-    const int rem = p.T % cus, t = tm >> 1, max_g = kq_max_ranges(tm, cus);
+    const int rem = p.T % cus, t = tm >> 1, max_g = kq_max_parts(tm, cus);
     const double sb = KQ_SB_US[ty == KF_TYPE_Q4_K ? 0 : ty == KF_TYPE_Q5_K ? 1 : 2][t];
     p.full = p.T;
     p.S = 1;
     // the tiles of the last round as S blocks each, S the cheapest that fits the CUs with two super-blocks a block or more
     double tail = rem ? KQ_ROUND_US[t] + sb * nsb : 0.0;
-    for (int S = 2; rem && rem * S <= max_g && 2 * S <= nsb; S++) {
+    for (int S = 2; split && rem && rem * S <= max_g && 2 * S <= nsb; S++) {
         const double part = KQ_ROUND_US[t] + KQ_PART_US[t] * tm * rem * S / cus, us = part + sb * ((nsb + S - 1) / S);
         if (part + 2 * sb >= tail) break;
         if (us < tail) {
@@ -895,12 +901,14 @@ KqPlan kq_plan_tm(uint32_t ty, int tm, int M, int N, int K) {
     return p;
 }
 
-KqPlan kq_plan(uint32_t ty, int M, int N, int K) {
+// `split`: the tiles of the last round may be split (KF_GEMM_NO_TAIL: never, a comparison knob)
+KqPlan kq_plan(uint32_t ty, int M, int N, int K, bool split) {
+    split = split && !kf_knob_on(KF_KNOB_GEMM_NO_TAIL);
     const int forced = ty == KF_TYPE_Q4_K && kf_knob_on(KF_KNOB_Q4K_KQ) ? (kf_knob(KF_KNOB_Q4K_KQ) ? 2 : 4) : kf_knob_or(KF_KNOB_KQ_TM, 0);
-    if (forced) return kq_plan_tm(ty, forced == 1 || forced == 2 ? forced : 4, M, N, K);
-    KqPlan best = kq_plan_tm(ty, 1, M, N, K);
+    if (forced) return kq_plan_tm(ty, forced == 1 || forced == 2 ? forced : 4, M, N, K, split);
+    KqPlan best = kq_plan_tm(ty, 1, M, N, K, split);
     for (int tm = 2; tm <= 4; tm *= 2) {
-        const KqPlan p = kq_plan_tm(ty, tm, M, N, K);
+        const KqPlan p = kq_plan_tm(ty, tm, M, N, K, split);
         if (p.us < best.us) best = p;
     }
     return best;
@@ -932,13 +940,14 @@ hipError_t kq_run(int blocks, hipStream_t s, const uint8_t* w, int64_t row_bytes
 
 }  // namespace
 
-// Whether the product costs less than `us`. What no plan goes below comes first: the plan's search would cost the shortest
+// Whether the product costs less than `us` on stream `s`, with the split scratch if it can have it. What no plan goes below comes first: the plan's search would cost the shortest
 // products a noticeable part of their launch.
-bool kf_gemm_kq_below(uint32_t ty, int M, int N, int K, double us) {
+bool kf_gemm_kq_below(uint32_t ty, int M, int N, int K, double us, hipStream_t s, bool graph) {
     const double least = std::min(K / 256 * KQ_SB_US[0][0], 2.0 + 2 * KQ_SB_US[0][0]);  // unsplit, split
     if (1.8 + KQ_ROUND_US[0] + least >= us) return false;
-    const KqPlan p = kq_plan(ty, M, N, K);
-    return p.us + (p.S > 1 ? 2.0 : 0.0) < us;  // the second launch's host work, which a short product does not hide
+    const KqPlan p = kq_plan(ty, M, N, K, true);
+    if (p.us + (p.S > 1 ? 2.0 : 0.0) >= us) return false;  // the second launch's host work, which a short product does not hide
+    return p.S == 1 || KfSplit::ready(s, graph) || kq_plan(ty, M, N, K, false).us < us;
 }
 
 // Host launcher, validated by the caller (kf_gemm_kq_ok; Q8K-kind activations in `act`); `graph`: under graph capture the
@@ -947,13 +956,17 @@ hipError_t kf_launch_gemm_kq(uint32_t ty, const void* w, int64_t row_bytes, cons
                              int M, int N, int K, hipStream_t s, bool graph) {
     const kf_act_offsets o = kf_act_layout((size_t)M, (size_t)K);
     const char* base = static_cast<const char*>(act);
-    // whole rounds of the CUs, then the split tiles (KF_GEMM_NO_TAIL: a block a tile, a comparison knob); these need the scratch
-    const KqPlan p = kq_plan(ty, M, N, K);
-    KqWork work{nullptr, nullptr, p.T, 1};
+    // whole rounds of the CUs, then the split tiles; these need the scratch, without it the plan is one of whole tiles (the split
+    // plan's tile height run whole left 64 rows of 14336 -> 4096 on 16 or 32 blocks)
+    KqPlan p = kq_plan(ty, M, N, K, true);
     std::optional<KfSplit> split;
-    if (p.S > 1 && !kf_knob_on(KF_KNOB_GEMM_NO_TAIL)) {
-        const KqWork r = kq_work(split.emplace(s, graph), p.full, p.S);
-        if (r.part) work = r;
+    KqWork work{nullptr, nullptr, p.T, 1};
+    if (p.S > 1) {
+        work = kq_work(split.emplace(s, graph), p.full, p.S);
+        if (!work.part) {
+            p = kq_plan(ty, M, N, K, false);
+            work = KqWork{nullptr, nullptr, p.T, 1};
+        }
     }
     const int blocks = work.full + (p.T - work.full) * work.S;
     const auto* wb = static_cast<const uint8_t*>(w);

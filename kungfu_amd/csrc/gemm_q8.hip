@@ -322,19 +322,14 @@ __global__ void __launch_bounds__(Q8_THREADS) q8_reduce_kernel(Q8Work work, cons
 
 template <int TM>
 hipError_t q8_run(const uint8_t* w, int64_t row_bytes, const int8_t* xq, const float* xd, const float* bias, const float* res, float* y, int M, int N,
-                  int K, int S, hipStream_t s, bool graph) {
+                  int K, int S, float* part, hipStream_t s) {
     using G = Q8Geo<TM>;
     const auto fn = gemm_q8_kernel<TM>;
     const hipError_t e = kf_raise_lds(reinterpret_cast<const void*>(fn), G::LDS);
     if (e != hipSuccess) return e;
     const int T = ((N + Q8_BN - 1) / Q8_BN) * ((M + G::BM - 1) / G::BM), rem = T % kf_cu_count();
     Q8Work work{nullptr, T, 1};
-    std::optional<KfSplit> scratch;
-    if (S > 1 && rem > 0 && !kf_knob_on(KF_KNOB_GEMM_NO_TAIL)) {
-        const size_t tile = (size_t)G::R * Q8_THREADS * 4;
-        if ((size_t)rem * S * tile <= KF_SPLIT_SCRATCH - (size_t)KF_SPLIT_TICKETS * 4) scratch.emplace(s, graph);
-        if (scratch && scratch->get()) work = Q8Work{reinterpret_cast<float*>(scratch->get() + (size_t)KF_SPLIT_TICKETS * 4), T - rem, S};
-    }
+    if (part) work = Q8Work{part, T - rem, S};
     const int split = T - work.full;
     fn<<<work.full + split * work.S, Q8_THREADS, G::LDS, s>>>(w, row_bytes, xq, xd, bias, res, y, M, N, K, work);
     if (split) q8_reduce_kernel<TM><<<split * G::R, Q8_THREADS, 0, s>>>(work, bias, res, y, M, N);
@@ -344,7 +339,8 @@ hipError_t q8_run(const uint8_t* w, int64_t row_bytes, const int8_t* xq, const f
 // Cost model of a launch (MI355X, us; least squares over 4-2048 rows at 2048 -> 6144, 2080 -> 1000, 4096 -> 4096, 4160 -> 6000,
 // 4096 -> 14336 and 14336 -> 4096, rms 4-7%): a launch, a round of the CUs (a block's first loads and its stores), a
 // 128-column stage, and the partial tiles' way through memory where tiles are split. The tile height is the cheapest by it: 32
-// rows of 14336 -> 4096 took 23 / 26 / 34 us with 32 / 64 / 128-row tiles, 2048 rows 603 / 392 / 318.
+// rows of 14336 -> 4096 took 23 / 26 / 34 us with 32 / 64 / 128-row tiles, 2048 rows 603 / 392 / 318. A product without the
+// scratch plans whole tiles: a split plan's tile height run whole left 64 rows on 16 blocks.
 constexpr int Q8_BMS[3] = {32, 64, 128};
 constexpr double Q8_LAUNCH_US[3] = {3.5, 1.0, 0.0}, Q8_ROUND_US[3] = {2.0, 3.9, 5.0}, Q8_ST_US[3] = {1.37, 1.80, 2.86}, Q8_PART_US[3] = {4.9, 7.3, 8.7};
 
@@ -353,12 +349,15 @@ struct Q8Plan {
     double us;
 };
 
-Q8Plan q8_plan_v(int v, int M, int N, int K) {
+constexpr size_t Q8_PART_ROOM = std::min(KF_SPLIT_SCRATCH, KF_SPLIT_SPARE) - (size_t)KF_SPLIT_TICKETS * 4;
+
+Q8Plan q8_plan_v(int v, int M, int N, int K, bool split) {
     const int cus = kf_cu_count(), nst = (K / 32 + Q8_G - 1) / Q8_G;
     const int T = ((N + Q8_BN - 1) / Q8_BN) * ((M + Q8_BMS[v] - 1) / Q8_BMS[v]), rem = T % cus;
     Q8Plan p{v, 1, 0.0};
     double tail = rem ? Q8_ROUND_US[v] + Q8_ST_US[v] * nst : 0.0;
-    for (int S = 2; rem && rem * S <= cus && 2 * S <= nst; S++) {
+    for (int S = 2; split && rem && rem * S <= cus && 2 * S <= nst; S++) {
+        if ((size_t)rem * S * Q8_BMS[v] * Q8_BN * 4 > Q8_PART_ROOM) break;
         const double part = Q8_ROUND_US[v] + Q8_PART_US[v] * rem * S / cus, us = part + Q8_ST_US[v] * ((nst + S - 1) / S);
         if (part + 2 * Q8_ST_US[v] >= tail) break;
         if (us < tail) {
@@ -370,12 +369,14 @@ Q8Plan q8_plan_v(int v, int M, int N, int K) {
     return p;
 }
 
-Q8Plan q8_plan(int M, int N, int K) {
+// `split`: the tiles of the last round may be split (KF_GEMM_NO_TAIL: never, a comparison knob)
+Q8Plan q8_plan(int M, int N, int K, bool split) {
+    split = split && !kf_knob_on(KF_KNOB_GEMM_NO_TAIL);
     const int forced = kf_knob_or(KF_KNOB_Q8_V, -1);
-    if (forced >= 0 && forced < 3) return q8_plan_v(forced, M, N, K);
-    Q8Plan best = q8_plan_v(0, M, N, K);
+    if (forced >= 0 && forced < 3) return q8_plan_v(forced, M, N, K, split);
+    Q8Plan best = q8_plan_v(0, M, N, K, split);
     for (int v = 1; v < 3; v++) {
-        const Q8Plan p = q8_plan_v(v, M, N, K);
+        const Q8Plan p = q8_plan_v(v, M, N, K, split);
         if (p.us < best.us) best = p;
     }
     return best;
@@ -383,13 +384,14 @@ Q8Plan q8_plan(int M, int N, int K) {
 
 }  // namespace
 
-// Whether the product costs less than `us`. What no plan goes below comes first: the plan's search would cost the shortest
+// Whether the product costs less than `us` on stream `s`, with the split scratch if it can have it. What no plan goes below comes first: the plan's search would cost the shortest
 // products a noticeable part of their launch.
-bool kf_gemm_q8_below(int M, int N, int K, double us) {
+bool kf_gemm_q8_below(int M, int N, int K, double us, hipStream_t s, bool graph) {
     const double least = std::min((K / 32 + Q8_G - 1) / Q8_G * Q8_ST_US[0], 2.0 + 2 * Q8_ST_US[0]);  // unsplit, split
     if (Q8_LAUNCH_US[0] + Q8_ROUND_US[0] + least >= us) return false;
-    const Q8Plan p = q8_plan(M, N, K);
-    return p.us + (p.S > 1 ? 2.0 : 0.0) < us;  // the second launch's host work, which a short product does not hide
+    const Q8Plan p = q8_plan(M, N, K, true);
+    if (p.us + (p.S > 1 ? 2.0 : 0.0) >= us) return false;  // the second launch's host work, which a short product does not hide
+    return p.S == 1 || KfSplit::ready(s, graph) || q8_plan(M, N, K, false).us < us;
 }
 
 // Host launcher: K a multiple of 32, Q8_0-kind activations in `act`, weights 16-byte aligned; `graph`: under graph capture
@@ -401,8 +403,16 @@ hipError_t kf_launch_gemm_q8(const void* w, int64_t row_bytes, const void* act, 
     const auto* xq = reinterpret_cast<const int8_t*>(base + o.q);
     const auto* xd = reinterpret_cast<const float*>(base + o.d32);
     const auto* wb = static_cast<const uint8_t*>(w);
-    const Q8Plan p = q8_plan(M, N, K);
-    if (p.v == 0) return q8_run<1>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, p.S, s, graph);
-    if (p.v == 1) return q8_run<2>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, p.S, s, graph);
-    return q8_run<4>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, p.S, s, graph);
+    Q8Plan p = q8_plan(M, N, K, true);
+    std::optional<KfSplit> split;
+    float* part = nullptr;
+    if (p.S > 1) {
+        if (char* scr = split.emplace(s, graph).get())
+            part = reinterpret_cast<float*>(scr + (size_t)KF_SPLIT_TICKETS * 4);
+        else
+            p = q8_plan(M, N, K, false);
+    }
+    if (p.v == 0) return q8_run<1>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, p.S, part, s);
+    if (p.v == 1) return q8_run<2>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, p.S, part, s);
+    return q8_run<4>(wb, row_bytes, xq, xd, bias, res, y, M, N, K, p.S, part, s);
 }

@@ -48,14 +48,22 @@ inline int kf_cu_count() {
 constexpr size_t KF_SPLIT_SCRATCH = 68u << 20;
 constexpr int KF_SPLIT_STREAM_SLOTS = 2;
 constexpr int KF_SPLIT_SLOTS = KF_SPLIT_STREAM_SLOTS + 1;
+// Two more slots, of the size a tile GEMM of one matrix needs at most (a 128 x 256 f32 partial tile a CU), for the
+// products whose rows or entry point have no claim on the others (kf_hip_gemv; rows that are not whole 16-byte pieces): a
+// stream that runs only these takes no stream slot from one that runs the others.
+constexpr size_t KF_SPLIT_SPARE = 34u << 20;
+constexpr int KF_SPLIT_SPARES = 2;
 constexpr int KF_SPLIT_TICKETS = 1 << 16;
 
 // One product's use of the scratch on its stream, alive until its kernels are launched. get() is null (and the product
-// takes its scratch-free form) for a stream that finds every stream slot held by other streams, and under capture when
-// the product may not use the graph slot (`graph` false), when a product of a parallel branch of the same graph has it,
-// and when KF_CAPTURE_NO_SPLIT is set.
+// takes its scratch-free form) for a stream that finds every slot held by other streams, and under capture when a product
+// of a parallel branch of the same graph has the graph slot, or KF_CAPTURE_NO_SPLIT is set. `graph` false: a product
+// that takes a spare slot only (or the stream slot its stream has already), and none under capture.
 class KfSplit {
 public:
+    // Whether a product launched next on `s` would get it (a stream takes its slot here already)
+    static bool ready(hipStream_t s, bool graph);
+
     KfSplit(hipStream_t s, bool graph);
     ~KfSplit();
     KfSplit(const KfSplit&) = delete;

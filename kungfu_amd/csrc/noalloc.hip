@@ -86,7 +86,7 @@ extern "C" int kf_hip_matmul_noalloc(uint32_t ty, const void* w, int n_in, int n
 // Within one capture the slot goes from product to product only along the graph's own order: the nodes recorded at the
 // end of the last product that used it have to be ancestors of the next one. Branches forked over several streams of
 // a capture run at the same time in a replay, and two products there would write over each other's partials.
-static __device__ __align__(256) uint8_t split_scratch[KF_SPLIT_SLOTS * KF_SPLIT_SCRATCH];
+static __device__ __align__(256) uint8_t split_scratch[KF_SPLIT_SLOTS * KF_SPLIT_SCRATCH + KF_SPLIT_SPARES * KF_SPLIT_SPARE];
 
 namespace {
 // A capture that has used the graph slot: its id, the nodes its last use ended with, and whether a product of it is
@@ -100,8 +100,34 @@ constexpr size_t KF_GRAPH_USES = 64;  // captures remembered per device; more of
 
 std::mutex g_split_mu;
 std::map<int, uint8_t*> g_split_base;                       // per device
-std::map<std::pair<int, hipStream_t>, int> g_split_slot;    // per (device, stream)
-std::map<int, unsigned> g_split_free;                       // per device: bit i set when slot i is free
+
+// Slots given to (device, stream) pairs
+struct SlotPool {
+    int count;
+    std::map<std::pair<int, hipStream_t>, int> held;
+    std::map<int, unsigned> taken;  // per device: bit i set when slot i is held
+
+    // the stream's slot, a free one if it has none yet; -1: every one is held by another stream
+    int take(int dev, hipStream_t s) {
+        const auto it = held.find({dev, s});
+        if (it != held.end()) return it->second;
+        unsigned& t = taken[dev];
+        for (int i = 0; i < count; i++)
+            if (!(t & (1u << i))) {
+                t |= 1u << i;
+                held[{dev, s}] = i;
+                return i;
+            }
+        return -1;
+    }
+    void give_back(int dev, hipStream_t s) {
+        const auto it = held.find({dev, s});
+        if (it == held.end()) return;
+        taken[dev] &= ~(1u << it->second);
+        held.erase(it);
+    }
+};
+SlotPool g_stream_slots{KF_SPLIT_STREAM_SLOTS, {}, {}}, g_spare_slots{KF_SPLIT_SPARES, {}, {}};
 std::map<int, std::deque<GraphUse>> g_graph_uses;           // per device, the newest last
 
 // A stream's capture: its id and the nodes that whatever it records next will depend on
@@ -169,7 +195,6 @@ void* split_slot(hipStream_t s, bool graph, bool take, bool* capturing) {
             return nullptr;
         }
         b = g_split_base.emplace(dev, static_cast<uint8_t*>(p)).first;
-        g_split_free[dev] = (1u << KF_SPLIT_STREAM_SLOTS) - 1;
     }
     if (*capturing) {
         unsigned long long id = 0;
@@ -188,19 +213,19 @@ void* split_slot(hipStream_t s, bool graph, bool take, bool* capturing) {
         }
         return b->second + (size_t)KF_SPLIT_STREAM_SLOTS * KF_SPLIT_SCRATCH;
     }
-    auto it = g_split_slot.find({dev, s});
-    if (it == g_split_slot.end()) {
-        unsigned& fr = g_split_free[dev];
-        if (fr == 0) return nullptr;  // every slot held by another stream: the scratch-free form
-        const int i = __builtin_ctz(fr);
-        fr &= ~(1u << i);
-        it = g_split_slot.emplace(std::make_pair(dev, s), i).first;
-    }
-    return b->second + (size_t)it->second * KF_SPLIT_SCRATCH;
+    const bool main = graph || g_stream_slots.held.count({dev, s});
+    const int i = (main ? g_stream_slots : g_spare_slots).take(dev, s);
+    if (i < 0) return nullptr;  // every slot held by another stream: the scratch-free form
+    return b->second + (main ? i * KF_SPLIT_SCRATCH : KF_SPLIT_SLOTS * KF_SPLIT_SCRATCH + i * KF_SPLIT_SPARE);
 }
 }  // namespace
 
 KfSplit::KfSplit(hipStream_t s, bool graph) : stream_(s), capturing_(false), p_(static_cast<char*>(split_slot(s, graph, true, &capturing_))) {}
+
+bool KfSplit::ready(hipStream_t s, bool graph) {
+    bool capturing = false;
+    return split_slot(s, graph, false, &capturing) != nullptr;
+}
 
 // Under capture: the product is recorded, its nodes are the slot's last use. Where they cannot be read the slot stays
 // busy, and the rest of this capture runs without it.
@@ -230,15 +255,14 @@ extern "C" int kf_hip_release_stream(void* stream) {
         return KF_E_HIP;
     }
     std::lock_guard<std::mutex> g(g_split_mu);
-    auto it = g_split_slot.find({dev, s});
-    if (it == g_split_slot.end()) return KF_OK;
-    // the slot is free only once the stream's products that use it have ended
+    if (!g_stream_slots.held.count({dev, s}) && !g_spare_slots.held.count({dev, s})) return KF_OK;
+    // a slot is free only once the stream's products that use it have ended
     e = hipStreamSynchronize(s);
     if (e != hipSuccess) {
         kf_set_error("hipStreamSynchronize: %s", hipGetErrorString(e));
         return KF_E_HIP;
     }
-    g_split_free[dev] |= 1u << it->second;
-    g_split_slot.erase(it);
+    g_stream_slots.give_back(dev, s);
+    g_spare_slots.give_back(dev, s);
     return KF_OK;
 }

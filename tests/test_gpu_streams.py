@@ -255,3 +255,50 @@ def test_captured_products_without_the_graph_slot(cuda, knobs, ty, rows, n, n_ou
         y = torch.full((rows, n_out), float("nan"), device=cuda)
         g = _graph(lambda: call(y))
         _replay_equal(cuda, g, [y], [plain])
+
+
+@pytest.mark.parametrize("ty", [kf.TYPE_Q4_K, kf.TYPE_Q5_K, kf.TYPE_Q6_K])
+def test_products_without_a_slot_are_planned_without_one(cuda, case, knobs, ty):
+    """64 rows of 14336 -> 4096: the tile GEMM pays only with K split. A stream that finds every slot held, and a captured
+    kf_hip_gemv, take the few-row product (its bits), as a stream with a slot takes the GEMM. The spare slots of
+    kf_hip_gemv leave the stream slots alone: a second stream still splits after two others ran kf_hip_gemv."""
+    import torch
+
+    rows, n, n_out = 64, 14336, 4096
+    w = _tensor(kf.quantize(ty, kf.synth_normal(107, 0.02, n_out * n).reshape(n_out, n)), cuda)
+    act = kf.alloc_act(rows, n, cuda)
+    kf.quant_act(_tensor(kf.synth_normal(108, 1.0, rows * n).reshape(rows, n), cuda), act, kf.ACT_Q8K)
+    ys = [torch.full((rows, n_out), float("nan"), device=cuda) for _ in range(2)]
+    torch.cuda.synchronize()
+
+    def run(stream=None, entry=kf.gemv):
+        ys[0].fill_(float("nan"))
+        torch.cuda.synchronize()
+        entry(ty, w, act, ys[0], rows, n, n_out, stream=stream)
+        torch.cuda.synchronize()
+        return _bits(ys[0])
+
+    split, plain = _refs(cuda, case, knobs)  # the default stream holds a stream slot
+    knobs.setenv("KF_KQ_GEMM", 0)
+    few = run()
+    knobs.setenv("KF_KQ_GEMM", 1)
+    gemm = run()
+    knobs.delenv("KF_KQ_GEMM")
+    assert not np.array_equal(few, gemm)
+    streams = [torch.cuda.Stream() for _ in range(5)]
+    handles = [s.cuda_stream for s in streams]
+    try:
+        assert np.array_equal(run(), gemm)
+        assert np.array_equal(run(handles[0]), gemm)  # the spare slots
+        assert np.array_equal(run(handles[1]), gemm)
+        y = _run(cuda, case, stream=handles[2])  # the other stream slot
+        torch.cuda.synchronize()
+        assert np.array_equal(_bits(y), split)
+        assert np.array_equal(run(handles[3]), few)
+        kf.release_stream(handles[1])
+        assert np.array_equal(run(handles[4]), gemm)
+        g = _graph(lambda: kf.gemv(ty, w, act, ys[1], rows, n, n_out))
+        _replay_equal(cuda, g, [ys[1]], [few])
+    finally:
+        for h in handles:
+            kf.release_stream(h)
