@@ -343,10 +343,12 @@ static double kq_few_rows_us(uint32_t ty, const void* w, int rows, int n_in, int
     return 5.5 + (rows + 15) / 16 * mb * (ty == KF_TYPE_Q4_K ? 0.22 : ty == KF_TYPE_Q5_K ? 0.20 : 0.32);
 }
 
-// Up to here the products of a decoded batch keep the few-row kernels' order of the f32 sums, one for every row count: layers
-// chained through int8 turn another order's last bits into differences of 2e-3 to 4e-3 after three of them (3840 -> 11008 at 12
-// rows, 10240 at 26), though either order is equally far from the exact result. It costs the q6_K rows of an odd number of
-// super-blocks most (6400 -> 2304 at 16 rows: 53 us against 18).
+// Up to here the K types, and q8_0 rows of whole 256-column steps, keep the few-row kernels and their order of the f32 sums
+// (from two rows on; a single row has the GEMV's). Either order is equally far from the exact result, but the outputs of a
+// decoded batch then agree with those of earlier builds: layers chained through int8 turn another order's last bits into
+// differences of 2e-3 to 4e-3 after three of them (3840 -> 11008 at 12 rows, 10240 at 26). Other q8_0 widths go by cost and
+// change the order with it, and K splits change it with the row count. The price: q4_K 4096 -> 14336 at 32 rows takes
+// 23.1 us against the GEMM's 18.9, q6_K rows of an odd number of super-blocks 53 against 18 (6400 -> 2304 at 16 rows).
 constexpr int KF_FEW_ROWS = 32;
 
 // Whether the tile GEMM beats the few-row product (KF_KQ_GEMM=0 / 1 forces the choice, a comparison knob)
@@ -371,13 +373,13 @@ static double q8_old_us(int rows, int n_in, int n_out, int64_t row_bytes, bool m
 }
 
 // Whether the q8_0 tile GEMM of any width (gemm_q8.hip) beats the product the entry point took before it (multi:
-// kf_hip_gemm_i8's). Rows of whole 256-column steps keep the older products up to KF_FEW_ROWS, others kf_hip_gemv's one-pass
-// product up to eight rows. The knobs that force an older kernel keep forcing it; KF_Q8_V = 0-2 forces this one, 3 the older
-// ones (a comparison knob)
+// kf_hip_gemm_i8's). Rows of whole 256-column steps keep the older products up to KF_FEW_ROWS; on other widths the cost
+// decides from two rows on (4032 -> 39435 at 3 rows: 54.6 us against the multi-row product's 62.7). The knobs that force an
+// older kernel keep forcing it; KF_Q8_V = 0-2 forces this one, 3 the older ones (a comparison knob)
 static bool q8_gemm_pays(int rows, int n_in, int n_out, int64_t row_bytes, bool multi, hipStream_t s, bool graph) {
     if (rows < 2) return false;
     if (kf_knob_on(KF_KNOB_Q8_V)) return kf_knob(KF_KNOB_Q8_V) < 3;
-    if (rows <= (n_in % 256 == 0 ? KF_FEW_ROWS : multi ? 1 : 8)) return false;
+    if (n_in % 256 == 0 && rows <= KF_FEW_ROWS) return false;
     for (KfKnob k : {KF_KNOB_GEMM_TILE, KF_KNOB_GEMM_SLICE, KF_KNOB_GEMM_SK, KF_KNOB_GEMM_SK_S, KF_KNOB_GEMM_SK_V, KF_KNOB_GEMM_NO_MR, KF_KNOB_GEMM_MR,
                      KF_KNOB_GEMM_SMALL_W, KF_KNOB_GEMM_SMALL_TN})
         if (kf_knob_on(k)) return false;
@@ -393,13 +395,7 @@ int product(uint32_t ty, const void* w, int64_t rb, const void* act, const float
     // several q8_0 rows are the int8 GEMM, which reads each weight byte once per 128 rows
     if (rows > 1 && ty == KF_TYPE_Q8_0 && n_in % kf_gemm_k_multiple() == 0 && n_out > 0)
         return kf_hip_gemm_i8(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream);
-    // other widths of q8_0: no older product but the multi-row one, which the tile GEMM beats from a few rows on
-    if (rows > 1 && ty == KF_TYPE_Q8_0 && n_out > 0 && !kf_knob_on(KF_KNOB_Q8_V) &&
-        kf_gemm_q8_below(rows, n_out, n_in, q8_old_us(rows, n_in, n_out, rb, false), static_cast<hipStream_t>(stream), graph_split(rb))) {
-        const hipError_t e = kf_launch_gemm_q8(w, rb, act, bias, res, y, rows, n_out, n_in, static_cast<hipStream_t>(stream), graph_split(rb));
-        return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
-    }
-    // the K types: kf_hip_gemv picks the tile GEMM or the few-row product
+    // other widths of q8_0, and the K types: the tile GEMM or the few-row product, by the one rule of kf_hip_gemv
     return gemv_product(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream, graph_split(rb));
 }
 

@@ -94,3 +94,23 @@ def test_infinite_activation_scale(cuda, knobs):
     finite = np.arange(rows) != 7
     assert np.isfinite(outs[0][finite]).all() and not np.isfinite(outs[0][7]).any()
     assert np.array_equal(np.isfinite(outs[0]), np.isfinite(outs[1]))
+
+
+@pytest.mark.parametrize("rows,n,n_out", [(2, 4064, 14000), (3, 4032, 9000), (5, 1056, 300), (8, 2336, 3001), (9, 2336, 726)])
+def test_matmul_and_gemv_take_the_same_product(cuda, rows, n, n_out):
+    """A few rows of a width that only kf_hip_gemv's rule covers: kf_hip_matmul, kf_hip_gemv and both group forms run the same
+    kernel, bit for bit."""
+    import torch
+
+    w = _t(_blocks(n_out, n, rows + n), cuda)
+    x = _t(kf.synth_normal(rows, 1.0, rows * n).reshape(rows, n), cuda)
+    act = kf.alloc_act(rows, n, cuda)
+    ys = [torch.full((rows, n_out), float("nan"), device=cuda) for _ in range(4)]
+    kf.matmul(TY, w, x, act, ys[0], n_out)
+    kf.matmul_group(TY, [(w, ys[1], None, None)], x, act)
+    kf.gemv(TY, w, act, ys[2], rows, n, n_out)
+    kf.gemv_group(TY, [(w, ys[3], None, None)], act, rows, n)
+    torch.cuda.synchronize()
+    bits = [y.cpu().numpy().view(np.uint32) for y in ys]
+    for b in bits[1:]:
+        assert np.array_equal(bits[0], b)
