@@ -221,6 +221,9 @@ static int gemv_product(uint32_t ty, const void* w, int64_t row_bytes, const voi
                         int n, int n_out, void* stream, bool graph) {
     const int rc = check_product(ty, w, row_bytes, act, y, rows, n, n_out);
     if (rc != KF_OK) return rc;
+    // one limit for every row count, whichever product these rows would take
+    if ((ty == KF_TYPE_Q8_0 || ty == KF_TYPE_Q4_K) && n > kf_gemv_max_n())
+        return fail(KF_E_UNSUPPORTED, "%d columns above the %d the GEMV stages in LDS", n, kf_gemv_max_n());
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (ty == KF_TYPE_Q8_0 && n_out > 0 && q8_gemm_pays(rows, n, n_out, row_bytes, false, s, graph)) {
         const hipError_t e = kf_launch_gemm_q8(w, row_bytes, act, bias, res, y, rows, n_out, n, s, graph);
@@ -244,7 +247,6 @@ static int gemv_product(uint32_t ty, const void* w, int64_t row_bytes, const voi
         const hipError_t e = kf_launch_gemv_k(ty, w, row_bytes, act, bias, res, y, rows, n, n_out, s);
         return e == hipSuccess ? KF_OK : hip_fail(e, "q5_K/q6_K product launch");
     }
-    if (n > kf_gemv_max_n()) return fail(KF_E_UNSUPPORTED, "%d columns above the %d the GEMV stages in LDS", n, kf_gemv_max_n());
     const kf_act_offsets o = kf_act_layout((size_t)rows, (size_t)n);
     const char* base = static_cast<const char*>(act);
     // several rows: each weight row streamed once against up to eight staged activation rows
@@ -394,6 +396,9 @@ int product(uint32_t ty, const void* w, int64_t rb, const void* act, const float
     // the row count picks the product, as matvec_rows / multi_kind do (exec.rs:1877-1945): one row is the GEMV;
     // several q8_0 rows are the int8 GEMM, which reads each weight byte once per 128 rows
     if (rows > 1 && ty == KF_TYPE_Q8_0 && n_in % kf_gemm_k_multiple() == 0 && n_out > 0)
+        return kf_hip_gemm_i8(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream);
+    // q4_K rows wider than kf_hip_gemv takes: the GEMM, from as many rows as it was ever the product here
+    if (rows >= 96 && ty == KF_TYPE_Q4_K && n_in > kf_gemv_max_n() && n_out > 0)
         return kf_hip_gemm_i8(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream);
     // other widths of q8_0, and the K types: the tile GEMM or the few-row product, by the one rule of kf_hip_gemv
     return gemv_product(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream, graph_split(rb));

@@ -88,3 +88,21 @@ def test_grouped_ranges(cuda, knobs, counts, tm, scratch):
         if r1 > r0:
             for at, w in ((0, wa), (half, wb)):
                 _close(got[r0:r1, at : at + half], oracle.matmul_i8(ty, w[s * half : (s + 1) * half], n, half, x[r0:r1], None))
+
+
+def test_matmul_past_the_gemv_width(cuda):
+    """q4_K rows wider than kf_hip_gemv takes: kf_hip_matmul runs them from 96 rows on, as the GEMM."""
+    import torch
+
+    ty, rows, n, n_out = kf.TYPE_Q4_K, 96, 33024, 40
+    w = _blocks(ty, n_out, n, 21)
+    x = kf.synth_normal(22, 0.5, rows * n).reshape(rows, n)
+    act = kf.alloc_act(rows, n, cuda)
+    y = torch.full((rows, n_out), float("nan"), device=cuda)
+    kf.matmul(ty, _t(w, cuda), _t(x, cuda), act, y, n_out)
+    torch.cuda.synchronize()
+    # 2^-24 for each of a row's sums of 129 super-block terms of magnitude below 16
+    err = np.abs(y.cpu().numpy().astype(np.float64) - oracle.matmul_i8(ty, w, n, n_out, x, None))
+    assert err.max() <= 2 * 129 * 2.0**-24 * 16
+    with pytest.raises(kf.KfError):
+        kf.matmul(ty, _t(w, cuda), _t(x[:95], cuda), act, y[:95], n_out)

@@ -267,3 +267,14 @@ def test_group_segment_table_is_validated_on_the_host():
     assert rc == kf.KF_E_INVALID and "200 columns" in L.kf_hip_last_error().decode()
     rc = L.kf_hip_matmul_group(2, FAKE, 256, FAKE, 1, FAKE, FAKE, np.asarray(good, np.int64).ctypes.data, 2, None)
     assert rc == kf.KF_E_UNSUPPORTED
+
+
+@pytest.mark.parametrize("ty,n", [(kf.TYPE_Q8_0, 32800), (kf.TYPE_Q8_0, 33024), (kf.TYPE_Q4_K, 33024)])
+@pytest.mark.parametrize("rows", [1, 2, 40, 95])
+def test_rows_too_wide_for_the_gemv_are_refused(ty, n, rows):
+    """kf_hip_gemv takes at most 32768 columns of q8_0 and q4_K, at any number of rows, and so does kf_hip_matmul where it has
+    no GEMM of its own for the shape (q8_0 widths that are no multiple of 128, q4_K below 96 rows). No GPU call is made."""
+    rb = kf.row_bytes(ty, n)
+    L = kf.lib()
+    assert L.kf_hip_gemv(ty, FAKE, rb, FAKE, None, None, FAKE, rows, n, 4096, None) == kf.KF_E_UNSUPPORTED
+    assert b"32768" in L.kf_hip_last_error()
