@@ -18,6 +18,9 @@
 // alignment; 176 keeps 16 rows on distinct banks) and activation scales [row][4]. Columns past the row's end read as zero
 // activations and zero scales.
 //
+// Sums: f32 over the range's groups; where that would be less exact than the products this one replaces, f32 over a few
+// stages and from there into 64-bit totals (q8_ragged and Q8_LONG).
+//
 // Measured (MI355X, one product, with the tiles, split and form the plan picks; before: the 128 x 128 kernel, the 64-row
 // small-batch kernel, or for rows that are not 16-byte aligned the multi-row product of kf_hip_gemv):
 // 14336 -> 4096 at 2048 rows 359 -> 318 us, 128 rows 64 -> 40, 64 rows 33 -> 27; 4160 -> 6000 at 64 rows 226 -> 19, 16 rows
@@ -68,9 +71,11 @@ struct Q8Geo {
 struct Q8Work {
     float* part;
     int full, S;
+    int fold;  // stages (a power of two, less one) after which the f32 sums go into the 64-bit ones
 };
 
-template <int TM>
+// FOLD: the f32 sums go into 64-bit ones after every few stages (32- and 64-row tiles: taller ones have no registers for these)
+template <int TM, bool FOLD>
 __global__ void __launch_bounds__(Q8_THREADS, 2) gemm_q8_kernel(const uint8_t* __restrict__ w, int64_t row_bytes, const int8_t* __restrict__ xq,
                                                                           const float* __restrict__ xd32, const float* __restrict__ bias,
                                                                           const float* __restrict__ res, float* __restrict__ y, int M, int N, int K,
@@ -152,6 +157,7 @@ __global__ void __launch_bounds__(Q8_THREADS, 2) gemm_q8_kernel(const uint8_t* _
     v16f acc[TM];
 #pragma unroll
     for (int i = 0; i < TM; i++) acc[i] = v16f{};
+    double tot[FOLD ? TM : 1][16] = {};
     const uint32_t a0 = kf_lds_addr(lds) + r32 * 128 + 16 * (half ^ ((r32 >> 1) & 7));
     const int wrow = wave * 32 + r32;
     const uint32_t w0 = kf_lds_addr(lds) + G::W + wrow * Q8_WROW;
@@ -257,6 +263,16 @@ __global__ void __launch_bounds__(Q8_THREADS, 2) gemm_q8_kernel(const uint8_t* _
         __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"((G::NST - 2) * G::BATCH) : "memory");
         __syncthreads();
         stage(Pc, __builtin_amdgcn_readfirstlane(st));
+        // (the last step of the stage still waits for its rescale: it goes into the next sum)
+        if constexpr (FOLD)
+            if (((st - s0 + 1) & work.fold) == 0) {
+#pragma unroll
+                for (int i = 0; i < TM; i++) {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) tot[i][r] += (double)acc[i][r];
+                    acc[i] = v16f{};
+                }
+            }
     };
     int st = s0;
     if (s0 & 1) {
@@ -272,6 +288,12 @@ __global__ void __launch_bounds__(Q8_THREADS, 2) gemm_q8_kernel(const uint8_t* _
     }
     if (st < s1) one(even{}, st);
     rescale(1, acc[TM - 1]);  // the last step's (an even number of them a stage)
+    if constexpr (FOLD) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][r] = (float)(tot[i][r] + (double)acc[i][r]);
+    }
 
     const int n = n0 + wave * 32 + r32;
     if (slot >= 0) {
@@ -295,9 +317,9 @@ __global__ void __launch_bounds__(Q8_THREADS, 2) gemm_q8_kernel(const uint8_t* _
         }
 }
 
-// Adds the S partial tiles of each split tile in K order, with bias and residual: one (register, block) slice a block, one
-// thread an output
-template <int TM>
+// Adds the S partial tiles of each split tile, eight at a time as a tree, or in 64 bits for a FOLD product (1-2.5 us more a
+// launch), with bias and residual: one (register, block) slice a block, one thread an output
+template <int TM, bool FOLD>
 __global__ void __launch_bounds__(Q8_THREADS) q8_reduce_kernel(Q8Work work, const float* __restrict__ bias, const float* __restrict__ res,
                                                                             float* __restrict__ y, int M, int N) {
     using G = Q8Geo<TM>;
@@ -308,31 +330,50 @@ __global__ void __launch_bounds__(Q8_THREADS) q8_reduce_kernel(Q8Work work, cons
     const int n = tn * Q8_BN + wave * 32 + (tid & 31);
     if (m >= M || n >= N) return;
     const float* p = work.part + ((size_t)tt * work.S * G::R + e) * Q8_THREADS + tid;
-    float v = 0.0f;
+    std::conditional_t<FOLD, double, float> v = 0.0f;
     for (int k = 0; k < work.S; k += 8) {
         float a[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) a[u] = k + u < work.S ? p[(size_t)(k + u) * G::R * Q8_THREADS] : 0.0f;
+        if constexpr (FOLD) {
 #pragma unroll
-        for (int u = 0; u < 8; u++) v += a[u];
+            for (int u = 0; u < 8; u++) v += (double)a[u];
+        } else {
+            v += ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+        }
     }
     const int64_t o = (int64_t)m * N + n;
-    y[o] = v + (bias ? bias[n] : 0.0f) + (res ? res[o] : 0.0f);
+    y[o] = (float)v + (bias ? bias[n] : 0.0f) + (res ? res[o] : 0.0f);
 }
 
-template <int TM>
+// Widths that are no whole number of 128-column steps. Before this kernel they ran the multi-row product, whose 64 lanes'
+// sums meet in a tree (7e-8 from the 64-bit result at 33-130 groups, 9e-8 at 449, against 2e-7 and 3.8e-7 for one f32 sum
+// over all of them), so here every second stage goes into the 64-bit sums (6-7e-8) and tiles without room for these are
+// left out: 2048 rows of 14368 -> 4096 take 472 us instead of 352, 300 rows 93 instead of 84, and 29 and 4.3 ms on the
+// multi-row product.
+bool q8_ragged(int K) { return K % (32 * Q8_G) != 0; }
+
+// Other widths had one f32 sum over all groups, or over half of them and less where the older kernels split K. So only
+// sums of more stages than half of 14336 columns go into 64-bit ones here, every eight stages (3% of the time at 64 rows of 4096 ->
+// 14336, 1e-7 where one sum over 14336 columns has 3.8e-7); 128-row tiles keep the one sum.
+constexpr int Q8_LONG = 56;
+
+template <int TM, bool FOLD = false>
 hipError_t q8_run(const uint8_t* w, int64_t row_bytes, const int8_t* xq, const float* xd, const float* bias, const float* res, float* y, int M, int N,
                   int K, int S, float* part, hipStream_t s) {
     using G = Q8Geo<TM>;
-    const auto fn = gemm_q8_kernel<TM>;
+    if constexpr (TM <= 2 && !FOLD)
+        if (q8_ragged(K) || (K / 32 + Q8_G - 1) / Q8_G > Q8_LONG * S) return q8_run<TM, true>(w, row_bytes, xq, xd, bias, res, y, M, N, K, S, part, s);
+    const auto fn = gemm_q8_kernel<TM, FOLD>;
     const hipError_t e = kf_raise_lds(reinterpret_cast<const void*>(fn), G::LDS);
     if (e != hipSuccess) return e;
     const int T = ((N + Q8_BN - 1) / Q8_BN) * ((M + G::BM - 1) / G::BM), rem = T % kf_cu_count();
-    Q8Work work{nullptr, T, 1};
-    if (part) work = Q8Work{part, T - rem, S};
+    const int fold = q8_ragged(K) ? 1 : 7;
+    Q8Work work{nullptr, T, 1, fold};
+    if (part) work = Q8Work{part, T - rem, S, fold};
     const int split = T - work.full;
     fn<<<work.full + split * work.S, Q8_THREADS, G::LDS, s>>>(w, row_bytes, xq, xd, bias, res, y, M, N, K, work);
-    if (split) q8_reduce_kernel<TM><<<split * G::R, Q8_THREADS, 0, s>>>(work, bias, res, y, M, N);
+    if (split) q8_reduce_kernel<TM, FOLD><<<split * G::R, Q8_THREADS, 0, s>>>(work, bias, res, y, M, N);
     return hipGetLastError();
 }
 
@@ -375,7 +416,7 @@ Q8Plan q8_plan(int M, int N, int K, bool split) {
     const int forced = kf_knob_or(KF_KNOB_Q8_V, -1);
     if (forced >= 0 && forced < 3) return q8_plan_v(forced, M, N, K, split);
     Q8Plan best = q8_plan_v(0, M, N, K, split);
-    for (int v = 1; v < 3; v++) {
+    for (int v = 1; v < (q8_ragged(K) ? 2 : 3); v++) {
         const Q8Plan p = q8_plan_v(v, M, N, K, split);
         if (p.us < best.us) best = p;
     }

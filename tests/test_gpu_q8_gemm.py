@@ -114,3 +114,41 @@ def test_matmul_and_gemv_take_the_same_product(cuda, rows, n, n_out):
     bits = [y.cpu().numpy().view(np.uint32) for y in ys]
     for b in bits[1:]:
         assert np.array_equal(bits[0], b)
+
+
+def _exact(w, act, rows, n, n_out):
+    """The product of the rows quantized in `act` with the weight bytes, in 64 bits."""
+    offs, raw = kf.act_offsets(rows, n), act.cpu().numpy()
+    xq = raw[offs[0] : offs[0] + rows * n].view(np.int8).reshape(rows, n // 32, 32).astype(np.float64)
+    xd = raw[offs[3] : offs[3] + rows * n // 32 * 4].view(np.float32).reshape(rows, n // 32, 1).astype(np.float64)
+    b = w.reshape(n_out, n // 32, 34)
+    wd = np.ascontiguousarray(b[:, :, :2]).view(np.float16).astype(np.float64)
+    wq = np.ascontiguousarray(b[:, :, 2:]).view(np.int8).astype(np.float64)
+    return (xq * xd).reshape(rows, n) @ (wq * wd).reshape(n_out, n).T
+
+
+@pytest.mark.parametrize("tail", [True, False])
+@pytest.mark.parametrize("rows,n,n_out", [(3, 4032, 2000), (33, 2080, 1000), (20, 14048, 640), (300, 14368, 512), (700, 4128, 300)])
+def test_ragged_widths_lose_no_precision(cuda, knobs, rows, n, n_out, tail):
+    """Widths that are no multiple of 128 columns, with K split and whole: no further from the 64-bit product than the
+    multi-row product, which sums over 64 lanes. Eight groups an f32 sum: the roundings of a partial sum of k of 8 equal
+    terms, k = 2..8, and of the term itself, each of rms at most 2^-24 / sqrt(3) of the partial, make sqrt(5.4) of these."""
+    import torch
+
+    w = _blocks(n_out, n, rows + n)
+    x = kf.synth_normal(rows, 1.0, rows * n).reshape(rows, n)
+    act = kf.alloc_act(rows, n, cuda)
+    kf.quant_act(_t(x, cuda), act, kf.ACT_Q8_0)
+    want = _exact(w, act, rows, n, n_out)
+    if not tail:
+        knobs.setenv("KF_GEMM_NO_TAIL", 1)
+    errs = []
+    # the product the cost picks, the 32- and 64-row tiles, the multi-row product
+    for v in (None, 0, 1, 3):
+        if v is not None:
+            knobs.setenv("KF_Q8_V", v)
+        y = torch.full((rows, n_out), float("nan"), device=cuda)
+        kf.matmul(TY, _t(w, cuda), _t(x, cuda), act, y, n_out)
+        torch.cuda.synchronize()
+        errs.append(np.linalg.norm(y.cpu().numpy() - want) / np.linalg.norm(want))
+    assert max(errs[:3]) <= errs[3] and max(errs[1:3]) <= np.sqrt(5.4) * 2.0**-24 / np.sqrt(3), errs

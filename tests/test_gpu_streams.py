@@ -278,6 +278,7 @@ def test_products_without_a_slot_are_planned_without_one(cuda, case, knobs, ty):
         torch.cuda.synchronize()
         return _bits(ys[0])
 
+    kf.release_stream(torch.cuda.current_stream().cuda_stream)  # whatever slots earlier products left it
     split, plain = _refs(cuda, case, knobs)  # the default stream holds a stream slot
     knobs.setenv("KF_KQ_GEMM", 0)
     few = run()
