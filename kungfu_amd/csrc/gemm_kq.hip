@@ -359,7 +359,13 @@ struct KqWeight {
     }
 };
 
-template <uint32_t TY, int TM, bool MOE>
+// WIDE: the outputs' sums over the super-blocks in 64 bits
+struct KqSums64 {
+    double v[16];
+    __device__ __forceinline__ double& operator[](int r) { return v[r]; }
+};
+
+template <uint32_t TY, int TM, bool MOE, bool WIDE>
 __global__ void __launch_bounds__(KQ_THREADS, 2) gemm_kq_kernel(const uint8_t* w_, int64_t row_bytes_, const int8_t* xq_, const _Float16* xa_,
                                                                  const float* xd_, const float* bias_, const float* res_, float* y_, int M_, int N_,
                                                                  int K_, KqWork work, KqMoe moe) {
@@ -518,9 +524,10 @@ __global__ void __launch_bounds__(KQ_THREADS, 2) gemm_kq_kernel(const uint8_t* w
             kq_adma16<(G::PW & 63) ? (G::PW & 63) : 1>(off(rw, sb < s1), vo, G::Q6 ? 0 : sb * G::SBB, buf + k * 1024);
     };
 
-    v16f acc[TM];
+    using Sums = std::conditional_t<WIDE, KqSums64, v16f>;
+    Sums acc[TM];
 #pragma unroll
-    for (int i = 0; i < TM; i++) acc[i] = v16f{};
+    for (int i = 0; i < TM; i++) acc[i] = Sums{};
 
     // The K loop over TLC 32-row tiles (a grouped tile with fewer rows skips the empty ones). Per super-block the tiles
     // run one after another, each as eight group steps: the step's two MFMAs, one eighth of the previous tile's rescale
@@ -569,7 +576,7 @@ __global__ void __launch_bounds__(KQ_THREADS, 2) gemm_kq_kernel(const uint8_t* w
                 for (int r = rat[g]; r < rat[g + 1]; r++) dxn[r - rat[g]] = reinterpret_cast<const float*>(rec)[i * 32 + half * 4 + 8 * (r >> 2) + (r & 3)];
             }
         };
-        auto rescale = [&](auto pc, auto gc, v16f& a, const float (&dx)[4], const uint8_t* rec, int i, float ds, float dms) __attribute__((always_inline)) {
+        auto rescale = [&](auto pc, auto gc, Sums& a, const float (&dx)[4], const uint8_t* rec, int i, float ds, float dms) __attribute__((always_inline)) {
             constexpr int p = decltype(pc)::value, g = decltype(gc)::value;
             if constexpr (g < 2) {
 #pragma unroll
@@ -583,7 +590,10 @@ __global__ void __launch_bounds__(KQ_THREADS, 2) gemm_kq_kernel(const uint8_t* w
                 for (int r = rat[g]; r < rat[g + 1]; r++) {
                     const float sf = (float)S[p][0][r];
                     const float t = G::Q6 ? ds * sf : fmaf(-dms, mins[r], ds * sf);
-                    a[r] = fmaf(t, dx[r - rat[g]], a[r]);
+                    if constexpr (WIDE)
+                        a[r] += (double)(t * dx[r - rat[g]]);
+                    else
+                        a[r] = fmaf(t, dx[r - rat[g]], a[r]);
                 }
             }
         };
@@ -767,7 +777,7 @@ __global__ void __launch_bounds__(KQ_THREADS, 2) gemm_kq_kernel(const uint8_t* w
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) pp[(i * 16 + r) * KQ_THREADS] = acc[i][r];
+            for (int r = 0; r < 16; r++) pp[(i * 16 + r) * KQ_THREADS] = (float)acc[i][r];
     } else {
         n += wave * 32 + r32;
         const float bn = bias && n < Nn ? bias[n] : 0.0f;
@@ -778,7 +788,7 @@ __global__ void __launch_bounds__(KQ_THREADS, 2) gemm_kq_kernel(const uint8_t* w
                 const int m = mb + i * 32 + (r & 3) + 8 * (r >> 2) + 4 * half;
                 if (m >= me || n >= Nn) continue;
                 const int64_t o = (int64_t)(out_rows ? out_rows[m] : m) * Nn + n;
-                y[o] = acc[i][r] + bn + (res ? res[o] : 0.0f);
+                y[o] = (float)acc[i][r] + bn + (res ? res[o] : 0.0f);
             }
     }
     }
@@ -790,7 +800,7 @@ __global__ void __launch_bounds__(KQ_THREADS, 2) gemm_kq_kernel(const uint8_t* w
     }
 }
 
-// Adds the partial tiles of the tiles that several blocks shared, in K order, with bias and residual. One thread an output;
+// Adds the partial tiles of the tiles that several blocks shared, in K order (four at a time as a tree), with bias and residual. One thread an output;
 // a block takes RED of the TM * 16 (register, 512 threads) slices of a tile, so every load and store is a run of whole
 // lines: one slice with one matrix, whose few tiles have many parts (four made 32 rows of 4096 x 4096 14.2 us, 12.7 with
 // one), four in the grouped form, where most blocks have nothing to add. A launch of its own: the last block to arrive adding them by itself took 10-40 us with 16 partial tiles, as
@@ -818,20 +828,17 @@ __global__ void __launch_bounds__(KQ_THREADS) kq_reduce_kernel(KqWork work, cons
     const int mb = d.m0 + (e0 >> 4) * 32 + 8 * ((e0 & 15) >> 2) + (e0 & 3) + 4 * ((tid >> 5) & 1);
     if (mb >= d.m_end || n >= N) return;
     const float* p = work.part + (first * R + e0) * KQ_THREADS + tid;
-    float v[RED];
-#pragma unroll
-    for (int e = 0; e < RED; e++) v[e] = p[e * KQ_THREADS];
-    p += (size_t)R * KQ_THREADS;
-    for (int k = 1; k < d.count; k += 4, p += 4 * step * R * KQ_THREADS) {
+    float v[RED] = {};
+    for (int k = 0; k < d.count; k += 4) {
         float a[4][RED];
 #pragma unroll
-        for (int u = 0; u < 4; u++)
+        for (int u = 0; u < 4; u++) {
+            const size_t at = k + u > 0 ? 1 + (k + u - 1) * step : 0;
 #pragma unroll
-            for (int e = 0; e < RED; e++) a[u][e] = k + u < d.count ? p[(u * step * R + e) * KQ_THREADS] : 0.0f;
+            for (int e = 0; e < RED; e++) a[u][e] = k + u < d.count ? p[(at * R + e) * KQ_THREADS] : 0.0f;
+        }
 #pragma unroll
-        for (int u = 0; u < 4; u++)
-#pragma unroll
-            for (int e = 0; e < RED; e++) v[e] += a[u][e];
+        for (int e = 0; e < RED; e++) v[e] += (a[0][e] + a[1][e]) + (a[2][e] + a[3][e]);
     }
     const float bn = bias ? bias[n] : 0.0f;
 #pragma unroll
@@ -872,8 +879,19 @@ int kq_max_parts(int tm, int cus) {
     return (int)std::min((size_t)kf_knob_or(KF_KNOB_KQ_G, cus), room);
 }
 
+// A block's f32 sum of more super-blocks than this is kept in 64 bits instead (WIDE), where the tile's registers have room:
+// 16 super-blocks of q4_K are 9.7e-8 from the 64-bit result with f32 sums and 7.3e-8 with these, 51 of q6_K 1.32e-7 and
+// 4.4e-8, at 10-12% (q4_K), 6% (q5_K) and 3% (q6_K) of the K loop. The few-row products and the shorter K ranges that these
+// blocks replace had 8.5-9.1e-8 and 8e-8. 128-row tiles, and 64-row ones of q5_K (four registers spilled), keep the f32
+// sum, as the tile kernels did whose whole rounds they took over; widths of q6_K that had no tile kernel before (rows
+// that are not whole 16-byte pieces) leave them out instead: 2048 rows of 13056 -> 4096 take 426 us in place of 294,
+// 6400 -> 2304 145 and 144, and 19.6 and 6.5 ms on the per-lane product.
+constexpr int KQ_LONG = 12;
+constexpr double KQ_WIDE_COST[3] = {1.12, 1.06, 1.03};  // [q4_K, q5_K, q6_K]
+
 struct KqPlan {
     int tm, T, full, S;
+    bool wide;
     double us;
 };
 
@@ -882,22 +900,31 @@ KqPlan kq_plan_tm(uint32_t ty, int tm, int M, int N, int K, bool split) {
     p.tm = tm;
     const int cus = kf_cu_count(), nsb = K / 256;
     p.T = ((N + KQ_BN - 1) / KQ_BN) * ((M + 32 * tm - 1) / (32 * tm));
-    const int rem = p.T % cus, t = tm >> 1, max_g = kq_max_parts(tm, cus);
-    const double sb = KQ_SB_US[ty == KF_TYPE_Q4_K ? 0 : ty == KF_TYPE_Q5_K ? 1 : 2][t];
+    const int rem = p.T % cus, t = tm >> 1, max_g = kq_max_parts(tm, cus), k = ty == KF_TYPE_Q4_K ? 0 : ty == KF_TYPE_Q5_K ? 1 : 2;
+    const double sb = KQ_SB_US[k][t];
+    const bool fits = tm == 1 || (tm == 2 && ty != KF_TYPE_Q5_K), ragged = ty == KF_TYPE_Q6_K && K % 2048 != 0;
+    // a block of n super-blocks, in a launch whose longest one has `most`
+    auto cost = [&](int n, int most) {
+        if (most > KQ_LONG && ragged && !fits) return 1e30;
+        return KQ_ROUND_US[t] + sb * n * (most > KQ_LONG && fits ? KQ_WIDE_COST[k] : 1.0);
+    };
+    const int rounds = p.T / cus;
     p.full = p.T;
     p.S = 1;
+    p.us = (rounds + (rem ? 1 : 0)) * cost(nsb, nsb);
     // the tiles of the last round as S blocks each, S the cheapest that fits the CUs with two super-blocks a block or more
-    double tail = rem ? KQ_ROUND_US[t] + sb * nsb : 0.0;
     for (int S = 2; split && rem && rem * S <= max_g && 2 * S <= nsb; S++) {
-        const double part = KQ_ROUND_US[t] + KQ_PART_US[t] * tm * rem * S / cus, us = part + sb * ((nsb + S - 1) / S);
-        if (part + 2 * sb >= tail) break;
-        if (us < tail) {
-            tail = us;
+        const int n = (nsb + S - 1) / S, most = rounds ? nsb : n;
+        const double part = rounds * cost(nsb, most) + KQ_PART_US[t] * tm * rem * S / cus, us = part + cost(n, most);
+        if (part + cost(2, 2) >= p.us) break;
+        if (us < p.us) {
+            p.us = us;
             p.full = p.T - rem;
             p.S = S;
         }
     }
-    p.us = 1.8 + (p.T / cus) * (KQ_ROUND_US[t] + sb * nsb) + tail;
+    p.us += 1.8;
+    p.wide = fits && (p.full > 0 ? nsb : (nsb + p.S - 1) / p.S) > KQ_LONG;
     return p;
 }
 
@@ -924,10 +951,10 @@ KqWork kq_work(const KfSplit& split, int full, int S) {
     return w;
 }
 
-template <uint32_t TY, int TM, bool MOE>
+template <uint32_t TY, int TM, bool MOE, bool WIDE>
 hipError_t kq_run(int blocks, hipStream_t s, const uint8_t* w, int64_t row_bytes, const int8_t* xq, const _Float16* xa, const float* xd,
                   const float* bias, const float* res, float* y, int M, int N, int K, KqWork work, KqMoe moe) {
-    const auto fn = gemm_kq_kernel<TY, TM, MOE>;
+    const auto fn = gemm_kq_kernel<TY, TM, MOE, WIDE>;
     constexpr int bytes = KqGeo<TY, TM>::LDS + KQ_EPI;
     const hipError_t e = kf_raise_lds(reinterpret_cast<const void*>(fn), bytes);
     if (e != hipSuccess) return e;
@@ -973,12 +1000,14 @@ hipError_t kf_launch_gemm_kq(uint32_t ty, const void* w, int64_t row_bytes, cons
     const auto* xq = reinterpret_cast<const int8_t*>(base + o.q);
     const auto* xa = reinterpret_cast<const _Float16*>(base + o.xa);
     const auto* xd = reinterpret_cast<const float*>(base + o.d32);
-#define KQ_GO(TY, TM) return kq_run<TY, TM, false>(blocks, s, wb, row_bytes, xq, xa, xd, bias, res, y, M, N, K, work, KqMoe{})
-#define KQ_TMS(TY)               \
-    {                            \
-        if (p.tm == 1) KQ_GO(TY, 1); \
-        if (p.tm == 2) KQ_GO(TY, 2); \
-        KQ_GO(TY, 4);            \
+#define KQ_GO(TY, TM, WIDE) return kq_run<TY, TM, false, WIDE>(blocks, s, wb, row_bytes, xq, xa, xd, bias, res, y, M, N, K, work, KqMoe{})
+#define KQ_TMS(TY)                                                     \
+    {                                                                  \
+        if (p.tm == 1 && p.wide) KQ_GO(TY, 1, true);                   \
+        if (p.tm == 1) KQ_GO(TY, 1, false);                            \
+        if (p.tm == 2 && p.wide) KQ_GO(TY, 2, (TY != KF_TYPE_Q5_K));   \
+        if (p.tm == 2) KQ_GO(TY, 2, false);                            \
+        KQ_GO(TY, 4, false);                                           \
     }
     if (ty == KF_TYPE_Q4_K) KQ_TMS(KF_TYPE_Q4_K)
     if (ty == KF_TYPE_Q5_K) KQ_TMS(KF_TYPE_Q5_K)
@@ -1005,7 +1034,7 @@ hipError_t kf_launch_gemm_kq_moe(const void* w, const void* w2, int64_t expert_b
     std::optional<KfSplit> split;
     const KqWork work = kf_knob_on(KF_KNOB_GEMM_NO_TAIL) ? KqWork{nullptr, nullptr, 0, G} : kq_work(split.emplace(s, true), 0, G);
 #define KQ_GO(TM)                                                                                                                             \
-    return kq_run<KF_TYPE_Q4_K, TM, true>(G, s, static_cast<const uint8_t*>(w), row_bytes, reinterpret_cast<const int8_t*>(base + o.q),      \
+    return kq_run<KF_TYPE_Q4_K, TM, true, false>(G, s, static_cast<const uint8_t*>(w), row_bytes, reinterpret_cast<const int8_t*>(base + o.q),      \
                                           reinterpret_cast<const _Float16*>(base + o.xa), reinterpret_cast<const float*>(base + o.d32),      \
                                           nullptr, nullptr, y, pairs, N, K, work, moe)
     if (tm == 1) KQ_GO(1);

@@ -106,3 +106,33 @@ def test_matmul_past_the_gemv_width(cuda):
     assert err.max() <= 2 * 129 * 2.0**-24 * 16
     with pytest.raises(kf.KfError):
         kf.matmul(ty, _t(w, cuda), _t(x[:95], cuda), act, y[:95], n_out)
+
+
+@pytest.mark.parametrize("rows,n,n_out", [(40, 6400, 600), (300, 13056, 512), (700, 6400, 2304), (2048, 6400, 300)])
+def test_ragged_q6_K_loses_no_precision(cuda, knobs, rows, n, n_out):
+    """q6_K rows of an odd number of super-blocks: no further from the 64-bit product than the per-lane product, which sums
+    over 64 lanes, by the plan and on 32- and 64-row tiles run whole. These sum in 64 bits: three roundings a super-block's
+    term (its integer, the two scales) and the last one, each of rms at most 2^-24 / sqrt(3)."""
+    import torch
+
+    ty = kf.TYPE_Q6_K
+    w = _blocks(ty, n_out, n, rows + n)
+    x = kf.synth_normal(rows, 1.0, rows * n).reshape(rows, n)
+    act = kf.alloc_act(rows, n, cuda)
+    kf.quant_act(_t(x, cuda), act, kf.ACT_Q8K)
+    offs, raw = kf.act_offsets(rows, n), act.cpu().numpy()
+    xq = raw[offs[0] : offs[0] + rows * n].view(np.int8).reshape(rows, n // 32, 32).astype(np.float64)
+    xd = raw[offs[3] : offs[3] + rows * n // 32 * 4].view(np.float32).reshape(rows, n // 32, 1).astype(np.float64)
+    # q6_K weights are exact in f32: 11 bits of d, 7 of the scale, 6 of the value
+    want = (xq * xd).reshape(rows, n) @ np.asarray(oracle.dequant(ty, w, n)).reshape(n_out, n).astype(np.float64).T
+    errs = []
+    for ks in ({"KF_KQ_GEMM": 0}, {}, {"KF_KQ_GEMM": 1, "KF_KQ_TM": 1, "KF_GEMM_NO_TAIL": 1}, {"KF_KQ_GEMM": 1, "KF_KQ_TM": 2, "KF_GEMM_NO_TAIL": 1}):
+        for k, v in ks.items():
+            knobs.setenv(k, v)
+        y = torch.full((rows, n_out), float("nan"), device=cuda)
+        kf.matmul(ty, _t(w, cuda), _t(x, cuda), act, y, n_out)
+        torch.cuda.synchronize()
+        errs.append(np.linalg.norm(y.cpu().numpy() - want) / np.linalg.norm(want))
+        for k in ks:
+            knobs.delenv(k)
+    assert max(errs[1:]) <= errs[0] and max(errs[2:]) <= 2.0**-23 / np.sqrt(3), errs
