@@ -136,3 +136,39 @@ def test_ragged_q6_K_loses_no_precision(cuda, knobs, rows, n, n_out):
         for k in ks:
             knobs.delenv(k)
     assert max(errs[1:]) <= errs[0] and max(errs[2:]) <= 2.0**-23 / np.sqrt(3), errs
+
+
+@pytest.mark.parametrize("tail", [True, False])
+@pytest.mark.parametrize("tm", [1, 2, 4])
+@pytest.mark.parametrize("ty", K_TYPES)
+def test_infinite_and_nan_block_scales(cuda, knobs, ty, tm, tail):
+    """A super-block whose scale is infinite or NaN (and, of q4_K / q5_K, its minimum's): its output column is infinite or
+    NaN as the CPU's is, and the other columns are those of the same matrix with finite scales, bit for bit."""
+    import torch
+
+    rows, n, n_out = 33, 4096, 300
+    w = _blocks(ty, n_out, n, 31).reshape(n_out, n // 256, -1)
+    bad = w.copy()
+    at = (208,) if ty == kf.TYPE_Q6_K else (0, 2)
+    for k, (row, sb, bits) in enumerate(((0, 0, 0x7C00), (31, 15, 0x7E00), (32, 7, 0xFC00), (255, 8, 0x7C00), (299, 3, 0x7E00))):
+        bad[row, sb, at[k % len(at)] : at[k % len(at)] + 2] = np.array([bits], np.uint16).view(np.uint8)
+    cols = [0, 31, 32, 255, 299]
+    x = kf.synth_normal(32, 1.0, rows * n).reshape(rows, n)
+    knobs.setenv("KF_KQ_GEMM", 1)
+    knobs.setenv("KF_KQ_TM", tm)
+    if not tail:
+        knobs.setenv("KF_GEMM_NO_TAIL", 1)
+    act = kf.alloc_act(rows, n, cuda)
+    outs = []
+    for m in (w, bad):
+        y = torch.full((rows, n_out), 0.5, device=cuda)
+        kf.matmul(ty, _t(m.reshape(n_out, -1), cuda), _t(x, cuda), act, y, n_out)
+        torch.cuda.synchronize()
+        outs.append(y.cpu().numpy())
+    rest = np.setdiff1d(np.arange(n_out), cols)
+    assert np.isfinite(outs[0]).all()
+    assert np.array_equal(outs[0][:, rest].view(np.uint32), outs[1][:, rest].view(np.uint32))
+    with np.errstate(all="ignore"):
+        want = oracle.matmul_i8(ty, np.ascontiguousarray(bad[cols]).reshape(len(cols), -1), n, len(cols), x, None)
+    # (which of the two, and an infinity's sign, follow the order of the terms; the CPU multiplies the scales out first)
+    assert not np.isfinite(want).any() and not np.isfinite(outs[1][:, cols]).any()

@@ -30,7 +30,7 @@ def _random_blocks(ty, n_out, n_in, rng):
 
 def _gauss_blocks(ty, n_out, n_in, seed):
     """Blocks from the build's encoder on N(0, 0.02) weights, the scale real checkpoints have: outputs of magnitude a
-    few units, where the f32 rounding of any summation order stays far below the north-star bar."""
+    few units, where the f32 rounding of any summation order stays far below the bar above."""
     return kf.quantize(ty, kf.synth_normal(seed, 0.02, n_out * n_in).reshape(n_out, n_in))
 
 
@@ -106,7 +106,7 @@ def test_multi_row_matrix_cores(cuda, ty, rows, n, n_out):
     waves): chunks of 16 rows past the first, ragged last tiles, 14336 columns; 2304 columns (nine super-blocks a row)
     leave q6_K rows 2-byte aligned, which the per-lane product takes instead. Encoder blocks of N(0, 0.02) weights
     (every bit pattern is covered by the block-integer test), with bias and residual, against the CPU backend's int8
-    path (ops::matmul_i8: the same quantized activations and dot_i8 integers) at the north-star bar."""
+    path (ops::matmul_i8: the same quantized activations and dot_i8 integers) at the bar above."""
     import torch
 
     rng = np.random.default_rng(rows * 31 + n + n_out + ty)
@@ -133,7 +133,7 @@ def test_gemm_tile_shapes(cuda, ty, rows, n, n_out):
     """The q5_K / q6_K prefill GEMM (64 x 256 block tiles over native super-blocks): ragged row panels and column
     tiles, one row, 14336 and 6144 columns (q6_K rows 16-byte aligned: n a multiple of 2048), encoder blocks of
     N(0, 0.02) weights, with bias and residual, against the CPU backend's int8 path (the same quantized activations and
-    dot_i8 integers) at the north-star bar. Every scale, min and bit pattern is covered by the block-integer test."""
+    dot_i8 integers) at the bar above. Every scale, min and bit pattern is covered by the block-integer test."""
     import torch
 
     rng = np.random.default_rng(rows * 7 + n + n_out + ty)
@@ -151,10 +151,10 @@ def test_gemm_tile_shapes(cuda, ty, rows, n, n_out):
 
 @pytest.mark.parametrize("ty", [kf.TYPE_Q5_K, kf.TYPE_Q6_K])
 @pytest.mark.parametrize("n,n_out", [(4096, 14336), (14336, 4096)])
-def test_gemm_prefill_shapes(cuda, ty, n, n_out):
+def test_gemm_prefill_shapes(cuda, knobs, ty, n, n_out):
     """M = 2048 at the Llama-3-8B gate and down shapes with weights from the build's encoder: every 97th row against
     the CPU backend's float product (rows are independent), and the whole output against the few-row matrix-core
-    product (kf_hip_gemv) within the same bar."""
+    product (kf_hip_gemv with KF_KQ_GEMM=0, 128 passes of 16 rows) within the same bar."""
     import torch
 
     rows = 2048
@@ -166,6 +166,7 @@ def test_gemm_prefill_shapes(cuda, ty, n, n_out):
     y = torch.full((rows, n_out), float("nan"), device=cuda)
     kf.gemm_i8(ty, wt, act, y, rows, n, n_out)
     y2 = torch.full((rows, n_out), float("nan"), device=cuda)
+    knobs.setenv("KF_KQ_GEMM", 0)
     kf.gemv(ty, wt, act, y2, rows, n, n_out)
     torch.cuda.synchronize()
     got = y.cpu().numpy()
@@ -176,9 +177,9 @@ def test_gemm_prefill_shapes(cuda, ty, n, n_out):
 
 @pytest.mark.parametrize("ty", [kf.TYPE_Q5_K, kf.TYPE_Q6_K])
 def test_gemm_shapes_it_declines(cuda, ty):
-    """2304 columns: q6_K's 210-byte super-block rows are then not 16-byte aligned, so kf_hip_gemm_i8 refuses
-    (KF_E_UNSUPPORTED) and kf_hip_matmul takes the few-row product; q5_K's 176-byte rows stay aligned and the GEMM takes
-    them. Against the CPU backend's int8 path either way."""
+    """2304 columns: q6_K's 210-byte super-block rows are then not 16-byte aligned, which kf_hip_gemm_i8 refuses by its
+    contract (KF_E_UNSUPPORTED) and kf_hip_matmul takes; q5_K's 176-byte rows stay aligned and both take them. Against the
+    CPU backend's int8 path either way."""
     import torch
 
     n, n_out, rows = 2304, 40, 128
@@ -198,9 +199,10 @@ def test_gemm_shapes_it_declines(cuda, ty):
 
 @pytest.mark.parametrize("ty", [kf.TYPE_Q5_K, kf.TYPE_Q6_K])
 @pytest.mark.parametrize("rows", [63, 97, 256])
-def test_matmul_picks_gemm_by_cost(cuda, ty, rows):
-    """kf_hip_matmul around its few-row / tile GEMM switch at the gate shape (4096 -> 14336: the cost model moves to
-    the GEMM at about 64 rows for q5_K and 32 for q6_K) gives the outputs of both products, within the bar."""
+def test_matmul_picks_gemm_by_cost(cuda, knobs, ty, rows):
+    """kf_hip_matmul past the row count up to which it keeps the few-row product, at the gate shape (4096 -> 14336, where
+    the cost model moves to the GEMM): the GEMM's outputs bit for bit, the few-row product's (KF_KQ_GEMM=0) within the
+    bar, and every 17th row of either against the CPU backend's int8 path."""
     import torch
 
     n, n_out = 4096, 14336
@@ -212,21 +214,28 @@ def test_matmul_picks_gemm_by_cost(cuda, ty, rows):
     y = torch.full((rows, n_out), float("nan"), device=cuda)
     kf.matmul(ty, wt, xt, act, y, n_out)
     y2 = torch.full((rows, n_out), float("nan"), device=cuda)
+    knobs.setenv("KF_KQ_GEMM", 0)
     kf.gemv(ty, wt, act, y2, rows, n, n_out)
+    knobs.delenv("KF_KQ_GEMM")
     y3 = torch.full((rows, n_out), float("nan"), device=cuda)
     kf.gemm_i8(ty, wt, act, y3, rows, n, n_out)
     torch.cuda.synchronize()
-    got = y.cpu().numpy()
-    _gemm_bound(got, y2.cpu().numpy())
-    _gemm_bound(got, y3.cpu().numpy())
+    got, few = y.cpu().numpy(), y2.cpu().numpy()
+    assert np.array_equal(got.view(np.uint32), y3.cpu().numpy().view(np.uint32))
+    assert not np.array_equal(got.view(np.uint32), few.view(np.uint32))
+    _gemm_bound(got, few)
+    sample = np.arange(0, rows, 17)
+    want = oracle.matmul_i8(ty, w, n, n_out, x[sample], None)
+    _gemm_bound(got[sample], want)
+    _gemm_bound(few[sample], want)
 
 
 @pytest.mark.parametrize("ty", [kf.TYPE_Q5_K, kf.TYPE_Q6_K])
 @pytest.mark.parametrize("rows,n,n_out", [(256, 14336, 4096), (100, 2048, 300), (64, 4096, 1000), (2048, 4096, 2304)])
 def test_gemm_tail_splits(cuda, knobs, ty, rows, n, n_out):
-    """The q5_K / q6_K GEMM's tail split: tiles of a last round at most half full (or a grid below half the CUs) run
-    as 2 or 4 blocks over K ranges, added in split order by the last to arrive. Bit-identical over two calls, within
-    the bar of the unsplit kernel (KF_GEMM_NO_TAIL), and the smaller shapes against the CPU backend's int8 path."""
+    """The q5_K / q6_K GEMM's tail split: the tiles of a last round that is not full (or of a grid below the CUs) run as
+    several blocks over K ranges, whose partial tiles a second launch adds in order. Bit-identical over two calls, within
+    the bar of the plan without splits (KF_GEMM_NO_TAIL), and the smaller shapes against the CPU backend's int8 path."""
     import torch
 
     rng = np.random.default_rng(rows + n + ty)

@@ -206,7 +206,7 @@ def _silu_mul(g, u):
 
 def _check_layer(got, stages, args, ty, n_exp, n_embd, n_ff, rows_checked):
     """Each stage against the CPU backend's int8 expert path on the stage's own inputs (experts::hidden_rows, then
-    down_cols on the GPU's hidden rows, crates/kf-backend-cpu/src/experts.rs:93-124) at the north-star bar; the fused
+    down_cols on the GPU's hidden rows, crates/kf-backend-cpu/src/experts.rs:93-124) at the outputs' bar; the fused
     entry point equal to the staged pipeline; the layer against the CPU float path moe::exec within the reference's
     own int8-vs-float bound (experts.rs:181-217: 2e-2 of the mean magnitude). The layer is not held to 1e-3 against
     the CPU as a whole: the hidden row is quantized again between the two products, and a last-bit difference in a
@@ -320,12 +320,11 @@ def test_moe_ffn_128_experts_top_8(cuda, rows):
 @pytest.mark.parametrize("kq", ["0", "1"])
 @pytest.mark.parametrize("rows,n_exp", [(512, 8), (100, 3)])
 def test_moe_ffn_grouped_gemm_top_2(cuda, knobs, rows, n_exp, kq, split):
-    """Past 64 routed pairs the q4_K layer runs on the grouped tile GEMM (KF_MOE_KQ: 0 the split-scale kernel, 128-row
-    tiles; 1 the one-MFMA-per-group kernel, 64-row tiles): 512 tokens top-2 over eight experts (about 128 pairs an
-    expert, several row tiles each), and 100 tokens over three (the last tile of a slot partial), with some pairs
-    unused; sampled tokens against the CPU backend stage by stage and the float path. The one-MFMA-per-group kernel
-    runs grids of at most two rounds as two K halves a tile (these layers' launches all are); KF_GEMM_NO_TAIL runs
-    them whole."""
+    """Past 64 routed pairs the q4_K layer runs on the grouped tile GEMM (KF_MOE_KQ: 0 its 128-row tiles, 1 its 64-row
+    ones): 512 tokens top-2 over eight experts (about 128 pairs an expert, several row tiles each), and 100 tokens over
+    three (the last tile of a slot partial), with some pairs unused; sampled tokens against the CPU backend stage by
+    stage and the float path. The tiles are cut into equal ranges, one a CU, whose parts a second launch adds;
+    KF_GEMM_NO_TAIL runs them whole."""
     knobs.setenv("KF_MOE_KQ", kq)
     if not split:
         knobs.setenv("KF_GEMM_NO_TAIL", "1")
@@ -343,9 +342,8 @@ def test_moe_ffn_grouped_gemm_top_2(cuda, knobs, rows, n_exp, kq, split):
 @pytest.mark.parametrize("kq", ["0", "1"])
 def test_grouped_gemm_partial_row_tiles(cuda, knobs, kq):
     """Slots whose rows end past a row tile (1, 17, 32, 62 or 72 rows in the last 128-row tile), slots of 5, 32 and 33
-    rows, an empty slot, on both grouped kernels (the one-MFMA-per-group kernel's tiles holding at most 32 rows run its
-    one-tile K loop, the others the full one); every row of every slot against the CPU backend's integer product for
-    its expert."""
+    rows, an empty slot, on both tile heights (a tile runs the K loop of as many 32-row parts as it holds); every row of
+    every slot against the CPU backend's integer product for its expert."""
     import torch
 
     knobs.setenv("KF_MOE_KQ", kq)

@@ -1,6 +1,6 @@
 """GPU parity of the HIP path against the CPU oracle, called through the C ABI on the same seeded inputs.
 
-Bar (from the north star): per-block int32 results bit-exact; fp32 outputs within |got - want| <= 1e-4 + 1e-3 * |want|
+Bar: per-block int32 results bit-exact; fp32 outputs within |got - want| <= 1e-4 + 1e-3 * |want|
 of kf-backend-cpu's matmul_slice (crates/kf-backend-cpu/src/ops.rs:304-346); the quantized activations bit-exact with
 quantize_activations (crates/kf-quant/src/lib.rs:81-140). Shapes follow the reference's differential tests
 (crates/kf-backend-cuda/tests/quant.rs:46-83: ragged n_out, several widths) plus the full Llama-3-8B shapes.
@@ -665,11 +665,10 @@ def test_gemm_q8_0_split_k(cuda, knobs, rows, n, n_out, splits, var):
 @pytest.mark.parametrize("kq", ["0", "1"])
 @pytest.mark.parametrize("rows,n,n_out", [(2048, 4096, 14336), (130, 2048, 600), (257, 1024, 300), (96, 14336, 512)])
 def test_gemm_q4_k_tail_halves(cuda, knobs, rows, n, n_out, kq):
-    """The q4_K GEMMs' tail split, both kernels (KF_Q4K_KQ: 0 the split-scale kernel, two K halves; 1 the
-    one-MFMA-per-group kernel, 2-4 K ranges): tiles of a last round at most half full (all of them when the grid is
-    below half the CUs) run over K ranges whose partial tiles the last to arrive adds in order. Against the unsplit
-    kernel (KF_GEMM_NO_TAIL) within the f32 bar, bit-identical over two calls on one stream (the tickets return to
-    zero), and the smaller shapes against the CPU backend; 4, 8 and 56 super-blocks a row, ragged tiles."""
+    """The q4_K GEMM's tail split at both of its taller tiles (KF_Q4K_KQ: 0 128 rows, 1 64 rows): the tiles of a last
+    round that is not full (all of them when the grid is below the CUs) run over K ranges whose partial tiles a second
+    launch adds in order. Against whole tiles (KF_GEMM_NO_TAIL) within the f32 bar, bit-identical over two calls on one
+    stream, and the smaller shapes against the CPU backend; 4, 8 and 56 super-blocks a row, ragged tiles."""
     import torch
 
     knobs.setenv("KF_Q4K_KQ", kq)
@@ -696,13 +695,19 @@ def test_gemm_q4_k_tail_halves(cuda, knobs, rows, n, n_out, kq):
         _close(outs[0], oracle.matmul_slice(kf.TYPE_Q4_K, w, n, n_out, x, bias))
 
 
+@pytest.mark.parametrize("old", [True, False])
 @pytest.mark.parametrize("rows,n,n_out", [(2048, 4096, 14336), (300, 1024, 1000), (129, 14336, 600)])
-def test_gemm_q8_0_tail_halves(cuda, knobs, rows, n, n_out):
-    """The q8_0 tile GEMM's tail split (two blocks a CU: a last round at most half full, or a grid below half of
-    them, runs its tiles as two K halves added in half order by the second to arrive): against the unsplit kernel
-    (KF_GEMM_NO_TAIL) within the f32 bar, bit-identical over two calls, the smaller shapes against the CPU backend."""
+def test_gemm_q8_0_tail_halves(cuda, knobs, rows, n, n_out, old):
+    """The q8_0 tile GEMMs' tail splits. The 128 x 128 kernel (old: KF_Q8_V=3, and KF_GEMM_TILE for no row slices; two
+    blocks a CU: a last round at most half full, or a grid below half of them, runs its tiles as two K halves added in
+    half order by the second to arrive), and the kernel the cost picks, the one of any width (K ranges, a second launch
+    adds the parts): against whole tiles (KF_GEMM_NO_TAIL) within the f32 bar, bit-identical over two calls, the smaller
+    shapes against the CPU backend."""
     import torch
 
+    if old:
+        knobs.setenv("KF_Q8_V", 3)
+        knobs.setenv("KF_GEMM_TILE", 1)
     w = _weights(kf.TYPE_Q8_0, n_out, n, seed=rows + n)
     x = kf.synth_normal(rows + 7, 1.0, rows * n).reshape(rows, n)
     bias = kf.synth_normal(6, 1.0, n_out)

@@ -1,7 +1,7 @@
 """kf_hip_matmul_noalloc (the entry point that allocates nothing: its activation scratch is a static per-GPU array in the
 library) against kf_hip_matmul with a caller-allocated scratch, through the C ABI: bit-identical outputs on two calls in
-a row, the second smaller than the first (the array keeps the first call's contents), and both within the north-star
-bar of the CPU backend's matmul_slice (crates/kf-backend-cpu/src/ops.rs:304-346)."""
+a row, the second smaller than the first (the array keeps the first call's contents), and both within the
+usual bar of the CPU backend's matmul_slice (crates/kf-backend-cpu/src/ops.rs:304-346)."""
 import numpy as np
 import pytest
 
