@@ -108,8 +108,9 @@ int kf_hip_gated_act_q8(const float* gate, const float* up, int rows, int n, int
  * row_bytes must equal the type's row size for n (rows are packed). */
 
 /* Decode and small-batch product of `rows` activation rows: one row is the streaming GEMV, several rows the
- * multi-row product that reads each weight row once per eight activation rows (q8_0) or sixteen (the K types, which take
- * the tile GEMM of kf_hip_gemm_i8 instead where a cost model fitted on MI355X favours it). Replaces matvec_i8_launch
+ * multi-row product that reads each weight row once per eight activation rows (q8_0) or sixteen (the K types), or the tile
+ * GEMM of kf_hip_gemm_i8 where a cost model fitted on MI355X favours it: from 33 rows on, and from two on q8_0 widths that
+ * are no multiple of 256. q8_0 and q4_K rows of at most 32768 columns. Replaces matvec_i8_launch
  * (exec.rs:1996-2039) with the kernels matvec_i8 / matvec_i8_1 / matvec_i8_1s / mm_i8_{8,16,32} /
  * mm_frag_{8,16,24,32} (crates/kf-backend-cuda/src/kernels/quant.cuh:604-627, mm_frag.cuh:294-300).
  * q5_K and q6_K weights (Q8K-kind activations, any row count: one launch per eight activation rows) run their own
@@ -121,8 +122,8 @@ int kf_hip_gemv(uint32_t ty, const void* w, int64_t row_bytes, const void* act, 
 /* Batched / prefill int8 GEMM on native rows: y [rows][n_out] from `rows` activation rows of the weight type's kind.
  * q8_0 (Q8_0-kind activations, n a multiple of 128): one int8 MFMA per 32-column group gives the exact int32 block
  * dots, rescaled by the group's activation and weight scales. q4_K, q5_K
- * and q6_K (Q8K-kind activations, n a multiple of 256; q6_K here only a multiple of 2048, kf_hip_matmul and kf_hip_gemv
- * take any): the products scale x value as two int8 operand planes, so two int8 MFMA chains form the exact super-block
+ * and q6_K (Q8K-kind activations, n a multiple of 256; q6_K here only a multiple of 2048, and q5_K and q6_K only below 2
+ * GB of weights, though kf_hip_matmul and kf_hip_gemv run the same kernel on any): the products scale x value as two int8 operand planes, so two int8 MFMA chains form the exact super-block
  * integer; the mins term by an exact f16 MFMA per super-block, and the float rescale once per 256 columns; other shapes
  * return KF_E_UNSUPPORTED.
  * Replaces kf8_gemm_dense / Store::gemm (crates/kf-backend-cuda/src/kernels/kf8.cu:375-395, HAS_M for q4_K / q5_K;

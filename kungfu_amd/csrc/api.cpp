@@ -275,8 +275,9 @@ int kf_hip_gemm_i8(uint32_t ty, const void* w, int64_t row_bytes, const void* ac
     const int rc = check_product(ty, w, row_bytes, act, y, rows, n, n_out);
     if (rc != KF_OK) return rc;
     if (ty == KF_TYPE_Q4_K || ty == KF_TYPE_Q5_K || ty == KF_TYPE_Q6_K) {
+        // the entry point's contract, narrower than the kernel's: callers that ask here first whether a shape is taken keep their answer
         if (ty != KF_TYPE_Q4_K && (row_bytes % 16 != 0 || (int64_t)n_out * row_bytes >= (1ll << 31)))
-            return fail(KF_E_UNSUPPORTED, "the q5_K/q6_K GEMM needs 16-byte aligned weights and rows (q6_K: %d columns, a multiple of 2048) and a matrix below 2 GB; kf_hip_gemv takes any", n);
+            return fail(KF_E_UNSUPPORTED, "kf_hip_gemm_i8 takes q5_K/q6_K rows of whole 16-byte pieces (q6_K: a multiple of 2048 columns, not %d) and a matrix below 2 GB; kf_hip_matmul and kf_hip_gemv take any", n);
         const hipError_t e = kf_launch_gemm_kq(ty, w, row_bytes, act, bias, res, y, rows, n_out, n, static_cast<hipStream_t>(stream), true);
         return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
     }

@@ -428,8 +428,10 @@ Q8Plan q8_plan(int M, int N, int K, bool split) {
 // Whether the product costs less than `us` on stream `s`, with the split scratch if it can have it. What no plan goes below comes first: the plan's search would cost the shortest
 // products a noticeable part of their launch.
 bool kf_gemm_q8_below(int M, int N, int K, double us, hipStream_t s, bool graph) {
-    const double least = std::min((K / 32 + Q8_G - 1) / Q8_G * Q8_ST_US[0], 2.0 + 2 * Q8_ST_US[0]);  // unsplit, split
-    if (Q8_LAUNCH_US[0] + Q8_ROUND_US[0] + least >= us) return false;
+    const int nst = (K / 32 + Q8_G - 1) / Q8_G;
+    bool may = false;
+    for (int v = 0; v < 3; v++) may |= Q8_LAUNCH_US[v] + Q8_ROUND_US[v] + std::min(nst * Q8_ST_US[v], 2.0 + 2 * Q8_ST_US[v]) < us;  // unsplit, split
+    if (!may) return false;
     const Q8Plan p = q8_plan(M, N, K, true);
     if (p.us + (p.S > 1 ? 2.0 : 0.0) >= us) return false;  // the second launch's host work, which a short product does not hide
     return p.S == 1 || KfSplit::ready(s, graph) || q8_plan(M, N, K, false).us < us;
