@@ -335,15 +335,19 @@ int kf_hip_rms_norm_matmul(uint32_t ty, const void* w, int n_in, int n_out, cons
 
 }  // extern "C"
 
-// The few-row products' cost on the K types (MI355X, us; fitted over 4-128 rows at 4096 -> 4096, 4096 -> 14336 and
-// 14336 -> 4096): about 5.5 plus, per 16 activation rows and MB of weights, 0.22 (q4_K), 0.20 (q5_K) or 0.32 (q6_K). q6_K
-// rows that start off a dword (an odd number of super-blocks) run the per-lane product, whose cost grows with each row
+// The few-row products' cost on the K types (MI355X, us; fitted over 33-512 rows at 1024 -> 512 to 8192 -> 8192 and 14336 ->
+// 512): the larger of 2.5 plus the latency of a pass of 16 activation rows, which grows with the super-blocks of a row, and
+// 5.5 plus its MB of weights, per pass. Matrices of few outputs cost their latency: 300 rows of q4_K 1024 -> 512 28 us against the
+// tile GEMM's 10, of q6_K 14336 -> 512 285 against 25. q6_K rows that start off a dword (an odd number of super-blocks) run the per-lane product, whose cost grows with each row
 // (1792 -> 3584, 6400 -> 2304 and 13056 -> 2048 at 2-16 rows: 7.1-36.6, 11.7-53.3 and 15.8-69.8 us); q4_K rows wider than the few-row product stages run as one GEMV launch per row.
 static double kq_few_rows_us(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes) {
     const double mb = (double)n_out * row_bytes / 1e6;
     if (ty == KF_TYPE_Q4_K && n_in > kf_rows_max_n(ty)) return rows * (2.5 + 0.22 * mb);
     if (!kf_rows_mma_1_ok(ty, w, row_bytes, n_in, n_out, rows)) return 2.0 + (rows + 7) / 8 * (1.0 + 0.3 * mb) + rows * (0.9 + 0.13 * mb);
-    return 5.5 + (rows + 15) / 16 * mb * (ty == KF_TYPE_Q4_K ? 0.22 : ty == KF_TYPE_Q5_K ? 0.20 : 0.32);
+    const int k = ty == KF_TYPE_Q4_K ? 0 : ty == KF_TYPE_Q5_K ? 1 : 2;
+    constexpr double pass[3] = {0.95, 1.0, 1.1}, sb[3] = {0.095, 0.114, 0.245}, per_mb[3] = {0.21, 0.20, 0.33};
+    const int passes = (rows + 15) / 16;
+    return std::max(2.5 + passes * (pass[k] + sb[k] * (n_in / 256)), 5.5 + passes * per_mb[k] * mb);
 }
 
 // Up to here the K types, and q8_0 rows of whole 256-column steps, keep the few-row kernels and their order of the f32 sums
@@ -363,14 +367,15 @@ static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_o
 
 // The older q8_0 products' cost (MI355X, us; fitted over 4-2048 rows at the shapes of gemm_q8.hip's model). kf_hip_gemv's
 // multi-row product costs so much a row (1888 -> 1774: 9.3 us at 9 rows, 14.2 at 16; 4128 -> 2048: 16.4 and 25.0), and past the
-// width it stages is one GEMV a row. kf_hip_gemm_i8's: up to 64 rows the small-batch kernels by the weights' MB, past that the
-// 128 x 128 tile kernel (two blocks a CU) by its tiles and 128-column stages, or 64-row slices through the small-batch
-// kernels; these need rows of whole 256-column steps, and other widths have only the tile GEMM.
+// width it stages is one GEMV a row. kf_hip_gemm_i8's: up to 64 rows the small-batch kernels by the weights' MB (1024 -> 512
+// at 33-64 rows 7.4-8.7 us against the tile GEMM's 11.4-12.4), past that the 128 x 128 tile kernel (two blocks a CU) by
+// its tiles and 128-column stages, or 64-row slices through the small-batch kernels; these need rows of whole 256-column
+// steps, and other widths have only the tile GEMM.
 static double q8_old_us(int rows, int n_in, int n_out, int64_t row_bytes, bool multi) {
     const double mb = (double)n_out * row_bytes / 1e6;
     if (!multi) return n_in > kf_rows_max_n(KF_TYPE_Q8_0) ? rows * (3.0 + 0.22 * mb) : 1.7 + 0.26 * mb + rows * (0.33 + 0.11 * mb);
     if (n_in % 256 != 0) return 1e30;
-    if (rows <= 64) return rows <= 16 ? 4.5 + 0.2 * mb : rows <= 32 ? 7.5 + 0.20 * mb : 10.5 + 0.33 * mb;
+    if (rows <= 64) return rows <= 16 ? 4.5 + 0.2 * mb : rows <= 32 ? 7.5 + 0.20 * mb : std::min(10.5, 7.5 + mb) + 0.33 * mb;
     const double t = (double)((n_out + 127) / 128) * ((rows + 127) / 128), st = n_in / 128;
     return std::min(6.0 + st * (t > 256 ? 3.2 * t / 512 : 0.75 + t / 224), ((rows + 63) / 64) * (9.0 + 0.45 * mb));
 }

@@ -172,3 +172,25 @@ def test_infinite_and_nan_block_scales(cuda, knobs, ty, tm, tail):
         want = oracle.matmul_i8(ty, np.ascontiguousarray(bad[cols]).reshape(len(cols), -1), n, len(cols), x, None)
     # (which of the two, and an infinity's sign, follow the order of the terms; the CPU multiplies the scales out first)
     assert not np.isfinite(want).any() and not np.isfinite(outs[1][:, cols]).any()
+
+
+@pytest.mark.parametrize("ty", K_TYPES)
+@pytest.mark.parametrize("rows,n,n_out,gemm", [(300, 1024, 512, True), (256, 14336, 40, True), (200, 1792, 600, True), (48, 1024, 512, False)])
+def test_few_outputs_price_the_few_row_products_latency(cuda, knobs, ty, rows, n, n_out, gemm):
+    """Matrices of few outputs: each 16-row pass of the few-row product costs the latency of a whole row, so many rows take
+    the tile GEMM (the bits of KF_KQ_GEMM=1) and 48 short ones do not (those of KF_KQ_GEMM=0)."""
+    import torch
+
+    w = _t(_blocks(ty, n_out, n, rows + n), cuda)
+    x = _t(kf.synth_normal(rows, 1.0, rows * n).reshape(rows, n), cuda)
+    act = kf.alloc_act(rows, n, cuda)
+    bits = []
+    for force in (None, 0, 1):
+        if force is not None:
+            knobs.setenv("KF_KQ_GEMM", force)
+        y = torch.full((rows, n_out), float("nan"), device=cuda)
+        kf.matmul(ty, w, x, act, y, n_out)
+        torch.cuda.synchronize()
+        bits.append(y.cpu().numpy().view(np.uint32))
+    assert not np.array_equal(bits[1], bits[2])
+    assert np.array_equal(bits[0], bits[2 if gemm else 1])

@@ -535,11 +535,10 @@ def test_matmul_q4_k_cost_model_rows(cuda, rows):
 
 
 @pytest.mark.parametrize("rows", [96, 256])
-def test_matmul_q4_k_wide_k_few_row_and_gemm(cuda, rows):
-    """Wide K (down's 14336 columns, a small n_out): the cost model keeps the few-row product here (its weight pass
-    is cheap against a GEMM round of 56 super-blocks), which then carries 96 or 256 rows in 64-row passes. The
-    selected kf_hip_matmul must equal that product (kf_hip_gemv) bit for bit; the few-row product and the tile GEMM
-    (kf_hip_gemm_i8) each against the CPU backend's int8 path on every 7th row."""
+def test_matmul_q4_k_wide_k_few_row_and_gemm(cuda, knobs, rows):
+    """Wide K (down's 14336 columns, a small n_out): the few-row product (KF_KQ_GEMM=0) carries 96 or 256 rows in passes
+    of 16. kf_hip_matmul and kf_hip_gemv give its bits; the few-row product and the tile GEMM (kf_hip_gemm_i8) each
+    against the CPU backend's int8 path on every 7th row."""
     import torch
 
     ty, n, n_out = kf.TYPE_Q4_K, 14336, 40
@@ -548,6 +547,7 @@ def test_matmul_q4_k_wide_k_few_row_and_gemm(cuda, rows):
     wt, xt = _tensor(w, cuda), _tensor(x, cuda)
     act = kf.alloc_act(rows, n, cuda)
     outs = {}
+    knobs.setenv("KF_KQ_GEMM", 0)
     for name in ("matmul", "gemv", "gemm"):
         y = torch.full((rows, n_out), float("nan"), device=cuda)
         if name == "matmul":

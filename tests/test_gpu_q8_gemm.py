@@ -152,3 +152,22 @@ def test_ragged_widths_lose_no_precision(cuda, knobs, rows, n, n_out, tail):
         torch.cuda.synchronize()
         errs.append(np.linalg.norm(y.cpu().numpy() - want) / np.linalg.norm(want))
     assert max(errs[:3]) <= errs[3] and max(errs[1:3]) <= np.sqrt(5.4) * 2.0**-24 / np.sqrt(3), errs
+
+
+def test_small_matrices_keep_the_small_batch_kernels(cuda, knobs):
+    """48 rows of 1024 -> 512: the small-batch kernels' bits (KF_Q8_V=3), not the tile GEMM's, which takes longer there."""
+    import torch
+
+    rows, n, n_out = 48, 1024, 512
+    w = _t(_blocks(n_out, n, 9), cuda)
+    x = _t(kf.synth_normal(rows, 1.0, rows * n).reshape(rows, n), cuda)
+    act = kf.alloc_act(rows, n, cuda)
+    bits = []
+    for v in (None, 3, 0):
+        if v is not None:
+            knobs.setenv("KF_Q8_V", v)
+        y = torch.full((rows, n_out), float("nan"), device=cuda)
+        kf.matmul(TY, w, x, act, y, n_out)
+        torch.cuda.synchronize()
+        bits.append(y.cpu().numpy().view(np.uint32))
+    assert np.array_equal(bits[0], bits[1]) and not np.array_equal(bits[0], bits[2])
