@@ -58,7 +58,7 @@ bool kf_gemm_kq_ok(uint32_t ty, const void* w, int64_t row_bytes, int K, int N);
 bool kf_gemm_kq_below(uint32_t ty, int M, int N, int K, double us, hipStream_t s, bool graph);
 hipError_t kf_launch_gemm_kq_moe(const void* w, const void* w2, int64_t expert_bytes, int64_t row_bytes, int n_split, const void* act, int pairs,
                                  int n_slots, const int32_t* offsets, const int32_t* out_rows, float* y, int N, int K, hipStream_t s);
-static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes, hipStream_t s, bool graph);
+static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes, hipStream_t s, bool matmul, bool graph);
 hipError_t kf_launch_gemm_kq(uint32_t ty, const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y,
                              int M, int N, int K, hipStream_t s, bool graph);
 int kf_rows_max_n(uint32_t ty);
@@ -215,12 +215,12 @@ int kf_hip_gated_act_q8(const float* gate, const float* up, int rows, int n, int
     return e == hipSuccess ? KF_OK : hip_fail(e, "gated_act_q8 launch");
 }
 
-// kf_hip_gemv, and the products kf_hip_matmul leaves to it. `graph`: under graph capture the product may use the graph slot
-// of the split scratch
+// kf_hip_gemv, and the products kf_hip_matmul leaves to it (`matmul`)
 static int gemv_product(uint32_t ty, const void* w, int64_t row_bytes, const void* act, const float* bias, const float* res, float* y, int rows,
-                        int n, int n_out, void* stream, bool graph) {
+                        int n, int n_out, void* stream, bool matmul) {
     const int rc = check_product(ty, w, row_bytes, act, y, rows, n, n_out);
     if (rc != KF_OK) return rc;
+    const bool graph = matmul && graph_split(row_bytes);  // whether a captured product may use the split scratch
     // one limit for every row count, whichever product these rows would take
     if ((ty == KF_TYPE_Q8_0 || ty == KF_TYPE_Q4_K) && n > kf_gemv_max_n())
         return fail(KF_E_UNSUPPORTED, "%d columns above the %d the GEMV stages in LDS", n, kf_gemv_max_n());
@@ -230,7 +230,7 @@ static int gemv_product(uint32_t ty, const void* w, int64_t row_bytes, const voi
         return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
     }
     // the K types: the tile GEMM where its cost is below the few-row product's
-    if (ty != KF_TYPE_Q8_0 && n_out > 0 && kq_gemm_pays(ty, w, rows, n, n_out, row_bytes, s, graph)) {
+    if (ty != KF_TYPE_Q8_0 && n_out > 0 && kq_gemm_pays(ty, w, rows, n, n_out, row_bytes, s, matmul, graph)) {
         const hipError_t e = kf_launch_gemm_kq(ty, w, row_bytes, act, bias, res, y, rows, n_out, n, s, graph);
         return e == hipSuccess ? KF_OK : hip_fail(e, "gemm launch");
     }
@@ -350,19 +350,35 @@ static double kq_few_rows_us(uint32_t ty, const void* w, int rows, int n_in, int
     return std::max(2.5 + passes * (pass[k] + sb[k] * (n_in / 256)), 5.5 + passes * per_mb[k] * mb);
 }
 
-// Up to here the K types, and q8_0 rows of whole 256-column steps, keep the few-row kernels and their order of the f32 sums
-// (from two rows on; a single row has the GEMV's). Either order is equally far from the exact result, but the outputs of a
-// decoded batch then agree with those of earlier builds: layers chained through int8 turn another order's last bits into
-// differences of 2e-3 to 4e-3 after three of them (3840 -> 11008 at 12 rows, 10240 at 26). Other q8_0 widths go by cost and
-// change the order with it, and K splits change it with the row count. The price: q4_K 4096 -> 14336 at 32 rows takes
-// 23.1 us against the GEMM's 18.9, q6_K rows of an odd number of super-blocks 53 against 18 (6400 -> 2304 at 16 rows).
-constexpr int KF_FEW_ROWS = 32;
+// Up to KF_FEW_ROWS rows kf_hip_matmul's choice on the K types, and the order of the f32 sums with it, stays what it was
+// before the few-row product's cost was fitted as above and the tile GEMM took its present form: the outputs of a decoded
+// batch agree with those of earlier builds, though another order would be equally far from the exact result. Layers chained
+// through int8 turn its last bits into differences of 2e-3 to 5e-3 after three of them (3840 -> 11008 at 12 rows, 4608 -> 27648
+// at 25). The tile GEMM, in two or four K ranges, is the product of the largest matrices from 17 rows (q4_K: 4608 -> 27648)
+// or 26 (q5_K, q6_K). The price: q4_K 4096 -> 14336 at 32 rows takes 23.1 us against the GEMM's 18.9, q6_K rows of an odd
+// number of super-blocks 53 against 18 (6400 -> 2304 at 16 rows). q8_0 rows of whole 256-column steps keep the small-batch
+// kernels up to there; other q8_0 widths go by cost and change the order with it, and their K splits change it with the
+// row count.
+static bool kq_few_rows_gemm(uint32_t ty, int rows, int n_in, int n_out, int64_t row_bytes) {
+    if (n_in > kf_rows_max_n(KF_TYPE_Q4_K) && ty == KF_TYPE_Q4_K) return false;
+    const double mb = (double)n_out * row_bytes / 1e6;
+    const int nsb = n_in / 256, cus = kf_cu_count(), T = (n_out + 255) / 256, rem = T % cus;
+    int S = 1;
+    while (S < 4 && rem * S * 2 <= cus && nsb / (S * 2) >= 2) S *= 2;
+    // rounds of 256-column tiles in super-blocks, the last one in S ranges, or at most in halves
+    const double full = (double)(T / cus) * nsb, ranges = full + (rem ? (double)nsb / S : 0.0), halves = full + (rem ? (double)nsb / std::min(S, 2) : 0.0);
+    if (ty == KF_TYPE_Q4_K) return std::min(13.2 + 2.95 * ranges, 7.4 + 4.84 * halves) < (rows + 15) / 16 * (0.28 * mb + 1.0);
+    if (row_bytes % 16 != 0 || (int64_t)n_out * row_bytes >= (1ll << 31)) return false;
+    return 14.5 + ranges * (ty == KF_TYPE_Q6_K ? 5.72 : 3.23) < rows / 64.0 * mb * (ty == KF_TYPE_Q6_K ? 1.55 : 1.05);
+}
 
-// Whether the tile GEMM beats the few-row product (KF_KQ_GEMM=0 / 1 forces the choice, a comparison knob)
-static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes, hipStream_t s, bool graph) {
+// Whether the tile GEMM beats the few-row product (KF_KQ_GEMM=0 / 1 forces the choice, a comparison knob); `matmul`: asked by
+// kf_hip_matmul (kf_hip_gemv takes the few-row product up to KF_FEW_ROWS)
+static bool kq_gemm_pays(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes, hipStream_t s, bool matmul, bool graph) {
     if (rows < 2 || !kf_gemm_kq_ok(ty, w, row_bytes, n_in, n_out)) return false;
     if (kf_knob_on(KF_KNOB_KQ_GEMM)) return kf_knob(KF_KNOB_KQ_GEMM) != 0;
-    return rows > KF_FEW_ROWS && kf_gemm_kq_below(ty, rows, n_out, n_in, kq_few_rows_us(ty, w, rows, n_in, n_out, row_bytes), s, graph);
+    if (rows <= KF_FEW_ROWS) return matmul && kq_few_rows_gemm(ty, rows, n_in, n_out, row_bytes);
+    return kf_gemm_kq_below(ty, rows, n_out, n_in, kq_few_rows_us(ty, w, rows, n_in, n_out, row_bytes), s, graph);
 }
 
 // The older q8_0 products' cost (MI355X, us; fitted over 4-2048 rows at the shapes of gemm_q8.hip's model). kf_hip_gemv's
@@ -407,7 +423,7 @@ int product(uint32_t ty, const void* w, int64_t rb, const void* act, const float
     if (rows >= 96 && ty == KF_TYPE_Q4_K && n_in > kf_gemv_max_n() && n_out > 0)
         return kf_hip_gemm_i8(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream);
     // other widths of q8_0, and the K types: the tile GEMM or the few-row product, by the one rule of kf_hip_gemv
-    return gemv_product(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream, graph_split(rb));
+    return gemv_product(ty, w, rb, act, bias, res, y, rows, n_in, n_out, stream, true);
 }
 
 // A grouped product's members from the reference's segment words (quant.cuh:301-305): per member the byte offsets of

@@ -800,7 +800,7 @@ __global__ void __launch_bounds__(KQ_THREADS, 2) gemm_kq_kernel(const uint8_t* w
     }
 }
 
-// Adds the partial tiles of the tiles that several blocks shared, in K order (four at a time as a tree), with bias and residual. One thread an output;
+// Adds the partial tiles of the tiles that several blocks shared, in K order (four at a time by themselves), with bias and residual. One thread an output;
 // a block takes RED of the TM * 16 (register, 512 threads) slices of a tile, so every load and store is a run of whole
 // lines: one slice with one matrix, whose few tiles have many parts (four made 32 rows of 4096 x 4096 14.2 us, 12.7 with
 // one), four in the grouped form, where most blocks have nothing to add. A launch of its own: the last block to arrive adding them by itself took 10-40 us with 16 partial tiles, as
@@ -838,7 +838,7 @@ __global__ void __launch_bounds__(KQ_THREADS) kq_reduce_kernel(KqWork work, cons
             for (int e = 0; e < RED; e++) a[u][e] = k + u < d.count ? p[(at * R + e) * KQ_THREADS] : 0.0f;
         }
 #pragma unroll
-        for (int e = 0; e < RED; e++) v[e] += (a[0][e] + a[1][e]) + (a[2][e] + a[3][e]);
+        for (int e = 0; e < RED; e++) v[e] += ((a[0][e] + a[1][e]) + a[2][e]) + a[3][e];
     }
     const float bn = bias ? bias[n] : 0.0f;
 #pragma unroll
@@ -912,19 +912,21 @@ KqPlan kq_plan_tm(uint32_t ty, int tm, int M, int N, int K, bool split) {
     p.full = p.T;
     p.S = 1;
     p.us = (rounds + (rem ? 1 : 0)) * cost(nsb, nsb);
-    // the tiles of the last round as S blocks each, S the cheapest that fits the CUs with two super-blocks a block or more
+    // the tiles of the last round as S blocks each, S the cheapest that fits the CUs with two super-blocks a block or more; up
+    // to KF_FEW_ROWS rows two or four, whichever fits, and f32 sums (the order a decoded batch keeps)
+    const bool few = M <= KF_FEW_ROWS && !ragged;
     for (int S = 2; split && rem && rem * S <= max_g && 2 * S <= nsb; S++) {
         const int n = (nsb + S - 1) / S, most = rounds ? nsb : n;
         const double part = rounds * cost(nsb, most) + KQ_PART_US[t] * tm * rem * S / cus, us = part + cost(n, most);
-        if (part + cost(2, 2) >= p.us) break;
-        if (us < p.us) {
+        if (few ? S > 4 : part + cost(2, 2) >= p.us) break;
+        if (few ? S != 3 : us < p.us) {
             p.us = us;
             p.full = p.T - rem;
             p.S = S;
         }
     }
     p.us += 1.8;
-    p.wide = fits && (p.full > 0 ? nsb : (nsb + p.S - 1) / p.S) > KQ_LONG;
+    p.wide = fits && !few && (p.full > 0 ? nsb : (nsb + p.S - 1) / p.S) > KQ_LONG;
     return p;
 }
 

@@ -22,6 +22,9 @@ inline hipError_t kf_raise_lds(const void* fn, int bytes) {
     return e;
 }
 
+// Up to here the products of a decoded batch keep an order of their f32 sums (api.cpp)
+constexpr int KF_FEW_ROWS = 32;
+
 // Compute units of the current device, read once per device and remembered under a lock (256 if the query fails).
 inline int kf_cu_count() {
     static std::mutex mu;

@@ -194,3 +194,40 @@ def test_few_outputs_price_the_few_row_products_latency(cuda, knobs, ty, rows, n
         bits.append(y.cpu().numpy().view(np.uint32))
     assert not np.array_equal(bits[1], bits[2])
     assert np.array_equal(bits[0], bits[2 if gemm else 1])
+
+
+@pytest.mark.parametrize("ty,rows,n,n_out,gemm", [(kf.TYPE_Q4_K, 16, 4608, 27648, False), (kf.TYPE_Q4_K, 25, 4608, 27648, True),
+                                                  (kf.TYPE_Q4_K, 32, 8192, 16384, True), (kf.TYPE_Q5_K, 32, 4096, 28672, True),
+                                                  (kf.TYPE_Q6_K, 28, 4096, 28672, True), (kf.TYPE_Q6_K, 17, 4096, 28672, False)])
+def test_decoded_batches_keep_their_product(cuda, knobs, ty, rows, n, n_out, gemm):
+    """Up to 32 rows kf_hip_matmul takes the tile GEMM on the largest matrices only, with K in two or four f32 ranges summed in
+    order (the bits of a 128- or 64-row tile's plan as well), the few-row product elsewhere; kf_hip_gemv always the latter."""
+    import torch
+
+    w = _t(np.tile(_blocks(ty, 512, n, rows + n), (n_out // 512, 1)), cuda)
+    x = _t(kf.synth_normal(rows, 1.0, rows * n).reshape(rows, n), cuda)
+    act = kf.alloc_act(rows, n, cuda)
+    kf.quant_act(x, act, kf.ACT_Q8K)
+
+    def bits(entry, **ks):
+        for k, v in ks.items():
+            knobs.setenv(k, v)
+        y = torch.full((rows, n_out), float("nan"), device=cuda)
+        entry(y)
+        torch.cuda.synchronize()
+        for k in ks:
+            knobs.delenv(k)
+        return y.cpu().numpy().view(np.uint32)
+
+    def matmul(y):
+        kf.matmul(ty, w, x, act, y, n_out)
+
+    def gemv(y):
+        kf.gemv(ty, w, act, y, rows, n, n_out)
+
+    few = bits(gemv, KF_KQ_GEMM=0)
+    tiles = [bits(matmul, KF_KQ_GEMM=1, KF_KQ_TM=tm) for tm in (1, 2, 4)]
+    assert np.array_equal(tiles[0], tiles[1]) and np.array_equal(tiles[0], tiles[2])
+    assert not np.array_equal(few, tiles[0])
+    assert np.array_equal(bits(matmul), tiles[0] if gemm else few)
+    assert np.array_equal(bits(gemv), few)
