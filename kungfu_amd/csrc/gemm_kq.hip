@@ -37,6 +37,8 @@
 #include "kf_device.h"
 #include "kf_host.h"
 
+#include <algorithm>
+#include <cmath>
 #include <optional>
 #include <type_traits>
 
@@ -116,8 +118,8 @@ struct KqDesc {
 //    block each, so that every CU gets the same work however the pairs fall on the slots; a tile weighs its number of
 //    32-row parts plus one (the weight side). A tile inside a range is stored directly; of a tile that is cut, every
 //    block leaves its part (slot 2 b + 1 for the part with the tile's first super-block, 2 b otherwise: a range has at
-//    most one of each) and the block with its start describes it in desc[b]. part == nullptr: a range takes the tiles
-//    that start in it, whole.
+//    most one of each) and the block with its start describes it in desc[b]. part == nullptr: every tile weighs one and
+//    is a block of its own, for grids where the parts' way through memory costs more than the rounds it evens out.
 struct KqWork {
     float* part;
     KqDesc* desc;
@@ -182,28 +184,30 @@ __device__ __forceinline__ T* kq_uniform(T* p) {
     return reinterpret_cast<T*>(kq_uniform((int64_t)reinterpret_cast<uint64_t>(p)));
 }
 
-// Grouped form: the weight of a slot of `rows` rows (per super-block and column tile) in tiles of TM 32-row parts
+// Grouped form: the weight of a slot of `rows` rows (per super-block and column tile) in tiles of TM 32-row parts, or
+// (whole) its number of tiles
 template <int TM>
-__device__ __forceinline__ int kq_slot_w(int rows) {
+__device__ __forceinline__ int kq_slot_w(int rows, bool whole) {
+    if (whole) return (rows + 32 * TM - 1) / (32 * TM);
     const int full = rows / (32 * TM), rest = rows - full * 32 * TM;
     return full * (TM + 1) + (rest > 0 ? (rest + 31) / 32 + 1 : 0);
 }
 
 // The sum of the slots' weights (every lane of the wave calls it)
 template <int TM>
-__device__ int kq_slots_w(const int32_t* __restrict__ offsets, int n_slots) {
+__device__ int kq_slots_w(const int32_t* __restrict__ offsets, int n_slots, bool whole) {
     int t = 0;
-    for (int s = threadIdx.x & 63; s < n_slots; s += 64) t += kq_slot_w<TM>(offsets[s + 1] - offsets[s]);
+    for (int s = threadIdx.x & 63; s < n_slots; s += 64) t += kq_slot_w<TM>(offsets[s + 1] - offsets[s], whole);
     return kq_uniform(kf_wave_isum(t));
 }
 
 // The slot whose weight range holds position q, and the position inside it
 template <int TM>
-__device__ int kq_find_slot(const int32_t* __restrict__ offsets, int n_slots, int& q) {
+__device__ int kq_find_slot(const int32_t* __restrict__ offsets, int n_slots, bool whole, int& q) {
     const int lane = threadIdx.x & 63;
     for (int base = 0;; base += 64) {
         const int s = base + lane;
-        int v = s < n_slots ? kq_slot_w<TM>(offsets[s + 1] - offsets[s]) : 0;
+        int v = s < n_slots ? kq_slot_w<TM>(offsets[s + 1] - offsets[s], whole) : 0;
         const int own = v;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -374,10 +378,12 @@ __global__ void __launch_bounds__(KQ_THREADS, 2) gemm_kq_kernel(const uint8_t* w
     extern __shared__ __align__(256) uint8_t lds[];
     KqState& st = *reinterpret_cast<KqState*>(lds + G::LDS);
     if constexpr (MOE) {
-        // positions are super-blocks times tile weights, from the first tile of all
-        const int nsb = K_ >> 8, NT = (N_ + KQ_BN - 1) / KQ_BN;
-        const int sw = kq_slots_w<TM>(moe.offsets, moe.n_slots), U = NT * nsb * sw;
-        const int Gr = max(min(work.S, U / (4 * (TM + 1))), U > 0 ? 1 : 0);  // at least a few super-blocks a range
+        // positions are super-blocks times tile weights, from the first tile of all (whole tiles: tiles)
+        const bool whole = !work.part;
+        const int unit = whole ? 1 : K_ >> 8, NT = (N_ + KQ_BN - 1) / KQ_BN;
+        const int sw = kq_slots_w<TM>(moe.offsets, moe.n_slots, whole), U = NT * unit * sw;
+        // at least a few super-blocks a range, where tiles are cut
+        const int Gr = whole ? min(work.S, U) : max(min(work.S, U / (4 * (TM + 1))), U > 0 ? 1 : 0);
         const bool idle = (int)blockIdx.x >= Gr;
         const int b = idle ? blockIdx.x : kq_order(Gr, blockIdx.x);
         if (threadIdx.x == 0 && work.desc) work.desc[b].count = 0;
@@ -402,19 +408,21 @@ __global__ void __launch_bounds__(KQ_THREADS, 2) gemm_kq_kernel(const uint8_t* w
     if constexpr (MOE) {
         // the tile at the range's position
         const int u = kq_uniform(st.u), u_end = kq_uniform(st.u_end);
-        const int sw = kq_uniform(st.slots_w), per = sw * nsb;
+        const bool whole = !kq_uniform(st.part);
+        const int unit = whole ? 1 : nsb, tw = whole ? 1 : TM + 1;  // of a full tile
+        const int sw = kq_uniform(st.slots_w), per = sw * unit;
         const int tn = u / per;
-        const int q = u - tn * per, q0 = q / nsb;
+        const int q = u - tn * per, q0 = q / unit;
         int qs = q0;
         const int32_t* offsets = kq_uniform(st.offsets);
-        const int sl = kq_find_slot<TM>(offsets, kq_uniform(st.n_slots), qs);
+        const int sl = kq_find_slot<TM>(offsets, kq_uniform(st.n_slots), whole, qs);
         const int r0 = kq_uniform(offsets[sl]), r1 = kq_uniform(offsets[sl + 1]);
-        const int slot_pos = (q0 - qs) * nsb;  // the slot's first position in the column tile
-        const int i = min((q - slot_pos) / (nsb * (TM + 1)), (r1 - r0) / BM);
+        const int slot_pos = (q0 - qs) * unit;  // the slot's first position in the column tile
+        const int i = min((q - slot_pos) / (unit * tw), (r1 - r0) / BM);
         m0 = r0 + i * BM;
         m_end = r1;
-        const int wgt = (min(r1 - m0, BM) + 31) / 32 + 1;
-        const int start = tn * per + slot_pos + i * nsb * (TM + 1), end = start + nsb * wgt;
+        const int wgt = whole ? 1 : (min(r1 - m0, BM) + 31) / 32 + 1;
+        const int start = tn * per + slot_pos + i * unit * tw, end = start + unit * wgt;
         n0 = tn * KQ_BN;
         nr0 = n0;
         const uint8_t* w2 = kq_uniform(st.w2);
@@ -430,7 +438,6 @@ __global__ void __launch_bounds__(KQ_THREADS, 2) gemm_kq_kernel(const uint8_t* w
         wt += sl * kq_uniform(st.expert_bytes);
         s0 = (u - start) / wgt;
         s1 = u_end >= end ? nsb : (u_end - start) / wgt;
-        if (!kq_uniform(st.part)) s1 = u > start ? s0 : nsb;  // no scratch: whole tiles
         int count = 0;
         if (s0 == 0 && s1 < nsb) {
             // the blocks after this one, up to the one that reaches the tile's end
@@ -943,6 +950,38 @@ KqPlan kq_plan(uint32_t ty, int M, int N, int K, bool split) {
     return best;
 }
 
+// Grouped: the tile height, and whether the tiles are cut into one range a CU (the height then by a slot's pairs) or run whole,
+// by the cost at the slots' average share of the pairs: the counts are on the device. Cutting pays for the partial tiles'
+// way through memory, a second launch and ranges of a few super-blocks, too much for small experts: layers of 512 columns
+// 1024 -> 512 -> 1024 with 202 tokens on two of four 104 us cut, 44 whole (59 on the 64-row kernel in K halves that the
+// ranges replaced); 8 of 1280 -> 768 with 209 tokens 74, 45 and 53. Large ones gain by it: 512 tokens on two of 8
+// of 4096 -> 14336 599 us cut, 652 whole.
+struct KqMoePlan {
+    int tm;
+    bool cut;
+    double us;
+};
+
+KqMoePlan kq_moe_plan(int pairs, int n_slots, int N, int K, int forced, bool may_cut) {
+    const int cus = kf_cu_count(), nsb = K / 256, slots = std::min(pairs, n_slots);
+    const double avg = (double)pairs / n_slots;
+    const int cut_tm = avg < 32 ? 1 : avg < 65 ? 2 : 4;
+    constexpr double cut_us[3] = {8.0, 17.5, 18.4};  // the parts and the reduce launch
+    KqMoePlan best{0, false, 1e30};
+    for (int tm = 1; tm <= 4; tm *= 2) {
+        if (forced && tm != (forced == 1 || forced == 2 ? forced : 4)) continue;
+        const int t = tm >> 1;
+        // tiles, and the 32-row parts of one (the empty ones are skipped): a slot's last tile is half full on average
+        const double T = (double)((N + KQ_BN - 1) / KQ_BN) * slots * std::max(1.0, avg / (32 * tm) + 0.5);
+        const double sb = 0.8 + 0.8 * std::min((double)tm, std::max(1.0, avg / 32 + 0.5));
+        const double whole = std::ceil(T / cus) * (KQ_ROUND_US[t] + sb * nsb);
+        if (whole < best.us) best = KqMoePlan{tm, false, whole};
+        const double cut = KQ_ROUND_US[t] + sb * std::max(4.0, nsb * T / cus) + cut_us[t];
+        if (may_cut && (forced || tm == cut_tm) && cut < best.us) best = KqMoePlan{tm, true, cut};
+    }
+    return best;
+}
+
 // The scratch's range area, null when the stream has none
 KqWork kq_work(const KfSplit& split, int full, int S) {
     KqWork w{nullptr, nullptr, full, S};
@@ -1026,17 +1065,22 @@ hipError_t kf_launch_gemm_kq_moe(const void* w, const void* w2, int64_t expert_b
                                  int n_slots, const int32_t* offsets, const int32_t* out_rows, float* y, int N, int K, hipStream_t s) {
     const kf_act_offsets o = kf_act_layout((size_t)pairs, (size_t)K);
     const char* base = static_cast<const char*>(act);
-    // The tile height by the pairs a slot gets on average (KF_MOE_KQ = 0 / 1: 128- or 64-row tiles, a comparison knob)
-    const int avg = pairs / n_slots;
-    int tm = kf_knob_on(KF_KNOB_MOE_KQ) ? (kf_knob(KF_KNOB_MOE_KQ) ? 2 : 4) : kf_knob_or(KF_KNOB_KQ_TM, avg <= 24 ? 1 : avg <= 64 ? 2 : 4);
-    const KqMoe moe{offsets, out_rows, static_cast<const uint8_t*>(w2), expert_bytes, n_slots, n_split};
-    // every CU takes an equal range of the tiles (without the scratch: the tiles that start in it)
-    const int G = kq_max_ranges(tm, kf_cu_count());
-    // KF_GEMM_NO_TAIL: without the scratch (a comparison knob)
+    // KF_MOE_KQ = 0 / 1: 128- or 64-row tiles (a comparison knob); KF_GEMM_NO_TAIL: whole tiles, without the scratch (another)
+    const int forced = kf_knob_on(KF_KNOB_MOE_KQ) ? (kf_knob(KF_KNOB_MOE_KQ) ? 2 : 4) : kf_knob_or(KF_KNOB_KQ_TM, 0);
+    KqMoePlan p = kq_moe_plan(pairs, n_slots, N, K, forced, !kf_knob_on(KF_KNOB_GEMM_NO_TAIL));
+    if (kf_knob_on(KF_KNOB_KQ_G)) p.cut = true;  // KF_KQ_G: the number of ranges (a third)
     std::optional<KfSplit> split;
-    const KqWork work = kf_knob_on(KF_KNOB_GEMM_NO_TAIL) ? KqWork{nullptr, nullptr, 0, G} : kq_work(split.emplace(s, true), 0, G);
+    KqWork work{nullptr, nullptr, 0, 0};
+    if (p.cut) {
+        work = kq_work(split.emplace(s, true), 0, kq_max_ranges(p.tm, kf_cu_count()));
+        if (!work.part) p = kq_moe_plan(pairs, n_slots, N, K, forced, false);
+    }
+    // whole tiles: as many blocks as there may be tiles
+    if (!work.part) work.S = ((N + KQ_BN - 1) / KQ_BN) * (pairs / (32 * p.tm) + std::min(n_slots, pairs));
+    const int G = work.S, tm = p.tm;
+    const KqMoe moe{offsets, out_rows, static_cast<const uint8_t*>(w2), expert_bytes, n_slots, n_split};
 #define KQ_GO(TM)                                                                                                                             \
-    return kq_run<KF_TYPE_Q4_K, TM, true, false>(G, s, static_cast<const uint8_t*>(w), row_bytes, reinterpret_cast<const int8_t*>(base + o.q),      \
+    return kq_run<KF_TYPE_Q4_K, TM, true, (TM == 1)>(G, s, static_cast<const uint8_t*>(w), row_bytes, reinterpret_cast<const int8_t*>(base + o.q),      \
                                           reinterpret_cast<const _Float16*>(base + o.xa), reinterpret_cast<const float*>(base + o.d32),      \
                                           nullptr, nullptr, y, pairs, N, K, work, moe)
     if (tm == 1) KQ_GO(1);

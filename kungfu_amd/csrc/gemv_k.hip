@@ -1,4 +1,4 @@
-// Decode and few-row product for q5_K and q6_K weights (SURVEY's second "next" row: the other K-quant weight types on
+// Decode and few-row product for q5_K and q6_K weights (the other K-quant weight types on
 // the same product; Q4_K_M files carry q6_K head and down projections). y[r][o] = sum over super-blocks of the
 // reference's dot_i8 integers scaled back to floats (crates/kf-quant/src/types/q5_k.rs:7-60, q6_k.rs:17-59) + bias +
 // res; it replaces the reference's q5_K / q6_K loaders of kf_matvec_i8 (crates/kf-backend-cuda/src/kernels/quant_q6_K.cu,

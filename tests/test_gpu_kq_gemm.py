@@ -74,7 +74,10 @@ def test_grouped_ranges(cuda, knobs, counts, tm, scratch):
     x = kf.synth_normal(pairs, 1.0, pairs * n).reshape(pairs, n)
     rows = np.random.default_rng(pairs).permutation(pairs).astype(np.int32)
     knobs.setenv("KF_KQ_TM", tm)
-    if not scratch:
+    # the tiles cut into ranges, or whole
+    if scratch:
+        knobs.setenv("KF_KQ_G", 256)
+    else:
         knobs.setenv("KF_GEMM_NO_TAIL", 1)
     act = kf.alloc_act(pairs, n, cuda)
     kf.quant_act(_t(x, cuda), act, kf.ACT_Q8K)
@@ -231,3 +234,29 @@ def test_decoded_batches_keep_their_product(cuda, knobs, ty, rows, n, n_out, gem
     assert not np.array_equal(few, tiles[0])
     assert np.array_equal(bits(matmul), tiles[0] if gemm else few)
     assert np.array_equal(bits(gemv), few)
+
+
+@pytest.mark.parametrize("n_slots,pairs,n,n_out,cut", [(8, 209, 1280, 1536, False), (16, 110, 1280, 1536, False),
+                                                       (8, 1024, 14336, 4096, True), (8, 128, 4096, 4096, True)])
+def test_grouped_tiles_are_cut_where_that_pays(cuda, knobs, n_slots, pairs, n, n_out, cut):
+    """Small experts run a block a tile (the bits of KF_GEMM_NO_TAIL), large ones in equal ranges (those of KF_KQ_G)."""
+    import torch
+
+    ty = kf.TYPE_Q4_K
+    w = _t(np.tile(_blocks(ty, 512, n, pairs), (n_slots * n_out // 512, 1)), cuda)
+    cnt = np.random.default_rng(1).multinomial(pairs, [1 / n_slots] * n_slots)
+    offs = _t(np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32), cuda)
+    act = kf.alloc_act(pairs, n, cuda)
+    kf.quant_act(_t(kf.synth_normal(pairs, 1.0, pairs * n).reshape(pairs, n), cuda), act, kf.ACT_Q8K)
+    bits = []
+    for name, value in ((None, None), ("KF_GEMM_NO_TAIL", 1), ("KF_KQ_G", 256)):
+        if name:
+            knobs.setenv(name, value)
+        y = torch.full((pairs, n_out), float("nan"), device=cuda)
+        kf.moe_gemm(ty, w, act, pairs, n, n_out, offs, n_slots, y, n_out * kf.row_bytes(ty, n))
+        torch.cuda.synchronize()
+        bits.append(y.cpu().numpy().view(np.uint32))
+        if name:
+            knobs.delenv(name)
+    assert not np.array_equal(bits[1], bits[2])
+    assert np.array_equal(bits[0], bits[2 if cut else 1])

@@ -323,10 +323,12 @@ def test_moe_ffn_grouped_gemm_top_2(cuda, knobs, rows, n_exp, kq, split):
     """Past 64 routed pairs the q4_K layer runs on the grouped tile GEMM (KF_MOE_KQ: 0 its 128-row tiles, 1 its 64-row
     ones): 512 tokens top-2 over eight experts (about 128 pairs an expert, several row tiles each), and 100 tokens over
     three (the last tile of a slot partial), with some pairs unused; sampled tokens against the CPU backend stage by
-    stage and the float path. The tiles are cut into equal ranges, one a CU, whose parts a second launch adds;
-    KF_GEMM_NO_TAIL runs them whole."""
+    stage and the float path. The tiles are cut into equal ranges, one a CU, whose parts a second launch adds
+    (KF_KQ_G), or run whole (KF_GEMM_NO_TAIL)."""
     knobs.setenv("KF_MOE_KQ", kq)
-    if not split:
+    if split:
+        knobs.setenv("KF_KQ_G", "256")
+    else:
         knobs.setenv("KF_GEMM_NO_TAIL", "1")
     n_embd, n_ff, n_used = 1024, 1536, 2
     args, got, stages = _moe_layer(cuda, kf.TYPE_Q4_K, n_exp, n_embd, n_ff, rows, n_used, 70 + n_exp, drop=0.05)
@@ -368,7 +370,7 @@ def test_grouped_gemm_partial_row_tiles(cuda, knobs, kq):
 
 
 def test_moe_ffn_config_c5_every_token(cuda):
-    """Config C5 at full size (8 experts of Q4_K 4096 -> 14336 -> 4096, 16 tokens, top-2): all 16 tokens against the
+    """Full size (8 experts of Q4_K 4096 -> 14336 -> 4096, 16 tokens, top-2): all 16 tokens against the
     CPU backend, stage by stage, and the layer against the CPU float path."""
     n_exp, n_embd, n_ff, rows, n_used = 8, 4096, 14336, 16, 2
     args, got, stages = _moe_layer(cuda, kf.TYPE_Q4_K, n_exp, n_embd, n_ff, rows, n_used, 0)

@@ -458,7 +458,7 @@ def test_matmul_q4_k_many_rows(cuda, rows, n_out):
 
 @pytest.mark.parametrize("n,n_out", [(4096, 14336), (14336, 4096)])
 def test_gemm_prefill_shapes_match_gemv(cuda, n, n_out):
-    """Config C4 at full size (M = 2048): the PREFILL_ROWS rows of the GEMM against the GEMV of that row on the same
+    """Full size (M = 2048): the PREFILL_ROWS rows of the GEMM against the GEMV of that row on the same
     quantized activations, and against the CPU backend's matmul_slice (rows are independent)."""
     import torch
 
@@ -571,7 +571,7 @@ LLAMA_SHAPES = {"qkv": (4096, 6144), "o": (4096, 4096), "gate": (4096, 14336), "
 @pytest.mark.parametrize("shape", list(LLAMA_SHAPES))
 @pytest.mark.parametrize("rows", [8, 16, 32, 64])
 def test_matmul_q8_0_small_batch_llama_shapes(cuda, shape, rows):
-    """Config C3: kf_hip_matmul on Q8_0 weights at the Llama-3-8B shapes and 8 / 16 / 32 / 64 activation rows (the
+    """kf_hip_matmul on Q8_0 weights at the Llama-3-8B shapes and 8 / 16 / 32 / 64 activation rows (the
     small-batch product), every 7th output column against the CPU backend's matmul_slice on those weight rows (output
     columns are independent) (crates/kf-backend-cuda/tests/quant.rs:46-112)."""
     import torch
