@@ -886,15 +886,21 @@ int kq_max_parts(int tm, int cus) {
     return (int)std::min((size_t)kf_knob_or(KF_KNOB_KQ_G, cus), room);
 }
 
-// A block's f32 sum of more super-blocks than this is kept in 64 bits instead (WIDE), where the tile's registers have room:
-// 16 super-blocks of q4_K are 9.7e-8 from the 64-bit result with f32 sums and 7.3e-8 with these, 51 of q6_K 1.32e-7 and
-// 4.4e-8, at 10-12% (q4_K), 6% (q5_K) and 3% (q6_K) of the K loop. The few-row products and the shorter K ranges that these
-// blocks replace had 8.5-9.1e-8 and 8e-8. 128-row tiles, and 64-row ones of q5_K (four registers spilled), keep the f32
+// A block's f32 sum of more super-blocks than kq_long is kept in 64 bits instead (WIDE), where the tile's registers have
+// room: 16 super-blocks of q4_K are 9.7e-8 from the 64-bit result with f32 sums and 7.3e-8 with these, 51 of q6_K 1.32e-7
+// and 4.4e-8, at 10% (q4_K), 6% (q5_K) and 3% (q6_K) of the K loop; priced higher on q4_K, as plans with K ranges in its place
+// measured 3-5% less than the model has (500 rows of 4096 -> 4096: 36.2 us in two ranges, 39.0 wide). The few-row products,
+// and the 64-row kernel in two or four K ranges, that these blocks replace had 8e-8 to 9.1e-8; where that kernel had whole
+// rounds of tiles it summed as many in f32. 128-row tiles, and 64-row ones of q5_K (four registers spilled), keep the f32
 // sum, as the tile kernels did whose whole rounds they took over; widths of q6_K that had no tile kernel before (rows
 // that are not whole 16-byte pieces) leave them out instead: 2048 rows of 13056 -> 4096 take 426 us in place of 294,
 // 6400 -> 2304 145 and 144, and 19.6 and 6.5 ms on the per-lane product.
-constexpr int KQ_LONG = 12;
-constexpr double KQ_WIDE_COST[3] = {1.12, 1.06, 1.03};  // [q4_K, q5_K, q6_K]
+int kq_long(bool ragged, int M, int N, int nsb, int cus) {
+    const int T = ((N + KQ_BN - 1) / KQ_BN) * ((M + 63) / 64);  // tiles of the 64-row kernel
+    if (ragged) return 12;
+    return std::max(12, T >= cus ? nsb : 4 * T <= cus ? (nsb + 3) / 4 : 2 * T <= cus ? (nsb + 1) / 2 : nsb);
+}
+constexpr double KQ_WIDE_COST[3] = {1.25, 1.06, 1.03};  // [q4_K, q5_K, q6_K]
 
 struct KqPlan {
     int tm, T, full, S;
@@ -910,10 +916,11 @@ KqPlan kq_plan_tm(uint32_t ty, int tm, int M, int N, int K, bool split) {
     const int rem = p.T % cus, t = tm >> 1, max_g = kq_max_parts(tm, cus), k = ty == KF_TYPE_Q4_K ? 0 : ty == KF_TYPE_Q5_K ? 1 : 2;
     const double sb = KQ_SB_US[k][t];
     const bool fits = tm == 1 || (tm == 2 && ty != KF_TYPE_Q5_K), ragged = ty == KF_TYPE_Q6_K && K % 2048 != 0;
+    const int longest = kq_long(ragged, M, N, nsb, cus);
     // a block of n super-blocks, in a launch whose longest one has `most`
     auto cost = [&](int n, int most) {
-        if (most > KQ_LONG && ragged && !fits) return 1e30;
-        return KQ_ROUND_US[t] + sb * n * (most > KQ_LONG && fits ? KQ_WIDE_COST[k] : 1.0);
+        if (most > longest && ragged && !fits) return 1e30;
+        return KQ_ROUND_US[t] + sb * n * (most > longest && fits ? KQ_WIDE_COST[k] : 1.0);
     };
     const int rounds = p.T / cus;
     p.full = p.T;
@@ -933,7 +940,7 @@ KqPlan kq_plan_tm(uint32_t ty, int tm, int M, int N, int K, bool split) {
         }
     }
     p.us += 1.8;
-    p.wide = fits && !few && (p.full > 0 ? nsb : (nsb + p.S - 1) / p.S) > KQ_LONG;
+    p.wide = fits && !few && (p.full > 0 ? nsb : (nsb + p.S - 1) / p.S) > longest;
     return p;
 }
 
