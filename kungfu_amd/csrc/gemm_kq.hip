@@ -233,6 +233,9 @@ __device__ __forceinline__ uint32_t kq_pk_mad(uint32_t a, uint32_t b, uint32_t c
     return __builtin_bit_cast(uint32_t, (u16x2)(__builtin_bit_cast(u16x2, a) * __builtin_bit_cast(u16x2, b) + __builtin_bit_cast(u16x2, c)));
 }
 
+// Bytes 1 and 3 of v as 16-bit pairs
+__device__ __forceinline__ uint32_t kq_odd(uint32_t v) { return __builtin_amdgcn_perm(v, v, 0x0c030c01u); }
+
 // Byte B of v in both 16-bit halves, zero- or sign-extended
 template <int B>
 __device__ __forceinline__ uint32_t kq_pair(uint32_t v) {
@@ -322,8 +325,8 @@ struct KqWeight {
             const uint32_t s = kq_pair<g & 3>(sc[g >> 2]);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const uint32_t q = (((g & 1) ? v[e] >> 4 : v[e]) & m4) | (((h[e] >> g) & 0x01010101u) << 4);
-                const uint32_t ev = kq_pk_mad(q & mb, s, 0x00800080u), ov = kq_pk_mad((q >> 8) & mb, s, 0x00800080u);
+                const uint32_t q = (((g & 1) ? v[e] >> 4 : v[e]) & m4) | ((g < 4 ? h[e] << (4 - g) : h[e] >> (g - 4)) & 0x10101010u);
+                const uint32_t ev = kq_pk_mad(q & mb, s, 0x00800080u), ov = kq_pk_mad(kq_odd(q), s, 0x00800080u);
                 p.lo[e] = kq_low16(ev, ov);
                 p.hi[e] = kq_high16(ev, ov);
             }
@@ -338,7 +341,7 @@ struct KqWeight {
             for (int e = 0; e < 4; e++) {
                 const uint32_t lo = ((k & 2) ? v[e] >> 4 : v[e]) & m4;
                 const uint32_t q = lo | (((h[e] >> (2 * k)) & 0x03030303u) << 4);
-                const uint32_t ev = kq_pk_mad(q & mb, s, c), ov = kq_pk_mad((q >> 8) & mb, s, c);
+                const uint32_t ev = kq_pk_mad(q & mb, s, c), ov = kq_pk_mad(kq_odd(q), s, c);
                 p.lo[e] = kq_low16(ev, ov);
                 p.hi[e] = kq_high16(ev, ov);
             }
