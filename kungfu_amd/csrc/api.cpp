@@ -35,6 +35,7 @@ hipError_t kf_launch_gemv1(uint32_t ty, const void* w, int64_t row_bytes, const 
 hipError_t kf_launch_block_ints(uint32_t ty, const void* w, int64_t row_bytes, const void* act, int rows, int n, int n_out,
                                 int32_t* out, hipStream_t s);
 bool kf_rows_mma_1_ok(uint32_t ty, const void* w, int64_t row_bytes, int n, int n_out, int rows);
+int kf_rows_mma_1_tiles(int n_out);
 hipError_t kf_launch_rows_mma_1(uint32_t ty, const void* w, int64_t row_bytes, const int8_t* xq, const int32_t* xs32, const float* xd32, int n,
                                 int n_out, int rows, const float* bias, const float* res, float* y, hipStream_t s);
 hipError_t kf_launch_gemv1_fused(uint32_t ty, const void* w, int64_t row_bytes, const float* x, const float* bias, const float* res, float* y,
@@ -335,19 +336,22 @@ int kf_hip_rms_norm_matmul(uint32_t ty, const void* w, int n_in, int n_out, cons
 
 }  // extern "C"
 
-// The few-row products' cost on the K types (MI355X, us; fitted over 33-512 rows at 1024 -> 512 to 8192 -> 8192 and 14336 ->
-// 512): the larger of 2.5 plus the latency of a pass of 16 activation rows, which grows with the super-blocks of a row, and
-// 5.5 plus its MB of weights, per pass. Matrices of few outputs cost their latency: 300 rows of q4_K 1024 -> 512 28 us against the
-// tile GEMM's 10, of q6_K 14336 -> 512 285 against 25. q6_K rows that start off a dword (an odd number of super-blocks) run the per-lane product, whose cost grows with each row
-// (1792 -> 3584, 6400 -> 2304 and 13056 -> 2048 at 2-16 rows: 7.1-36.6, 11.7-53.3 and 15.8-69.8 us); q4_K rows wider than the few-row product stages run as one GEMV launch per row.
+// The few-row products' cost on the K types (MI355X, us; fitted over 34-300 rows of nineteen shapes from 1024 -> 512 to 8192 ->
+// 8192 and 14336 -> 512, 2-5% rms): 2.5, and for every 16 activation rows a pass over the super-blocks of the 16-output tiles
+// that a block takes, one block a CU, or 5.5 and a pass over the weights' MB where that is more. The tiles count where they
+// fill the CUs badly: 272 of them are two a block, and 96 rows of q4_K 4096 -> 4352 take 29.7 us with the quantization where the
+// GEMM takes 20.2; so does the latency of a pass: 300 rows of 14336 -> 512 take 122-285 us against 20-25. q6_K rows
+// that start off a dword (an odd number of super-blocks) run the per-lane product, whose cost grows with each row
+// (1792 -> 3584, 6400 -> 2304 and 13056 -> 2048 at 2-16 rows: 7.1-36.6, 11.7-53.3 and 15.8-69.8 us); q4_K rows wider than the
+// few-row product stages run as one GEMV launch per row.
 static double kq_few_rows_us(uint32_t ty, const void* w, int rows, int n_in, int n_out, int64_t row_bytes) {
     const double mb = (double)n_out * row_bytes / 1e6;
     if (ty == KF_TYPE_Q4_K && n_in > kf_rows_max_n(ty)) return rows * (2.5 + 0.22 * mb);
     if (!kf_rows_mma_1_ok(ty, w, row_bytes, n_in, n_out, rows)) return 2.0 + (rows + 7) / 8 * (1.0 + 0.3 * mb) + rows * (0.9 + 0.13 * mb);
-    const int k = ty == KF_TYPE_Q4_K ? 0 : ty == KF_TYPE_Q5_K ? 1 : 2;
-    constexpr double pass[3] = {0.95, 1.0, 1.1}, sb[3] = {0.095, 0.114, 0.245}, per_mb[3] = {0.21, 0.20, 0.33};
-    const int passes = (rows + 15) / 16;
-    return std::max(2.5 + passes * (pass[k] + sb[k] * (n_in / 256)), 5.5 + passes * per_mb[k] * mb);
+    const int k = ty == KF_TYPE_Q4_K ? 0 : ty == KF_TYPE_Q5_K ? 1 : 2, per_block = kf_rows_mma_1_tiles(n_out), cus = kf_cu_count();
+    constexpr double sb[3] = {0.102, 0.120, 0.255}, per_mb[3] = {0.21, 0.20, 0.33};
+    const int passes = (rows + 15) / 16, rounds = ((n_out + 15) / 16 + per_block * cus - 1) / (per_block * cus);
+    return std::max(2.5 + passes * (0.88 + sb[k] * (n_in / 256) * per_block * rounds), 5.5 + passes * per_mb[k] * mb);
 }
 
 // Up to KF_FEW_ROWS rows kf_hip_matmul's choice on the K types, and the order of the f32 sums with it, stays what it was

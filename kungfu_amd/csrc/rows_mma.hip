@@ -659,26 +659,24 @@ bool kf_rows_mma_1_ok(uint32_t ty, const void* w, int64_t row_bytes, int n, int 
     return (ty == KF_TYPE_Q4_K || ty == KF_TYPE_Q5_K) && row_bytes % 16 == 0;
 }
 
+// 16-output tiles a block of the one-slot few-row product takes. A block's two stage buffers per wave hold most of a CU's
+// LDS, so one block runs per CU: the fewest tiles a block whose grid still fits in one round of the CUs (QKV at 4096 x 6144:
+// 192 blocks of two tiles, 8.5 us at 8 rows, against 384 blocks of one tile in two rounds, 10.7 us)
+int kf_rows_mma_1_tiles(int n_out) {
+    const int forced = kf_knob_or(KF_KNOB_RM1_TILES, 0);  // a tuning knob (1, 2, 4 or 8 tiles a block)
+    if (forced == 1 || forced == 2 || forced == 4 || forced == 8) return forced;
+    const int tiles = (n_out + 15) / 16, cus = kf_cu_count();
+    for (int t = 1; t < 8; t *= 2)
+        if ((tiles + t - 1) / t <= cus) return t;
+    return 8;
+}
+
 // Host launcher of the one-slot few-row product (rows_mma_1_kernel) for q4_K, q5_K and q6_K weights, validated by the
-// caller (kf_rows_mma_1_ok). Tiles per block chosen so the grid has about one block per CU or more.
+// caller (kf_rows_mma_1_ok)
 hipError_t kf_launch_rows_mma_1(uint32_t ty, const void* w, int64_t row_bytes, const int8_t* xq, const int32_t* xs32, const float* xd32, int n,
                                 int n_out, int rows, const float* bias, const float* res, float* y, hipStream_t s) {
     if (!kf_rows_mma_1_ok(ty, w, row_bytes, n, n_out, rows)) return hipErrorInvalidValue;
-    const int tiles = (n_out + 15) / 16;
-    const int forced = kf_knob_or(KF_KNOB_RM1_TILES, 0);  // a tuning knob (1, 2, 4 or 8 tiles a block)
-    // a block's two stage buffers per wave hold most of a CU's LDS, so one block runs per CU: the fewest tiles a block
-    // whose grid still fits in one round of the CUs (QKV at 4096 x 6144: 192 blocks of two tiles, 8.5 us at 8 rows,
-    // against 384 blocks of one tile in two rounds, 10.7 us)
-    int tpb = forced == 1 || forced == 2 || forced == 4 || forced == 8 ? forced : 0;
-    if (tpb == 0) {
-        const int cus = kf_cu_count();
-        tpb = 8;
-        for (int t = 1; t < 8; t *= 2)
-            if ((tiles + t - 1) / t <= cus) {
-                tpb = t;
-                break;
-            }
-    }
+    const int tiles = (n_out + 15) / 16, tpb = kf_rows_mma_1_tiles(n_out);
     const auto* wb = static_cast<const uint8_t*>(w);
 #define KF_R1(TY, T)                                                                                               \
     {                                                                                                              \

@@ -178,10 +178,11 @@ def test_infinite_and_nan_block_scales(cuda, knobs, ty, tm, tail):
 
 
 @pytest.mark.parametrize("ty", K_TYPES)
-@pytest.mark.parametrize("rows,n,n_out,gemm", [(300, 1024, 512, True), (256, 14336, 40, True), (200, 1792, 600, True), (48, 1024, 512, False)])
+@pytest.mark.parametrize("rows,n,n_out,gemm", [(300, 1024, 512, True), (256, 14336, 40, True), (200, 1792, 600, True), (48, 1024, 512, False), (96, 4096, 4352, True)])
 def test_few_outputs_price_the_few_row_products_latency(cuda, knobs, ty, rows, n, n_out, gemm):
     """Matrices of few outputs: each 16-row pass of the few-row product costs the latency of a whole row, so many rows take
-    the tile GEMM (the bits of KF_KQ_GEMM=1) and 48 short ones do not (those of KF_KQ_GEMM=0)."""
+    the tile GEMM (the bits of KF_KQ_GEMM=1) and 48 short ones do not (those of KF_KQ_GEMM=0). So do 96 rows of 272 tiles, two
+    a block on half the CUs."""
     import torch
 
     w = _t(_blocks(ty, n_out, n, rows + n), cuda)
