@@ -1,6 +1,6 @@
 """Benchmark of the MI355X-native quantized linear-layer hot path (one JSON line on stdout).
 
-Workload (BASELINE configs[1]): the Q4_K decode GEMV at the Llama-3-8B layer shapes, batch 1 — one step is one
+Workload: the Q4_K decode GEMV at the Llama-3-8B layer shapes, batch 1 — one step is one
 decoder layer's linear products: QKV 4096->6144, O 4096->4096, gate and up 4096->14336 each, down 14336->4096. Gate
 and up share their input, so their weights are stored as one [2 * 14336][row] tensor and run as one launch (the same
 bytes and outputs as two launches; the layout a loader chooses when it reads the two GGUF tensors).
@@ -116,7 +116,7 @@ SMALL_BATCH_Q4_K = SMALL_BATCH + [96, 128, 192, 256]
 
 
 def gemm_section(dev, m=2048, ty=None):
-    """int8 MFMA GEMM of configs[3]: M=2048 Q8_0-kind activation rows against Q8_0 weights, both prefill shapes
+    """int8 MFMA GEMM: M=2048 Q8_0-kind activation rows against Q8_0 weights, both prefill shapes
     (with ty = q4_K: the same shapes with Q4_K weights and Q8K-kind activations, the tile GEMM kf_hip_matmul takes for
     Q4_K prefill). TOPS = 2*M*N*K / kernel time (the quant_act launch is timed beside it); two weight copies alternate."""
     import torch
@@ -149,14 +149,14 @@ def gemm_q4_k_section(dev):
 
 
 def gemm_k_quants_section(dev):
-    """The q5_K and q6_K prefill GEMM (SURVEY's second "next" row) at the configs[3] shapes, M = 2048."""
+    """The q5_K and q6_K prefill GEMM at the shapes of gemm_section, M = 2048."""
     import kungfu_amd as kf
 
     return {"q5_K": gemm_section(dev, ty=kf.TYPE_Q5_K), "q6_K": gemm_section(dev, ty=kf.TYPE_Q6_K)}
 
 
 def small_batch_section(dev):
-    """batch 8..64 of the Llama-3-8B shapes with Q8_0 weights: the product kernel alone on resident
+    """Batch 8..64 of the Llama-3-8B shapes with Q8_0 weights: the product kernel alone on resident
     quantized activations (µs per call, weight-streaming GB/s, TOPS) and the whole kf_hip_matmul (quant_act + product)."""
     import torch
 
@@ -182,9 +182,9 @@ def small_batch_section(dev):
 
 
 def small_batch_q4_k_section(dev):
-    """Batch 8..64 of the Llama-3-8B shapes with Q4_K weights (the reference's mm_frag range): the multi-row product
-    (kf_hip_gemv: 16 activation rows a weight pass on the matrix cores) and the tile GEMM (kf_hip_gemm_i8) alone on
-    resident quantized activations, and the whole kf_hip_matmul (quant_act + the product it selects); weight copies
+    """Batch 8..64 of the Llama-3-8B shapes with Q4_K weights (the reference's mm_frag range): kf_hip_gemv (16
+    activation rows a weight pass on the matrix cores, or the tile GEMM by cost past 32 rows) and the tile GEMM
+    (kf_hip_gemm_i8) alone on resident quantized activations, and the whole kf_hip_matmul (quant_act + the product it selects); weight copies
     rotated past the MALL."""
     import torch
 
@@ -213,7 +213,7 @@ def small_batch_q4_k_section(dev):
 
 
 def moe_section(dev, seed=0, rows=16):
-    """the routed expert layer (kf_hip_moe_ffn) for 8 Q4_K experts of gate/up 4096->14336 and down
+    """The routed expert layer (kf_hip_moe_ffn) for 8 Q4_K experts of gate/up 4096->14336 and down
     14336->4096, 16 tokens, top-2 uniform without replacement. GB/s over the weight bytes of the touched experts (each
     read once per call) plus the fp32 activations in and out; two copies of the expert set alternate (1.6 GB).
     With rows = 512 (1024 routed pairs, the grouped tile GEMM): also TOPS = 2 * pairs * 3 * n_ff * n_embd / time, the
@@ -583,7 +583,7 @@ def main():
     achieved = k1_bytes / k1_us / 1e3
     probe = read_probe(shapes[2], dev)
 
-    # Q8_0 GEMV of configs[0] (4096x4096) on the GPU, rotating copies
+    # Q8_0 GEMV 4096x4096 on the GPU, rotating copies
     q8 = Shape("q8_0", kf.TYPE_Q8_0, 4096, 4096, max(2, -(-2 * MALL_BYTES // (kf.row_bytes(8, 4096) * 4096)) + 1), dev)
     us_q8 = time_launches(q8.gemv, 200)
     ceil_q8 = same_bytes_ceiling(q8.w, dev)

@@ -19,8 +19,8 @@
 // weight operand is expanded once for TM tiles. The operands of a whole super-block stay in registers (64) and the tiles
 // run one after another, eight group steps each: a step's two MFMAs go with an eighth of the previous tile's rescale
 // and, in the last tile, with the expansion of the next super-block's operands, so no phase of a wave is without MFMAs
-// and the two waves of a SIMD need no offset. What bounds it at TM = 4: MFMA busy 47% and VALU issue 51% of the cycles,
-// which overlap only in part, and LDS and DMA waits. Choices that measured (2048 rows, us): reloads of spilled registers
+// and the two waves of a SIMD need no offset. What bounds it at TM = 4 (2048 rows of q4_K): MFMA busy 47-53% and
+// VALU issue 56-61% of the cycles, which overlap only in part, and LDS and DMA waits (29-33% of a wave's cycles). Choices that measured (2048 rows, us): reloads of spilled registers
 // in the K loop wait for every load in flight (446 -> 295, 4096 -> 14336 q4_K); the loads of a super-block spread over
 // the steps instead of all at its start, where eight waves queue them behind each other, and each step's LDS
 // reads one step ahead (267 -> 241, 14336 -> 4096 q4_K).
@@ -29,9 +29,10 @@
 // waves share ([tile][row 32][256] with the 16-byte chunk swizzle c ^ (row % 16)); every wait is explicit. Blocks run in
 // XCD order, so the blocks in flight on an XCD share their weight tiles in its L2.
 // Measured, us, before (the one-MFMA form on q5_K / q6_K, a 128 x 256 tile kernel without the interleaved rescale on q4_K, the
-// per-lane product on q6_K rows off 16 bytes) and now, 4096 -> 14336 / 14336 -> 4096: 2048 rows q4_K 281 / 260 -> 270 / 239, q5_K
-// 370 / 345 -> 304 / 272, q6_K 620 / 597 -> 325 / 287; 128 rows q4_K 46 / 62 -> 34 / 32, q5_K 74 / 78 -> 36 / 37, q6_K
-// 138 / 125 -> 39 / 40; 63 rows of q6_K 2816 -> 7052 305 -> 25.
+// per-lane product on q6_K rows off 16 bytes) and now, 4096 -> 14336 / 14336 -> 4096: 2048 rows q4_K 291 / 266 -> 285 / 245, q5_K
+// 348 / 322 -> 316 / 278, q6_K 629 / 609 -> 338 / 291; 128 rows q4_K 36 / 48 -> 33 / 32, q5_K 38 / 51 -> 36 / 34, q6_K
+// 58 / 86 -> 38 / 37; 63 rows of q6_K 2816 -> 7052 273 -> 22. On 64-row tiles of q5_K the expansion of two planes costs more than the
+// one-MFMA form did: 378 rows of 1792 -> 10584 32.7 -> 36.8 with the quantization, 510 of 3072 -> 8192 46.7 -> 52.5.
 #include "kf_knobs.h"
 #include "kf_blocks.h"
 #include "kf_device.h"

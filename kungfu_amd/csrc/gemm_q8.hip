@@ -23,8 +23,8 @@
 //
 // Measured (MI355X, one product, with the tiles, split and form the plan picks; before: the 128 x 128 kernel, the 64-row
 // small-batch kernel, or for rows that are not 16-byte aligned the multi-row product of kf_hip_gemv):
-// 14336 -> 4096 at 2048 rows 359 -> 318 us, 128 rows 64 -> 40, 64 rows 33 -> 27; 4160 -> 6000 at 64 rows 226 -> 19, 16 rows
-// 59 -> 14.6.
+// 14336 -> 4096 at 2048 rows 359 -> 322 us, 128 rows 60 -> 36, 64 rows 30 -> 25 (4096 -> 14336: 370 -> 368 at 2048 rows, 30 ->
+// 26 at 64); 4160 -> 6000 at 64 rows 226 -> 21, 16 rows 60 -> 17.
 #include "kf_device.h"
 #include "kf_host.h"
 #include "kf_knobs.h"
@@ -349,7 +349,7 @@ __global__ void __launch_bounds__(Q8_THREADS) q8_reduce_kernel(Q8Work work, cons
 // Widths that are no whole number of 128-column steps. Before this kernel they ran the multi-row product, whose 64 lanes'
 // sums meet in a tree (7e-8 from the 64-bit result at 33-130 groups, 9e-8 at 449, against 2e-7 and 3.8e-7 for one f32 sum
 // over all of them), so here every second stage goes into the 64-bit sums (6-7e-8) and tiles without room for these are
-// left out: 2048 rows of 14368 -> 4096 take 472 us instead of 352, 300 rows 93 instead of 84, and 29 and 4.3 ms on the
+// left out: 2048 rows of 14368 -> 4096 take 472 us instead of 352, 300 rows 93 instead of 84, and 56 and 4.3 ms on the
 // multi-row product.
 bool q8_ragged(int K) { return K % (32 * Q8_G) != 0; }
 
