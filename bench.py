@@ -304,7 +304,7 @@ def layer_with_producers_section(shapes, dev):
 
 
 def fused_section(dev):
-    """The fused activation producers (SURVEY's first "next" row): rms_norm_q8 over the hidden width and gated_act_q8
+    """The fused activation producers: rms_norm_q8 over the hidden width and gated_act_q8
     over the FFN width (silu, gate and up as the halves of one fused gate+up output row), at decode (1 row) and
     prefill (2048 rows), Q8K kind (the q4_K weights' kind). GB/s over the f32 read and the scratch written; quant_act
     of the same f32 input beside it, for the cost the fusion removes (the f32 write and re-read of the normed values)."""
@@ -332,7 +332,7 @@ def fused_section(dev):
 
 
 def kquant_section(dev):
-    """q6_K and q5_K weights (SURVEY's second "next" row) at the Llama-3-8B shapes, batch 1 (the GEMV) and batch 8 (eight
+    """q6_K and q5_K weights at the Llama-3-8B shapes, batch 1 (the GEMV) and batch 8 (eight
     activation rows against one weight pass): us per call and GB/s over weight bytes + f32 activations in and out,
     weight copies rotated past the MALL."""
     import kungfu_amd as kf
@@ -488,7 +488,7 @@ def cpu_baseline(shapes, budget_s):
     """The CPU backend's product (oracle restatement of ops::matmul_slice, OpenMP over output rows, as rayon's par_iter
     over rows) on the same weights and input: whole layer passes until budget_s of wall time is spent; then the same
     for its integer path (ops::matmul_i8: the activations quantized once per call, dot_i8 per row). Threads: every
-    logical core the process may run on, capped by OMP_NUM_THREADS where the host sets it (a GPU box's CPU share)."""
+    logical core the process may run on, capped by OMP_NUM_THREADS where the host sets it (a shared host's CPU share)."""
     import oracle
 
     avail = len(os.sched_getaffinity(0)) if hasattr(os, "sched_getaffinity") else (os.cpu_count() or 1)

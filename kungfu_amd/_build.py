@@ -1,7 +1,7 @@
 """Builds the kf-hip C-ABI library for gfx950: kungfu_amd/lib/libkf_hip.so.
 
-The library is compiled in-tree with hipcc (no JIT cache), so the built .so travels with the repository snapshot to
-the GPU box. Every HIP translation unit is compiled with packed-FP32 instructions disabled.
+The library is compiled in-tree with hipcc (no JIT cache), so the built .so travels with a copy of the tree.
+Every HIP translation unit is compiled with packed-FP32 instructions disabled.
 """
 from __future__ import annotations
 

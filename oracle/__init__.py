@@ -2,7 +2,7 @@
 
 This package wraps ``oracle/build/libkf_oracle.so`` (built from ``oracle/kf_oracle.c`` by ``oracle/Makefile``) with
 numpy-friendly functions. Only ``tests/``, ``__graft_entry__.smoke()`` and the CPU-baseline leg of ``bench.py`` may
-import it, and only as the checker: the product library ``kungfu_amd`` never routes through it.
+import it, and only to compare with: the product library ``kungfu_amd`` never routes through it.
 
 Each C function restates a piece of the Rust reference and cites the file:line it follows (see kf_oracle.c).
 """

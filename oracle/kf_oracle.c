@@ -2,7 +2,7 @@
  * kf_oracle.c — CPU restatement of kungfu's quantized linear-layer arithmetic (the parity oracle).
  *
  * TEST INFRASTRUCTURE ONLY: the product never links or loads this file's library; tests/, the smoke check and the
- * benchmark's CPU-baseline leg use it as the checker. Built with -ffp-contract=off so every float operation rounds
+ * benchmark's CPU-baseline leg compare with it. Built with -ffp-contract=off so every float operation rounds
  * where the Rust source rounds (Rust never contracts a*b+c into an fma on its own).
  *
  * Third-party arithmetic restated here: f16 conversion of the `half` crate 2.7.1 (IEEE binary16, round to nearest

@@ -1,7 +1,7 @@
 /*
  * kf_oracle — CPU restatement of kungfu's quantized linear-layer arithmetic.
  *
- * TEST INFRASTRUCTURE ONLY. Nothing in the product links, loads or calls this library. It is the checker the
+ * TEST INFRASTRUCTURE ONLY. Nothing in the product links, loads or calls this library. It is what the
  * parity tests, the smoke check and the CPU-baseline leg of the benchmark compare the HIP path against.
  *
  * Every function restates one piece of the Rust reference (nickheyer/kungfu) and cites the file:line it follows.

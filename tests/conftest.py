@@ -9,7 +9,7 @@ if ROOT not in sys.path:
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs an MI355X (runs on the GPU box through the C ABI)")
+    config.addinivalue_line("markers", "gpu: needs an MI355X (runs through the C ABI)")
 
 
 @pytest.fixture(scope="session")
